@@ -8,7 +8,8 @@ include/mynah_asr_hip.h at one size:
   attention    relative-position attention core             mynah_asr_hip_relpos_attention_dev
   layer        one FastConformer encoder layer              mynah_asr_hip_encoder_layer_dev
   subsampling  mel features to encoder rows                 mynah_asr_hip_subsampling_dev
-  decoder      AED decoder over given tokens                mynah_asr_hip_aed_forced_dev
+  decoder      AED greedy decoding, then the logits of the
+               decoded tokens (their confidences)           mynah_asr_hip_aed_decode_dev, _aed_forced_dev
   host_ffn     the feed-forward on the caller's host arrays mynah_asr_hip_qffn
 
 Sizes are the FastConformer-0.6B / Canary-style ones of the benchmark
@@ -32,6 +33,7 @@ FORMATS = {"F32": M.F32, "INT8": M.INT8, "INT4": M.INT4, "Q8_0": M.Q8_0, "Q4_K":
 CONV_K = 9
 
 _lib = None
+_stream = None
 
 
 def lib():
@@ -39,6 +41,14 @@ def lib():
     if _lib is None:
         _lib = M.HipLib()
     return _lib
+
+
+def stream():
+    """The one stream all device calls run on: a thread's calls share its workspaces, so they are ordered."""
+    global _stream
+    if _stream is None:
+        _stream = torch.cuda.Stream()
+    return _stream
 
 
 # ------------------------------------------------------------------ the cases
@@ -64,8 +74,8 @@ def listed():
         {"name": "attention_stream_16x60s", "kind": "attention", "T": 750, "nseq": 16, "d": 1024, "H": 8, "left": 70, "right": 13},
         # the convolutional front end, 4 x 60 s of 80 mel features
         {"name": "subsampling_4x60s", "kind": "subsampling", "frames": 6000, "nseq": 4, "mels": 80, "C": 256, "d": 1024, "causal": False},
-        # 32 decoder positions over one 60 s utterance
-        {"name": "decoder_32", "kind": "decoder", "fmt": "Q8_0", "T": 750, "tokens": 32, "layers": 4, "d": 1024, "H": 8,
+        # 24 tokens decoded and scored over one 60 s utterance
+        {"name": "decoder_24", "kind": "decoder", "fmt": "Q8_0", "T": 750, "tokens": 24, "layers": 4, "d": 1024, "H": 8,
          "f": 4096, "vocab": 16384},
         # the drop-in call of a C caller that keeps its activations in host memory, 20 s
         {"name": "host_ffn_250", "kind": "host_ffn", "fmt": "Q8_0", "rows": 250, "d": 1024, "f": 4096},
@@ -110,7 +120,7 @@ def draw(rng):
                 "mels": rng.choice([80, 128]), "C": 256, "d": rng.choice([1024, 512]), "causal": rng.random() < 0.3}
     if kind == "decoder":
         return {"kind": kind, "fmt": rng.choice(["Q8_0", "Q8_0", "Q4_K"]), "T": _between(rng, 40, 750),
-                "tokens": _between(rng, 4, 31), "layers": rng.choice([2, 4]), "d": 1024, "H": 8, "f": 4096,
+                "tokens": _between(rng, 4, 23), "layers": rng.choice([2, 4]), "d": 1024, "H": 8, "f": 4096,
                 "vocab": rng.choice([16384, 5248])}
     return {"kind": kind, "fmt": rng.choice(["Q8_0", "Q4_K", "INT8"]), "rows": _between(rng, 1, 750), "d": 1024, "f": 4096}
 
@@ -235,11 +245,12 @@ class Linear:
         self.rows, self.mode = case["rows"], M.INT8ACT if case["int8act"] else M.EXACT
         self.x = r.normal(case["rows"], case["k"])
         self.y = torch.empty(case["rows"], case["n"], device="cuda")
+        self.stream = stream().cuda_stream
 
     def run(self):
         if self.mode != M.EXACT:
             lib().set_numerics(self.mode)
-        self.w.gemm(self.x.data_ptr(), self.y.data_ptr(), self.rows)
+        self.w.gemm(self.x.data_ptr(), self.y.data_ptr(), self.rows, 0, self.stream)
         if self.mode != M.EXACT:
             lib().set_numerics(M.EXACT)
         return self.y
@@ -252,9 +263,10 @@ class Ffn:
         self.rows = case["rows"]
         self.x = r.normal(case["rows"], case["d"])
         self.y = torch.empty(case["rows"], case["d"], device="cuda")
+        self.stream = stream().cuda_stream
 
     def run(self):
-        M.ffn_dev(lib(), self.w1, self.w2, self.x.data_ptr(), self.y.data_ptr(), self.rows)
+        M.ffn_dev(lib(), self.w1, self.w2, self.x.data_ptr(), self.y.data_ptr(), self.rows, self.stream)
         return self.y
 
 
@@ -318,11 +330,12 @@ class Attention:
         self.case = case
         self.inputs = _attention_inputs(case, Draws(seed))
         self.ctx = torch.empty(case["nseq"], case["T"], case["d"], device="cuda")
+        self.stream = stream().cuda_stream
 
     def run(self):
         c = self.case
         M.relpos_attention_dev(lib(), *[t.data_ptr() for t in self.inputs], self.ctx.data_ptr(), c["T"], c["d"], c["H"],
-                               c["left"], c["right"], c["nseq"])
+                               c["left"], c["right"], c["nseq"], self.stream)
         return self.ctx
 
 
@@ -411,7 +424,7 @@ class Layer:
         self.pe = _positions(case["T"], case["d"])
         self.x0 = r.normal(case["nseq"] * case["T"], case["d"])
         self.x = torch.empty_like(self.x0)
-        self.stream = torch.cuda.Stream()
+        self.stream = stream()
 
     def run(self):
         c, (left, right) = self.case, _context(self.case)
@@ -494,10 +507,11 @@ class Subsampling:
                                       int(case["causal"]))
         self.mel = r.normal(case["nseq"] * case["frames"], case["mels"])
         self.out = torch.empty(case["nseq"] * _sub_sizes(case)[0][3], case["d"], device="cuda")
+        self.stream = stream().cuda_stream
 
     def run(self):
         c = self.case
-        self.ss.run(self.mel.data_ptr(), c["frames"], c["nseq"], c["mels"], self.out.data_ptr())
+        self.ss.run(self.mel.data_ptr(), c["frames"], c["nseq"], c["mels"], self.out.data_ptr(), 1.0, self.stream)
         return self.out
 
 
@@ -527,6 +541,9 @@ def _exact_subsampling(case, seed):
 
 
 # ---------------------------------------------------------------------- decoder
+PROMPT = 4   # prompt tokens
+
+
 def _decoder_params(case, r):
     d, f, v, fmt = case["d"], case["f"], case["vocab"], case["fmt"]
     layers = []
@@ -538,29 +555,31 @@ def _decoder_params(case, r):
         for n in ("self", "cross", "ffn"):
             p[f"ln_{n}_w"], p[f"ln_{n}_b"] = r.normal(d, sigma=0.02, mean=1.0), r.normal(d, sigma=0.02)
         layers.append(p)
-    top = {"emb": r.normal(v, d), "pos": r.normal(case["tokens"], d, sigma=0.3),
+    top = {"emb": r.normal(v, d), "pos": r.normal(PROMPT + case["tokens"], d, sigma=0.3),
            "embln_w": r.normal(d, sigma=0.02, mean=1.0), "embln_b": r.normal(d, sigma=0.02),
            "fin_w": r.normal(d, sigma=0.02, mean=1.0), "fin_b": r.normal(d, sigma=0.02), "head": r.weight(fmt, v, d),
            "head_b": r.normal(v, sigma=0.02)}
     enc = r.normal(case["T"], d)
-    tokens = torch.randint(0, v, (case["tokens"],), device="cuda", generator=r.g, dtype=torch.int64)
-    return top, layers, enc, tokens
+    prompt = torch.randint(0, v, (PROMPT,), device="cuda", generator=r.g, dtype=torch.int64)
+    return top, layers, enc, prompt
 
 
 class Decoder:
     def __init__(self, case, seed):
-        top, layers, self.enc, tokens = _decoder_params(case, Draws(seed))
-        self.T, self.keep = case["T"], []
-        self.tokens = np.ascontiguousarray(tokens.cpu().numpy(), np.int32)
+        top, layers, self.enc, prompt = _decoder_params(case, Draws(seed))
+        self.T, self.cap, self.keep = case["T"], case["tokens"], []
+        self.tokens = np.zeros(PROMPT + self.cap, np.int32)   # the prompt, then what is decoded
+        self.tokens[:PROMPT] = prompt.cpu().numpy()
         self.layers = (M.AedLayerC * len(layers))()
         for c, p in zip(self.layers, layers):
             for n, t in p.items():
                 setattr(c, n, self._dev(t))
-        self.c = M.AedC(case["layers"], case["d"], case["H"], case["f"], case["vocab"], case["tokens"])
+        self.c = M.AedC(case["layers"], case["d"], case["H"], case["f"], case["vocab"], PROMPT + self.cap)
         for n, t in top.items():
             setattr(self.c, n, self._dev(t))
         self.c.layers = self.layers
-        self.logits = torch.empty(case["tokens"], case["vocab"], device="cuda")
+        self.logits = torch.empty(PROMPT + self.cap - 1, case["vocab"], device="cuda")
+        self.stream = stream().cuda_stream
 
     def _dev(self, t):
         t = device_weight(t) if isinstance(t, tuple) else t
@@ -568,19 +587,23 @@ class Decoder:
         return t.h if isinstance(t, M.DeviceWeight) else t.data_ptr()
 
     def run(self):
-        rc = lib().L.mynah_asr_hip_aed_forced_dev(ctypes.byref(self.c), self.enc.data_ptr(), self.T,
-                                                  self.tokens.ctypes.data, len(self.tokens), self.logits.data_ptr(), None)
-        if rc != 0:
+        L, c, t = lib().L, ctypes.byref(self.c), self.tokens
+        n = L.mynah_asr_hip_aed_decode_dev(c, self.enc.data_ptr(), self.T, t.ctypes.data, PROMPT, -1,
+                                           t[PROMPT:].ctypes.data, self.cap, self.stream)
+        if n != self.cap or L.mynah_asr_hip_aed_forced_dev(c, self.enc.data_ptr(), self.T, t.ctypes.data,
+                                                           PROMPT + n - 1, self.logits.data_ptr(), self.stream) != 0:
             raise RuntimeError(lib().last_error())
-        return self.logits
+        return t[PROMPT:], self.logits
 
 
 def _exact_decoder(case, seed):
-    """src/decoder_aed.c:139-232 over given tokens, all positions at once (each sees the ones before it)."""
+    """src/decoder_aed.c:139-232 in 64 bits: the prompt's positions and each token's, over all tokens so far."""
     top, layers, enc, tokens = _decoder_params(case, Draws(seed))
     val = lambda t: t[3] if isinstance(t, tuple) else t.double()  # noqa: E731
     top, layers, enc = {n: val(t) for n, t in top.items()}, [{n: val(t) for n, t in p.items()} for p in layers], enc.double()
     H, dk = case["H"], case["d"] // case["H"]
+    lin = lambda a, p, n: a @ p[n].T + p[n + "_b"]  # noqa: E731
+    cross = [(lin(enc, p, "ck"), lin(enc, p, "cv")) for p in layers]
 
     def attend(q, k, v, mask):
         out = torch.empty_like(q)
@@ -590,16 +613,21 @@ def _exact_decoder(case, seed):
             out[:, c] = torch.softmax(s.masked_fill(mask, -math.inf) if mask is not None else s, 1) @ v[:, c]
         return out
 
-    x = _layer_norm64(top["emb"][tokens] + top["pos"], top["embln_w"], top["embln_b"])
-    i = torch.arange(len(tokens), device="cuda")
-    for p in layers:
-        lin = lambda a, n: a @ p[n].T + p[n + "_b"]  # noqa: B023, E731
-        h = _layer_norm64(x, p["ln_self_w"], p["ln_self_b"])
-        x = x + lin(attend(lin(h, "sq"), lin(h, "sk"), lin(h, "sv"), i[None] > i[:, None]), "so")
-        h = _layer_norm64(x, p["ln_cross_w"], p["ln_cross_b"])
-        x = x + lin(attend(lin(h, "cq"), lin(enc, "ck"), lin(enc, "cv"), None), "co")
-        x = x + lin(torch.relu(lin(_layer_norm64(x, p["ln_ffn_w"], p["ln_ffn_b"]), "ff1")), "ff2")
-    return _layer_norm64(x, top["fin_w"], top["fin_b"]) @ top["head"].T + top["head_b"]
+    def logits(tokens):
+        i = torch.arange(len(tokens), device="cuda")
+        x = _layer_norm64(top["emb"][tokens] + top["pos"][i], top["embln_w"], top["embln_b"])
+        for p, kv in zip(layers, cross):
+            h = _layer_norm64(x, p["ln_self_w"], p["ln_self_b"])
+            x = x + lin(attend(lin(h, p, "sq"), lin(h, p, "sk"), lin(h, p, "sv"), i[None] > i[:, None]), p, "so")
+            h = _layer_norm64(x, p["ln_cross_w"], p["ln_cross_b"])
+            x = x + lin(attend(lin(h, p, "cq"), *kv, None), p, "co")
+            x = x + lin(torch.relu(lin(_layer_norm64(x, p["ln_ffn_w"], p["ln_ffn_b"]), p, "ff1")), p, "ff2")
+        return _layer_norm64(x, top["fin_w"], top["fin_b"]) @ top["head"].T + top["head_b"]
+
+    for _ in range(case["tokens"]):
+        out = logits(tokens)
+        tokens = torch.cat([tokens, out[-1:].argmax(1)])
+    return tokens[PROMPT:].to(torch.int32), out
 
 
 # ------------------------------------------------------------------- the contract
@@ -611,7 +639,7 @@ _EXACT = {"linear": _exact_linear, "ffn": _exact_ffn, "attention": _exact_attent
 
 def prepare(case, seed):
     state = _STATE[case["kind"]](case, seed)
-    torch.cuda.synchronize()   # the framework's calls run on its own stream
+    torch.cuda.synchronize()   # the inputs are ready before a call on another stream reads them
     return state
 
 
@@ -653,10 +681,12 @@ def work(case):
                 "flops": 2 * n * C * (9 * (t[1] * f[1] + t[2] * f[2] + t[3] * f[3]) + C * (t[2] * f[2] + t[3] * f[3]) +
                                       t[3] * f[3] * d)}
     d, f, v, T, s = case["d"], case["f"], case["vocab"], case["T"], case["tokens"]
-    per = 6 * wb(d, d) + 2 * wb(f, d)
-    return {"bytes": s * (case["layers"] * (per + 8 * T * d) + wb(v, d) + 4 * v) + case["layers"] * 2 * wb(d, d),
-            "flops": 2 * s * (case["layers"] * (6 * d * d + 2 * d * f + 2 * d * T + d * s) + v * d) +
-            case["layers"] * 4 * T * d * d}
+    n, per = PROMPT + s - 1, case["layers"] * (6 * wb(d, d) + 2 * wb(f, d))
+    # decoding reads the linears and the cross keys and values once a position, scoring once in all
+    return {"bytes": n * (per + wb(v, d) + case["layers"] * 8 * T * d) + per + wb(v, d) + 4 * n * v +
+            2 * case["layers"] * (2 * wb(d, d) + 8 * T * d) + 8 * T * d,
+            "flops": 2 * (2 * n * (case["layers"] * (6 * d * d + 2 * d * f + 2 * d * T + d * n) + v * d) +
+                          case["layers"] * 4 * T * d * d)}
 
 
 def tolerance(case):
