@@ -108,7 +108,6 @@ struct Ctx {
     DBuf enc;    // the encoder layer's activations
     DBuf ssb;    // the subsampling's activations
     DBuf gs;     // split-K GEMV workspace
-    DBuf gk;     // split-K GEMM workspace (chunk results)
     int *pin = nullptr;   // pinned host int[2][2]: the step state of two positions read back
     hipEvent_t pev[2] = {nullptr, nullptr};   // their copies' completion
     PrepBuf pa;  // the products' input (prep_dev / qgemm_prepped_dev use this one)
@@ -286,11 +285,8 @@ int run_from(Ctx *c, const PrepBuf &P, const mynah_asr_hip_weight *W, float *dy,
     if (P.i8 == MH_I8_QMAT) {
         e = mh_launch_gemm_i8(W->qtype, W->dw, (const uint8_t *)P.xp.p, (const float *)P.xs16.p, dy, T, act, st);
     } else {
-        // few tiles: K split over workgroups, through the calling thread's workspace
-        const size_t n = mh_gemm_ws_floats(W->dw, T);
-        float *ws = n ? (float *)c->gk.get(n * sizeof(float)) : nullptr;
         e = mh_launch_gemm(W->qtype, W->dw, (const uint8_t *)P.xp.p, (const float *)P.xs16.p,
-                           (const float *)P.xpf.p, dy, T, act, ws, st, P.i8 != 0);
+                           (const float *)P.xpf.p, dy, T, act, st, P.i8 != 0);
     }
     if (e != hipSuccess) return fail("gemm launch failed", hipGetErrorString(e));
     return 0;
@@ -396,10 +392,8 @@ int qkv_dev(Ctx *c, const mynah_asr_hip_weight *const W[3], const float *dx, flo
         }
         J.n = 3;
         const PrepBuf &P = c->pa;
-        const size_t n = mh_gemm_ws_floats(W[0]->dw, T, 3);
-        float *ws = n ? (float *)c->gk.get(n * sizeof(float)) : nullptr;
         hipError_t e = mh_launch_gemm_jobs(W[0]->qtype, J, (const uint8_t *)P.xp.p, (const float *)P.xs16.p,
-                                           (const float *)P.xpf.p, T, ws, st, P.i8 != 0);
+                                           (const float *)P.xpf.p, T, st, P.i8 != 0);
         if (e != hipSuccess) return fail("gemm launch failed", hipGetErrorString(e));
         return 0;
     }
@@ -761,7 +755,7 @@ int gemm_noalloc(const mynah_asr_hip_weight *W, const float *dx, float *dy, int 
     e = launch_prep(kind, W, dx, T, xp, xs16, xpf, st);
     if (e == hipSuccess) {
         if (kind == MH_I8_QMAT) e = mh_launch_gemm_i8(W->qtype, W->dw, xp, xs16, dy, T, act, st);
-        else e = mh_launch_gemm(W->qtype, W->dw, xp, xs16, xpf, dy, T, act, nullptr, st, kind != 0);
+        else e = mh_launch_gemm(W->qtype, W->dw, xp, xs16, xpf, dy, T, act, st, kind != 0);
     }
     return e == hipSuccess ? 0 : fail("launch failed", hipGetErrorString(e));
 }

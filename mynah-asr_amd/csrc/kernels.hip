@@ -18,317 +18,7 @@
 //
 // The 32x32x16 MFMA is used throughout: on gfx950 it issues twice the work of
 // the 16x16x32 shape per cycle (measured 2.04 vs 1.19 PFLOP/s f16).
-#include "fmt.h"
-#include "launch.h"
-
-#define KSTEPS 4  // ksteps per chunk
-#define HSTEPS 8  // half-steps per chunk
-
-__device__ __forceinline__ f16v mfma32(half8 a, half8 b, f16v c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ f16v zero16() {
-    f16v z;
-#pragma unroll
-    for (int e = 0; e < 16; e++) z[e] = 0.0f;
-    return z;
-}
-
-// D-layout row of accumulator element e for lane half hh
-__device__ __forceinline__ int drow(int e, int hh) { return 8 * (e >> 2) + 4 * hh + (e & 3); }
-
-__device__ __forceinline__ float silu_f(float v) {
-    // x * sigmoid(x) with the reference's stable sigmoid (src/qmat.h:31-35):
-    // exp only of -|x| (never overflows); 1/(1+e) for x >= 0, e/(1+e) below.
-    // Hardware exp2 and reciprocal (~1 ulp each), like the reference's own
-    // -ffast-math build; every kernel applies this same function.
-    const float e = __expf(-fabsf(v));
-    const float r = __builtin_amdgcn_rcpf(1.0f + e);
-    return v * (v >= 0.0f ? r : e * r);
-}
-
-// ---------------------------------------------------------------------------
-// Activation split of one chunk, in the A-operand layout: lane (r = l&31,
-// hh = l>>5) holds elements 16u + 8hh .. +7 of half-step u for row m. The
-// chunk's largest magnitude is shared by the two lanes of a row through one
-// xor shuffle (every lane of the wave must call this).
-struct XChunk {
-    half8 h[HSTEPS], l[HSTEPS];
-    float s8[HSTEPS];  // sum of the lane's 8 scaled values of half-step u, in order
-    float p;           // 2^-sh: the chunk's fold factor for this row
-};
-
-// f16(x0 - h.lo), f16(x1 - h.hi) as one packed pair: x - h is exact in f32
-// (h is x rounded to f16), and v_fma_mixlo / v_fma_mixhi form it with h read as f16 in place
-// and rounds it to f16 once: the value of (_Float16)(x - (float)h), in two
-// instructions per pair instead of six.
-__device__ __forceinline__ uint32_t lo_pair(uint32_t hpair, float x0, float x1) {
-    uint32_t r;
-    asm volatile("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(hpair), "v"(x0));
-    asm volatile("v_fma_mixhi_f16 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-                 : "+v"(r)
-                 : "v"(hpair), "v"(x1));
-    return r;
-}
-
-// the split of NU half-steps' values v[u][j] with shift sh
-template <int NU>
-__device__ __forceinline__ void split_part(const float (&v)[NU][8], int sh, half8 (&h)[NU], half8 (&l)[NU],
-                                           float (&s8)[NU]) {
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-        float acc = 0.0f;
-        float xs[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            xs[j] = ldexpf(v[u][j], sh);
-            h[u][j] = (_Float16)xs[j];
-            acc += xs[j];
-        }
-        s8[u] = acc;
-        uint32_t hw[4], lw[4];
-        __builtin_memcpy(hw, &h[u], 16);
-#pragma unroll
-        for (int t = 0; t < 4; t++) lw[t] = lo_pair(hw[t], xs[2 * t], xs[2 * t + 1]);
-        __builtin_memcpy(&l[u], lw, 16);
-    }
-}
-
-// the split of one chunk's values v[u][j] (element 16u + 8hh + j of row m)
-__device__ __forceinline__ void split_vals(const float (&v)[HSTEPS][8], XChunk &o) {
-    float amax = 0.0f;
-#pragma unroll
-    for (int u = 0; u < HSTEPS; u++)
-#pragma unroll
-        for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(v[u][j]));
-    amax = fmaxf(amax, __shfl_xor(amax, 32));
-    const int sh = chunk_shift(amax);
-    o.p = ldexpf(1.0f, -sh);
-    split_part<HSTEPS>(v, sh, o.h, o.l, o.s8);
-}
-
-// VEC: K % 8 == 0 and 16-byte aligned rows (each lane's 8 elements are
-// wholly inside or wholly past K), two float4 loads per half-step
-template <bool VEC>
-__device__ __forceinline__ void load_chunk(const float *__restrict__ x, int M, int K, int m, int c, int hh,
-                                           float (&v)[HSTEPS][8]) {
-    const bool live = m < M;
-    const float *row = x + (size_t)(live ? m : 0) * K;
-#pragma unroll
-    for (int u = 0; u < HSTEPS; u++) {
-        const int k0 = 128 * c + 16 * u + 8 * hh;
-        if constexpr (VEC) {
-            float4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
-            if (live && k0 < K) {
-                a = *(const float4 *)(row + k0);
-                b = *(const float4 *)(row + k0 + 4);
-            }
-            v[u][0] = a.x; v[u][1] = a.y; v[u][2] = a.z; v[u][3] = a.w;
-            v[u][4] = b.x; v[u][5] = b.y; v[u][6] = b.z; v[u][7] = b.w;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 8; j++) v[u][j] = (live && k0 + j < K) ? row[k0 + j] : 0.0f;
-        }
-    }
-}
-
-template <bool VEC>
-__device__ __forceinline__ void split_chunk(const float *__restrict__ x, int M, int K, int m, int c, int hh,
-                                            XChunk &o) {
-    float v[HSTEPS][8];
-    load_chunk<VEC>(x, M, K, m, c, hh, v);
-    split_vals(v, o);
-}
-
-// ---------------------------------------------------------------------------
-// Weight fragments of WN column groups: per-chunk headers and per-kstep words.
-// Formats whose integer sub-block factors fold into the decoded weights (the
-// FHdr traits): a chunk's MFMAs then accumulate straight through its four
-// ksteps, and the factors d (and the mins, through one more MFMA) apply once
-// per chunk instead of once per sub-block
-template <int QT> constexpr bool fold_fmt() {
-    return QT == QT_Q2_K || QT == QT_Q3_K || QT == QT_Q4_K || QT == QT_Q5_K;
-}
-template <int QT, bool FOLD = fold_fmt<QT>()> struct KHdr { using T = typename Fmt<QT>::Hdr; };
-template <int QT> struct KHdr<QT, true> { using T = typename Fmt<QT>::FHdr; };
-
-template <int QT, int WN> struct BH { typename KHdr<QT>::T h[WN]; };
-template <int QT, int WN> struct BK { typename Fmt<QT>::RawK r[WN]; };
-
-template <int QT, int WN>
-__device__ __forceinline__ void load_bh(const DevW &W, int Kc, const int (&gn)[WN], int c, int lane, BH<QT, WN> &b) {
-#pragma unroll
-    for (int j = 0; j < WN; j++) {
-        if constexpr (fold_fmt<QT>()) Fmt<QT>::load_fhdr(W, Kc, gn[j], c, lane, b.h[j]);
-        else Fmt<QT>::load_hdr(W, Kc, gn[j], c, lane, b.h[j]);
-    }
-}
-template <int QT, int WN>
-__device__ __forceinline__ void load_bk(const DevW &W, int Kc, const int (&gn)[WN], int c, int s, int lane,
-                                        BK<QT, WN> &b) {
-#pragma unroll
-    for (int j = 0; j < WN; j++) Fmt<QT>::load_k(W, Kc, gn[j], c, s, lane, b.r[j]);
-}
-
-// A fragments of one kstep for WM row groups: the two f16 terms of its two
-// half-steps
-template <int WM> struct AK {
-    half8 h[WM][2], l[WM][2];
-};
-
-// The exact product of one kstep into the chunk accumulator. Folded formats:
-// acc += xh*(q f) + xl*(q f) for both half-steps, MFMA after MFMA; the others:
-// t = the kstep's MFMAs from zero, acc = fma(sc, t, acc) per sub-block. The
-// float operations each output sees, and their order, are the same in every
-// caller.
-//
-// A1 (INT8ACT numerics): the activations are int8 values held as f16 (exact),
-// one term: the xl MFMAs drop out, and every sum the MFMAs form is an exact
-// integer (the kernels keep each accumulation below 2^24 in magnitude).
-//
-// NE: the per-element f32 work covers accumulator elements e < NE only (the
-// GEMV of M rows reads elements 0 .. NE-1: rows drow(e, hh) below M); the
-// elements it covers see the same operations at every NE.
-template <int QT, int WM, int WN, bool A1 = false, int NE = 16>
-__device__ __forceinline__ void kstep(const AK<WM> &a, const BK<QT, WN> &b, const BH<QT, WN> &hd, int s,
-                                      f16v (&acc)[WM][WN]) {
-    using F = Fmt<QT>;
-    if constexpr (fold_fmt<QT>()) {
-#pragma unroll
-        for (int j = 0; j < WN; j++) {
-            const half8 b0 = F::decode_f(b.r[j], s, 0, hd.h[j]), b1 = F::decode_f(b.r[j], s, 1, hd.h[j]);
-#pragma unroll
-            for (int i = 0; i < WM; i++) {
-                acc[i][j] = mfma32(a.h[i][0], b0, acc[i][j]);
-                acc[i][j] = mfma32(a.h[i][1], b1, acc[i][j]);
-                if constexpr (!A1) {
-                    acc[i][j] = mfma32(a.l[i][0], b0, acc[i][j]);
-                    acc[i][j] = mfma32(a.l[i][1], b1, acc[i][j]);
-                }
-            }
-        }
-    } else if constexpr (QT == QT_F32) {
-        static_assert(!A1, "f32 weights have no int8-activation form");
-        // f32 weights: resident as (wh, wl) f16 pairs scaled per row by
-        // 2^shw_n; acc += xh*wh + xh*wl + xl*wh straight into the chunk
-        // accumulator (no per-kstep factor)
-#pragma unroll
-        for (int kh = 0; kh < 2; kh++)
-#pragma unroll
-            for (int j = 0; j < WN; j++)
-#pragma unroll
-                for (int i = 0; i < WM; i++) {
-                    acc[i][j] = mfma32(a.h[i][kh], b.r[j].h[kh], acc[i][j]);
-                    acc[i][j] = mfma32(a.h[i][kh], b.r[j].l[kh], acc[i][j]);
-                    acc[i][j] = mfma32(a.l[i][kh], b.r[j].h[kh], acc[i][j]);
-                }
-    } else if constexpr (!F::SUB16) {
-        static_assert(!F::MINS, "affine formats fold");
-#pragma unroll
-        for (int j = 0; j < WN; j++) {
-            const half8 b0 = F::decode(b.r[j], s, 0), b1 = F::decode(b.r[j], s, 1);
-            float sc, mn;
-            F::scale(hd.h[j], s, 0, sc, mn);
-#pragma unroll
-            for (int i = 0; i < WM; i++) {
-                f16v t = mfma32(a.h[i][0], b0, zero16());
-                t = mfma32(a.h[i][1], b1, t);
-                if constexpr (!A1) {
-                    t = mfma32(a.l[i][0], b0, t);
-                    t = mfma32(a.l[i][1], b1, t);
-                }
-#pragma unroll
-                for (int e = 0; e < NE; e++) acc[i][j][e] = __builtin_fmaf(sc, t[e], acc[i][j][e]);
-            }
-        }
-    } else {
-        static_assert(!F::MINS, "affine formats fold");
-#pragma unroll
-        for (int j = 0; j < WN; j++) {
-            half8 b0, b1;
-            if constexpr (QT == QT_Q6_K) {   // the same values, fewer instructions
-                b0 = F::decode_fast(b.r[j], s, 0);
-                b1 = F::decode_fast(b.r[j], s, 1);
-            } else {
-                b0 = F::decode(b.r[j], s, 0);
-                b1 = F::decode(b.r[j], s, 1);
-            }
-            float sc0, mn0, sc1, mn1;
-            F::scale(hd.h[j], s, 0, sc0, mn0);
-            F::scale(hd.h[j], s, 1, sc1, mn1);
-#pragma unroll
-            for (int i = 0; i < WM; i++) {
-                f16v t0 = mfma32(a.h[i][0], b0, zero16());
-                if constexpr (!A1) t0 = mfma32(a.l[i][0], b0, t0);
-                f16v t1 = mfma32(a.h[i][1], b1, zero16());
-                if constexpr (!A1) t1 = mfma32(a.l[i][1], b1, t1);
-#pragma unroll
-                for (int e = 0; e < NE; e++) {
-                    acc[i][j][e] = __builtin_fmaf(sc0, t0[e], acc[i][j][e]);
-                    acc[i][j][e] = __builtin_fmaf(sc1, t1[e], acc[i][j][e]);
-                }
-            }
-        }
-    }
-}
-
-// The affine folded formats' row sums as the A operand of the chunk's mins
-// MFMA: sub-block sum x_j (NS per chunk: the 16-element sums (first 8 in
-// order) + (next 8), for 32-element sub-blocks two of them added) scaled by
-// 2^-5 (|x_j| < 2^20, so the result fits f16) and split into f16 hi_j + lo_j;
-// lane half 0 carries hi_j in slot j, half 1 lo_j, slots >= NS are zero. The
-// mins product is then sum_j (hi_j + lo_j) * m_j = 2^-5 * sum_j x_j m_j.
-__device__ __forceinline__ _Float16 xm_part(float xsum, int hh) {
-    const float v = xsum * 0.03125f;
-    const _Float16 hi = (_Float16)v;
-    return hh ? (_Float16)(v - (float)hi) : hi;
-}
-template <int NS>
-__device__ __forceinline__ half8 xm_frag(const float (&s8)[HSTEPS], int hh) {
-    float s16[HSTEPS];
-#pragma unroll
-    for (int u = 0; u < HSTEPS; u++) s16[u] = s8[u] + __shfl_xor(s8[u], 32);
-    half8 r;
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        if (j < NS) r[j] = xm_part(NS == 8 ? s16[j] : s16[2 * j] + s16[2 * j + 1], hh);
-        else r[j] = (_Float16)0.0f;
-    }
-    return r;
-}
-
-// End of a chunk of a folded format: acc (= sum of x * q f over the chunk)
-// becomes d * acc - dm * (mins product), the chunk result the fold takes
-template <int QT, int NE = 16>
-__device__ __forceinline__ void fold_finish(const half8 &xm, const typename KHdr<QT>::T &H, f16v &acc) {
-    if constexpr (Fmt<QT>::MINS) {
-        const f16v t2 = mfma32(xm, H.mb, zero16());
-#pragma unroll
-        for (int e = 0; e < NE; e++) acc[e] = __builtin_fmaf(-H.dm, t2[e], H.d * acc[e]);
-    } else {
-#pragma unroll
-        for (int e = 0; e < NE; e++) acc[e] = H.d * acc[e];
-    }
-}
-
-// the per-row weight shift of the f32 format (0 for the quantized ones)
-template <int QT>
-__device__ __forceinline__ int wshift(const DevW &W, int n) {
-    if constexpr (QT == QT_F32) return (int)W.h2[n];
-    return 0;
-}
-
-__device__ __forceinline__ f16v load_rows16(const float *b) {
-    // the lane's 16 D-layout rows from a [32]-row float vector (b at row 4*hh)
-    f16v r;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const float4 v = *(const float4 *)(b + 8 * q);
-        r[4 * q + 0] = v.x; r[4 * q + 1] = v.y; r[4 * q + 2] = v.z; r[4 * q + 3] = v.w;
-    }
-    return r;
-}
+#include "product.h"
 
 // ---------------------------------------------------------------------------
 // Global -> LDS copies (global_load_lds: no VGPRs; the LDS destination is
@@ -406,24 +96,6 @@ template <int QT, bool A1 = false, int NCG = 4, int NRG = 2, bool BD = false> st
     static constexpr int BYTES = XS + (F::MINS ? NRG * 1024 : 0);
 };
 
-// Where a product's result goes: EPI_Y stores y (SiLU applied when act);
-// EPI_PREP (the first product of the FFN) applies SiLU and, instead of
-// storing the f32 intermediate, prepares it as the second product's input —
-// the workgroup's 128 output columns are exactly one 128-element chunk of
-// the second product's K, so the chunk's shift, split and sums are formed
-// here by split_part, the same function the preparation pass runs, on the
-// same f32 values (bit-identical to storing y and preparing it).
-enum { EPI_Y = 0, EPI_PREP = 1, EPI_PART = 2 };
-// EPI_PART (launches with few tiles): workgroup (tile, split) runs one range
-// of chunks and stores each chunk's result to part[c][Mpad][Np] instead of
-// folding it; k_gemm_fold then folds them in chunk order from zero, with the
-// prepared input's fold factors: the operations the fold in registers runs.
-struct PrepOut {
-    uint8_t *xp, *xm;
-    float *xpf;
-    int Kc, xsum;   // mins A operands (xm_frag): 0 none, 1 of 8 sub-blocks, 2 of 4
-};
-
 // workgroups per CU the register budget is sized for: as many as the LDS
 // ring allows (three double-buffered workgroups: 25-27 KiB stages, 24 KiB
 // one-kstep stages for f32 weights; four of 32-row tiles, three for f32
@@ -437,21 +109,10 @@ struct PrepOut {
 #ifndef GQ_OCC
 #define GQ_OCC 3
 #endif
-// The products' output epilogue (k_gemm_fold's; k_gemm's spells it out): act
-// 1 SiLU; act 2 and 3 accumulate into y, y = fmaf(1 or 1/2, v, y) (the
-// residual adds x += tmp and x += tmp / 2 of the encoder layer, with their
-// operations); otherwise v.
-__device__ __forceinline__ float epi_out(int act, float v, const float *yp) {
-    if (act == 1) return silu_f(v);
-    if (act >= 2) return fmaf(act == 3 ? 0.5f : 1.0f, v, *yp);
-    return v;
-}
-
 template <int QT, int EPI, bool A1 = false, int WN = 1, int WM = 2> constexpr int gemm_occ() {
-    if (QT == QT_Q8_0 && !A1 && WN == 1 && WM == 2 && EPI != EPI_PART) return GQ_OCC;
+    if (QT == QT_Q8_0 && !A1 && WN == 1 && WM == 2) return GQ_OCC;
     if (WN > 1) return 2;
     if (WM == 1) return QT == QT_Q6_K || QT == QT_F32 ? 3 : 4;
-    if (EPI == EPI_PART && (QT == QT_INT4 || (A1 && QT == QT_Q5_K))) return 2;
     return QT == QT_Q6_K ? 2 : 3;
 }
 
@@ -480,7 +141,7 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
                                                  const uint8_t *__restrict__ xm,
                                                  const float *__restrict__ xpf,
                                                  int M, int act, int tilesM, int tilesN, PrepOut po,
-                                                 float *__restrict__ part, int ksplit, int ngrp) {
+                                                 int ngrp) {
     using F = Fmt<QT>;
     // the weight planes go straight to registers, one stage ahead (measured
     // 3-6% faster than through LDS on every format: less LDS traffic), except
@@ -488,7 +149,7 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
     // them: with them it spilled, and 4096->1024 at 750 rows took 129 us, not
     // 50) and, for f32 weights, in the FFN's fused form (its epilogue's LDS
     // tile needs the larger stages)
-    constexpr bool BD = EPI != EPI_PART && (QT != QT_F32 || EPI == EPI_Y);
+    constexpr bool BD = QT != QT_F32 || EPI == EPI_Y;
     using L = StageLayout<QT, A1, 4 * WN, WM, BD>;
     typename F::RawK rb[2][WN][L::SPS];   // BD: the weight planes of the stage in flight and the current one
     static_assert(!(A1 && EPI == EPI_PREP), "the fused FFN hand-off is EXACT only");
@@ -504,29 +165,16 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
     // Several products of one input (J.n jobs) share the row bands: the tiles
     // of band tm are (job, column tile) pairs, so one XCD runs all of a band's
     // products and reads its activations into its L2 once.
-    // With EPI_PART, a band's splits follow each other (band, split, tile).
-    // Without a K split, the order is N-group-major with ngrp groups of
+    // The order is N-group-major with ngrp groups of
     // column tiles (ngrp divides nj * tilesN), band-major inside a group: an
     // XCD's run then covers the bands of one group only, so the group's
     // slice of the weights can stay in its L2 while the bands stream past
     // (the host picks ngrp from the operand sizes; 1 = plain band-major).
-    const int KS = EPI == EPI_PART ? ksplit : 1;
-    const int nj = J.n, nt = nj * tilesN, ntiles = nt * tilesM * KS, bid = blockIdx.x;
+    const int nj = J.n, nt = nj * tilesN, ntiles = nt * tilesM, bid = blockIdx.x;
     const int q = ntiles / 8, rem = ntiles % 8, xcd = bid % 8, loc = bid / 8;
     const int t = xcd < rem ? xcd * (q + 1) + loc : rem * (q + 1) + (xcd - rem) * q + loc;
-    int tm, ks, tr;
-    if (EPI == EPI_PART) {
-        tm = t / (nt * KS);
-        const int ts = t - tm * nt * KS;
-        ks = ts / nt;
-        tr = ts - ks * nt;
-    } else {
-        const int ntg = nt / ngrp, per = tilesM * ntg;
-        const int g = t / per, r = t - g * per;
-        tm = r / ntg;
-        tr = g * ntg + (r - tm * ntg);
-        ks = 0;
-    }
+    const int ntg = nt / ngrp, per = tilesM * ntg;
+    const int g = t / per, r = t - g * per, tm = r / ntg, tr = g * ntg + (r - tm * ntg);
     const int job = tr / tilesN, tn = tr - job * tilesN;
     const DevW W = job == 0 ? J.W[0] : (job == 1 ? J.W[1] : J.W[2]);
     float *__restrict__ y = job == 0 ? J.y[0] : (job == 1 ? J.y[1] : J.y[2]);
@@ -535,8 +183,6 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
     const int hh = lane >> 5, col = lane & 31;
     const int Kc = W.Kp / 128;
     const int G0 = tm * WM, GC0 = tn * 4 * WN;   // wave w: column groups GC0 + WN w + j
-    const int cps = (Kc + KS - 1) / KS;
-    const int c0 = EPI == EPI_PART ? ks * cps : 0, c1 = EPI == EPI_PART ? min(c0 + cps, Kc) : Kc;
 
     auto stage = [&](int c, int q, uint8_t *B) {
         const int rg = wave / WPR, pw = wave % WPR;
@@ -624,8 +270,8 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
     for (int i = 0; i < WM; i++)
 #pragma unroll
         for (int j = 0; j < WN; j++) total[i][j] = zero16();
-    if (EPI != EPI_PART || c0 < c1) stage(c0, 0, sbuf[0]);
-    for (int c = c0; c < c1; c++) {
+    stage(0, 0, sbuf[0]);
+    for (int c = 0; c < Kc; c++) {
         BH<QT, WN> hd;
         f16v acc[WM][WN];
         int half0[HALVES ? WM : 1][HALVES ? WN : 1][HALVES ? 16 : 1];
@@ -642,7 +288,7 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
             wait_vm<0>();
             __syncthreads();
             if (q + 1 < L::NST) stage(c, q + 1, sbuf[(q + 1) & 1]);
-            else if (c + 1 < c1) stage(c + 1, 0, sbuf[0]);
+            else if (c + 1 < Kc) stage(c + 1, 0, sbuf[0]);
             if (q == 0) {
                 // the chunk's factors, from its headers (staged with every stage)
 #pragma unroll
@@ -686,18 +332,6 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
                 for (int j = 0; j < WN; j++) fold_finish<QT>(xmv, hd.h[j], acc[i][j]);
             }
         }
-        if constexpr (EPI == EPI_PART) {
-            const size_t Mp = (size_t)tilesM * 32 * WM;
-#pragma unroll
-            for (int j = 0; j < WN; j++) {
-                float *pc = part + ((size_t)job * Kc + c) * Mp * W.Np + 32 * (GC0 + WN * wave + j) + col;
-#pragma unroll
-                for (int i = 0; i < WM; i++)
-#pragma unroll
-                    for (int e = 0; e < 16; e++) pc[(size_t)(32 * (G0 + i) + drow(e, hh)) * W.Np] = acc[i][j][e];
-            }
-            continue;
-        }
 #pragma unroll
         for (int i = 0; i < WM; i++) {
             const f16v pv = lds_rows16(sbuf[1] + L::PF + i * 128, hh);
@@ -708,7 +342,6 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
         }
     }
     wait_vm<0>();
-    if constexpr (EPI == EPI_PART) return;
     if constexpr (EPI == EPI_PREP) {
         // the 64 x 128 SiLU tile through LDS (row stride 132 floats: 16-byte
         // aligned rows), then wave w splits half-steps 4*(w>>1) .. +3 of row
@@ -814,52 +447,6 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
                 if constexpr (QT == QT_F32) v = ldexpf(v, -shw);
                 y[(size_t)m * W.n + n] = act ? silu_f(v) : v;
             }
-    }
-}
-
-// The fold of EPI_PART's chunk results: y[m][n] from part[job][c][m][n], c
-// in order from zero, with factor xpf[m/32][c][m%32] (what k_gemm stages as
-// the chunk's fold factors), then k_gemm's own epilogue. Thread = (row m, four
-// columns), blockIdx.y = job; the loads go out eight chunks at a time.
-template <int QT>
-__global__ __launch_bounds__(256) void k_gemm_fold(GemmJobs J, const float *__restrict__ part,
-                                                   const float *__restrict__ xpf, int M, int Mp, int act) {
-    const int job = blockIdx.y;
-    const DevW W = job == 0 ? J.W[0] : (job == 1 ? J.W[1] : J.W[2]);
-    float *__restrict__ y = job == 0 ? J.y[0] : (job == 1 ? J.y[1] : J.y[2]);
-    const int n4 = W.Np / 4;
-    const int idx = blockIdx.x * 256 + threadIdx.x;
-    const int m = idx / n4, n = 4 * (idx - m * n4);
-    if (m >= M) return;
-    const int Kc = W.Kp / 128;
-    const float *pf = xpf + (size_t)(m >> 5) * Kc * 32 + (m & 31);
-    const float *pp = part + (size_t)job * Kc * Mp * W.Np + (size_t)m * W.Np + n;
-    float total[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int c0 = 0; c0 < Kc; c0 += 8) {
-        float4 pv[8];
-        float fv[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-            if (c0 + u < Kc) {
-                pv[u] = *(const float4 *)(pp + (size_t)(c0 + u) * Mp * W.Np);
-                fv[u] = pf[(c0 + u) * 32];
-            }
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-            if (c0 + u < Kc) {
-                total[0] = __builtin_fmaf(fv[u], pv[u].x, total[0]);
-                total[1] = __builtin_fmaf(fv[u], pv[u].y, total[1]);
-                total[2] = __builtin_fmaf(fv[u], pv[u].z, total[2]);
-                total[3] = __builtin_fmaf(fv[u], pv[u].w, total[3]);
-            }
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        if (n + j >= W.n) return;
-        float v = total[j];
-        if constexpr (QT == QT_F32) v = ldexpf(v, -wshift<QT>(W, n + j));
-        float *yp = y + (size_t)m * W.n + n + j;
-        *yp = epi_out(act, v, yp);
     }
 }
 
@@ -2093,36 +1680,6 @@ static hipError_t gemv_t(const GJobs &J, const float *x, int M, int vec, const G
     return launch_gemv<QT, 4, 1>(J, x, M, vec, pro, st);
 }
 
-// K split for a launch of few tiles (at most one workgroup per CU otherwise,
-// each running its chunks as one long dependent chain): enough (tile, split)
-// workgroups for three per CU, none of them empty. 1: no split. It pays when
-// the chain it shortens is long (16 chunks or more) or the chunk results the
-// fold reads back are few (outputs of at most 512K elements over all jobs);
-// measured on 1024 -> 1024 at M = 750 (8 chunks, 786K outputs), and on three
-// such products at M = 256, it does not.
-static int gemm_ksplit(int Kc, int tiles, size_t outs) {
-    if (tiles > 256 || Kc < 2 || (Kc < 16 && outs > ((size_t)512 << 10))) return 1;
-    if ((size_t)Kc * outs > ((size_t)64 << 20)) return 1;   // workspace above 256 MiB: unsplit
-    int s = (768 + tiles - 1) / tiles;
-    if (s > Kc) s = Kc;
-    const int cps = (Kc + s - 1) / s;
-    return (Kc + cps - 1) / cps;
-}
-
-size_t mh_gemm_ws_floats(const DevW &W, int M, int jobs) {
-    const int Kc = W.Kp / 128, tilesM = mh_mpad(M) / 64;
-    const size_t outs = (size_t)jobs * tilesM * 64 * W.Np;   // over all jobs
-    if (W.Np % 128 != 0 || gemm_ksplit(Kc, jobs * tilesM * (W.Np / 128), outs) == 1) return 0;
-    return (size_t)Kc * outs;
-}
-
-// Weight bytes per element of the resident layout (planes and headers)
-template <int QT> constexpr float w_bpe() {
-    return QT == QT_F32 ? 4.0f : QT == QT_INT8 ? 1.0f : QT == QT_INT4 ? 0.5625f : QT == QT_Q4_0 ? 0.5625f
-         : QT == QT_Q8_0 ? 1.0625f : QT == QT_Q2_K ? 0.33f : QT == QT_Q3_K ? 0.43f : QT == QT_Q4_K ? 0.5625f
-         : QT == QT_Q5_K ? 0.6875f : 0.82f;
-}
-
 // Column-tile groups of the tile order (k_gemm's ngrp): the count in {1, 2, 4}
 // that minimises a model of the L2 misses. Each XCD runs about 96 tiles at a
 // time (32 CUs x 3) out of an L2 of 4 MB. A group's weight slice that fits
@@ -2182,7 +1739,7 @@ static bool gemm_wide(const DevW &W, int tilesM, int jobs) {
 
 template <int QT, bool A1>
 static hipError_t gemm_launch(const GemmJobs &J, const uint8_t *xp, const float *xs16, const float *xpf, int M,
-                              int act, const PrepOut *po, float *ws, hipStream_t st) {
+                              int act, const PrepOut *po, hipStream_t st) {
     const DevW &W = J.W[0];
     const int mpad = mh_mpad(M);
     if (mpad % 64 != 0 || W.Np % 128 != 0 || J.n < 1 || J.n > 3) return hipErrorInvalidValue;
@@ -2191,36 +1748,30 @@ static hipError_t gemm_launch(const GemmJobs &J, const uint8_t *xp, const float 
     const int tilesM = mpad / 64, tilesN = W.Np / 128, grid = J.n * tilesM * tilesN;
     const int ngrp = gemm_ngroups(w_bpe<QT>() * W.Np * W.Kp * J.n, (A1 ? 2.0f : 4.0f) * mpad * W.Kp, tilesM,
                                   J.n * tilesN);
+    if (po && (po->Kc != tilesN || J.n != 1)) return hipErrorInvalidValue;
+    if (mh_use_gemm_ks(W, M, J.n, po != nullptr)) return mh_launch_gemm_ks(QT, J, xp, xs16, xpf, M, act, po, A1, st);
     if (po) {
         if constexpr (A1) {
             return hipErrorInvalidValue;
         } else {
-            if (po->Kc != tilesN || J.n != 1) return hipErrorInvalidValue;
             hipLaunchKernelGGL((k_gemm<QT, EPI_PREP>), dim3(grid), dim3(256), 0, st, J, xp, (const uint8_t *)xs16,
-                               xpf, M, 1, tilesM, tilesN, *po, nullptr, 1, ngrp);
+                               xpf, M, 1, tilesM, tilesN, *po, ngrp);
             return hipGetLastError();
         }
     }
-    const int ks = ws ? gemm_ksplit(W.Kp / 128, grid, (size_t)J.n * mpad * W.Np) : 1;
-    if (ks > 1) {
-        hipLaunchKernelGGL((k_gemm<QT, EPI_PART, A1>), dim3(grid * ks), dim3(256), 0, st, J, xp,
-                           (const uint8_t *)xs16, xpf, M, act, tilesM, tilesN, PrepOut{}, ws, ks, 1);
-        const int threads = M * (W.Np / 4);
-        hipLaunchKernelGGL((k_gemm_fold<QT>), dim3((threads + 255) / 256, J.n), dim3(256), 0, st, J, (const float *)ws,
-                           xpf, M, mpad, act);
-    } else if (gemm_narrow(grid)) {
+    if (gemm_narrow(grid)) {
         hipLaunchKernelGGL((k_gemm<QT, EPI_Y, A1, 1, 1>), dim3(2 * grid), dim3(256), 0, st, J, xp,
-                           (const uint8_t *)xs16, xpf, M, act, 2 * tilesM, tilesN, PrepOut{}, nullptr, 1, ngrp);
+                           (const uint8_t *)xs16, xpf, M, act, 2 * tilesM, tilesN, PrepOut{}, ngrp);
     } else if (gemm_wide<QT, A1>(W, tilesM, J.n)) {
         if constexpr (wide_fmt<QT, A1>()) {   // (the other formats never instantiate it)
             const int tN2 = W.Np / 256, ng2 = gemm_ngroups(w_bpe<QT>() * W.Np * W.Kp * J.n,
                                                           (A1 ? 2.0f : 4.0f) * mpad * W.Kp, tilesM, J.n * tN2);
             hipLaunchKernelGGL((k_gemm<QT, EPI_Y, A1, 2>), dim3(J.n * tilesM * tN2), dim3(256), 0, st, J, xp,
-                               (const uint8_t *)xs16, xpf, M, act, tilesM, tN2, PrepOut{}, nullptr, 1, ng2);
+                               (const uint8_t *)xs16, xpf, M, act, tilesM, tN2, PrepOut{}, ng2);
         }
     } else {
         hipLaunchKernelGGL((k_gemm<QT, EPI_Y, A1>), dim3(grid), dim3(256), 0, st, J, xp, (const uint8_t *)xs16, xpf,
-                           M, act, tilesM, tilesN, PrepOut{}, nullptr, 1, ngrp);
+                           M, act, tilesM, tilesN, PrepOut{}, ngrp);
     }
     return hipGetLastError();
 }
@@ -2229,30 +1780,15 @@ static hipError_t gemm_launch(const GemmJobs &J, const uint8_t *xp, const float 
 // formats INT8 / INT4 and f32 weights have none
 template <int QT>
 static hipError_t gemm_t(const GemmJobs &J, const uint8_t *xp, const float *xs16, const float *xpf, int M,
-                         int act, const PrepOut *po, float *ws, hipStream_t st, bool a1 = false) {
+                         int act, const PrepOut *po, hipStream_t st, bool a1 = false) {
     if constexpr (QT == QT_F32 || QT == QT_INT8 || QT == QT_INT4) {
         if (a1) return hipErrorInvalidValue;
-        return gemm_launch<QT, false>(J, xp, xs16, xpf, M, act, po, ws, st);
+        return gemm_launch<QT, false>(J, xp, xs16, xpf, M, act, po, st);
     } else {
-        if (a1) return gemm_launch<QT, true>(J, xp, xs16, xpf, M, act, po, ws, st);
-        return gemm_launch<QT, false>(J, xp, xs16, xpf, M, act, po, ws, st);
+        if (a1) return gemm_launch<QT, true>(J, xp, xs16, xpf, M, act, po, st);
+        return gemm_launch<QT, false>(J, xp, xs16, xpf, M, act, po, st);
     }
 }
-
-#define MH_DISPATCH(fn, qtype, ...)                                  \
-    switch (qtype) {                                                 \
-    case QT_F32: return fn<QT_F32>(__VA_ARGS__);                     \
-    case QT_INT8: return fn<QT_INT8>(__VA_ARGS__);                   \
-    case QT_INT4: return fn<QT_INT4>(__VA_ARGS__);                   \
-    case QT_Q4_0: return fn<QT_Q4_0>(__VA_ARGS__);                   \
-    case QT_Q8_0: return fn<QT_Q8_0>(__VA_ARGS__);                   \
-    case QT_Q2_K: return fn<QT_Q2_K>(__VA_ARGS__);                   \
-    case QT_Q3_K: return fn<QT_Q3_K>(__VA_ARGS__);                   \
-    case QT_Q4_K: return fn<QT_Q4_K>(__VA_ARGS__);                   \
-    case QT_Q5_K: return fn<QT_Q5_K>(__VA_ARGS__);                   \
-    case QT_Q6_K: return fn<QT_Q6_K>(__VA_ARGS__);                   \
-    }                                                                \
-    return hipErrorInvalidValue;
 
 bool mh_use_gemv(const DevW &W, int M) { return M <= 16 && (W.Kp / 128) * gemv_wng(W) <= 64; }
 
@@ -2315,17 +1851,17 @@ hipError_t mh_launch_gemv(int qtype, const DevW &W, const float *x, int M, int v
 }
 
 hipError_t mh_launch_gemm(int qtype, const DevW &W, const uint8_t *xp, const float *xs16,
-                          const float *xpf, float *y, int M, int act, float *ws, hipStream_t st, bool a1) {
+                          const float *xpf, float *y, int M, int act, hipStream_t st, bool a1) {
     GemmJobs J{};
     J.W[0] = J.W[1] = J.W[2] = W;
     J.y[0] = J.y[1] = J.y[2] = y;
     J.n = 1;
-    MH_DISPATCH(gemm_t, qtype, J, xp, xs16, xpf, M, act, nullptr, ws, st, a1)
+    MH_DISPATCH(gemm_t, qtype, J, xp, xs16, xpf, M, act, nullptr, st, a1)
 }
 
 hipError_t mh_launch_gemm_jobs(int qtype, const GemmJobs &J, const uint8_t *xp, const float *xs16,
-                               const float *xpf, int M, float *ws, hipStream_t st, bool a1) {
-    MH_DISPATCH(gemm_t, qtype, J, xp, xs16, xpf, M, 0, nullptr, ws, st, a1)
+                               const float *xpf, int M, hipStream_t st, bool a1) {
+    MH_DISPATCH(gemm_t, qtype, J, xp, xs16, xpf, M, 0, nullptr, st, a1)
 }
 
 hipError_t mh_launch_gemm_prep_out(int qtype, const DevW &W, const uint8_t *xp, const float *xs16,
@@ -2335,7 +1871,7 @@ hipError_t mh_launch_gemm_prep_out(int qtype, const DevW &W, const uint8_t *xp, 
     GemmJobs J{};
     J.W[0] = J.W[1] = J.W[2] = W;
     J.n = 1;
-    MH_DISPATCH(gemm_t, qtype, J, xp, xs16, xpf, M, 1, &po, nullptr, st)
+    MH_DISPATCH(gemm_t, qtype, J, xp, xs16, xpf, M, 1, &po, st)
 }
 
 hipError_t mh_launch_read_floor(const void *p, size_t bytes, hipStream_t st) {
