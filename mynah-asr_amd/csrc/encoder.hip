@@ -12,8 +12,8 @@
 //   k_dwconv    depthwise conv over time within each segment (causal: left
 //               pad k-1; else 'same'), + dw_b, then the folded batch norm
 //               x * scale + shift and SiLU when scale is given     :434-459
-//   k_dwconv_tile  the same on LDS tiles of 32 rows, optionally forming the
-//               GLU as it stages its input
+//   k_dwconv_tile  the same on LDS tiles, forming the GLU as it stages its
+//               input
 //
 // and of the dw_striding subsampling in front of the layers
 // (src/subsampling.c:208-268, 109-200), with activations channel-last,
@@ -35,11 +35,13 @@
 
 namespace {
 
-// the reference's stable sigmoid (src/qmat.h:31-35): exp only of -|x|
+// the reference's stable sigmoid (src/qmat.h:31-35): exp only of -|x|, 1 / (1 +
+// e) for x >= 0, e / (1 + e) below. One exponential and one division whatever
+// the sign (as two branches a wave runs both: GLU and conv of 12000 x 1024 at
+// 63 us, a third of it these).
 __device__ __forceinline__ float sigmoid_f(float x) {
-    if (x >= 0.0f) return 1.0f / (1.0f + expf(-x));
-    const float e = expf(x);
-    return e / (1.0f + e);
+    const float e = expf(x >= 0.0f ? -x : x);
+    return (x >= 0.0f ? 1.0f : e) / (1.0f + e);
 }
 
 // One wave per row of d = 256 V4 floats (lane l holds elements 4l + 256u ..
@@ -225,58 +227,84 @@ __global__ __launch_bounds__(256) void k_dwconv(const float *__restrict__ g, con
     *(float4 *)(out + (size_t)row * d + i) = o;
 }
 
-// The same in tiles: a workgroup = DW_R rows of one segment x 256 channels.
-// The rows t0 - pc .. t0 + DW_R - 1 - pc + k - 1 of g (zero outside the
-// segment) and the k taps are staged in LDS once, so each input row is read
-// from memory once per tile instead of once per tap; thread = (4 channels,
-// every 4th row of the tile). Per output the operations and their order are
-// those of k_dwconv (taps outside the segment skipped, not added as zeros).
-// GLU: g is formed from pw1's output h [rows][2d] as it is staged (k_glu's
+// The same in tiles: a workgroup = R rows of one segment x 256 channels. The
+// rows t0 - pc .. t0 + R - 1 - pc + k - 1 of the GLU (zero outside the segment) are
+// staged in LDS once, so each input row is read from memory once per tile
+// instead of once per tap; wave w = rows R/4 w .. of the tile, lane = 4
+// channels. Per output the operations and their order are those of k_dwconv
+// (taps outside the segment skipped, not added as zeros).
+// The GLU is formed from pw1's output h [rows][2d] as it is staged (k_glu's
 // operations; the halo rows' values are formed again by the next tile).
-constexpr int DW_R = 32;
 // PREP: the output rows are written as the EXACT products' prepared input
 // (xp, xpf, for M = nseq T rows padded to 64, as k_add_ln_prep writes it)
 // instead of into out: per (row, 128-channel chunk: 32 lanes) the split the
 // preparation forms, held in registers until the tile is done, then staged
 // in the input rows' LDS so the stores run along rows.
-template <bool GLU, bool PREP>
+//
+// K: the kernel width where it is known at compile time (0: at run time). Then
+// a tile that touches no segment end keeps its taps in registers and slides
+// along its rows, reading each staged row once per wave instead of once per tap.
+// R: 32 rows, or 8 when 32-row tiles are fewer than the CUs (a segment of 63
+// frames is 8 tiles of 32 rows: each one long chain of loads; the halo, 8 rows
+// per tile at width 9, is then read twice as often, from L2).
+template <bool PREP, int R, int K>
 __global__ __launch_bounds__(256) void k_dwconv_tile(const float *__restrict__ g, const float *__restrict__ w,
                                                      const float *__restrict__ bias, const float *__restrict__ scale,
                                                      const float *__restrict__ shift, float *__restrict__ out,
-                                                     int T, int d, int k, int pc, uint8_t *__restrict__ xp,
+                                                     int T, int d, int kr, int pc, uint8_t *__restrict__ xp,
                                                      float *__restrict__ xpf) {
-    // [DW_R + k - 1][64] rows of g, then [k][64] taps; PREP, once the tile is
-    // done: the staged slots [DW_R rows][2 chunks][8 half-steps][2 terms][2
-    // halves] over the rows, the fold factors [DW_R][2] over the taps
+    // [R + k - 1][64] rows of g, then [k][64] taps; PREP, once the tile is
+    // done: the staged slots [R rows][2 chunks][8 half-steps][2 terms][2
+    // halves] over the rows, the fold factors [R][2] over the taps
     extern __shared__ float4 dws[];
-    uint2 ph[PREP ? DW_R / 4 : 1], pl[PREP ? DW_R / 4 : 1];
-    float pf[PREP ? DW_R / 4 : 1];
-    const int tid = threadIdx.x, q = tid & 63, t0 = blockIdx.x * DW_R, c0 = blockIdx.y * 256;
-    const int nrow = DW_R + k - 1;
-    const int gw = GLU ? 2 * d : d;   // the input's row width
+    constexpr int RW = R / 4;   // rows per wave
+    uint2 ph[PREP ? RW : 1], pl[PREP ? RW : 1];
+    float pf[PREP ? RW : 1];
+    const int k = K ? K : kr;
+    const int tid = threadIdx.x, q = tid & 63, t0 = blockIdx.x * R, c0 = blockIdx.y * 256;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nrow = R + k - 1;
+    const int gw = 2 * d;   // the input's row width
     const float *gs = g + (size_t)blockIdx.z * T * gw + c0;
     float4 *taps = dws + nrow * 64;
-    for (int i = tid; i < nrow * 64; i += 256) {
-        const int t = t0 - pc + (i >> 6);
-        float4 o = {0.f, 0.f, 0.f, 0.f};
-        if (t >= 0 && t < T) {
-            const float *p = gs + (size_t)t * gw + 4 * (i & 63);
-            o = *(const float4 *)p;
-            if constexpr (GLU) {
-                const float4 b = *(const float4 *)(p + d);
-                o = float4{o.x * sigmoid_f(b.x), o.y * sigmoid_f(b.y), o.z * sigmoid_f(b.z), o.w * sigmoid_f(b.w)};
+    // the taps of w [d][k] written tap-major (each tap of 4 channels one
+    // float4): thread = channel c0 + tid, its k taps, loaded ahead of the rows
+    constexpr int KT = K ? K : 16;
+    float tv[KT];
+    const float *wc = w + (size_t)(c0 + tid) * k;
+#pragma unroll
+    for (int j = 0; j < KT; j++) tv[j] = j < k ? wc[j] : 0.0f;
+    constexpr int UB = 4;   // rows of a wave in flight
+    for (int i0 = wave; i0 < nrow; i0 += 4 * UB) {
+        float4 a[UB], b[UB];
+#pragma unroll
+        for (int u = 0; u < UB; u++) {
+            const int r = i0 + 4 * u, t = t0 - pc + r;
+            a[u] = float4{0.f, 0.f, 0.f, 0.f};
+            b[u] = a[u];
+            if (r < nrow && t >= 0 && t < T) {
+                const float *p = gs + (size_t)t * gw + 4 * q;
+                a[u] = *(const float4 *)p;
+                b[u] = *(const float4 *)(p + d);
             }
         }
-        dws[i] = o;
+#pragma unroll
+        for (int u = 0; u < UB; u++) {
+            const int r = i0 + 4 * u, t = t0 - pc + r;
+            if (r >= nrow) continue;
+            float4 o = a[u];
+            if (t >= 0 && t < T)
+                o = float4{o.x * sigmoid_f(b[u].x), o.y * sigmoid_f(b[u].y), o.z * sigmoid_f(b[u].z),
+                           o.w * sigmoid_f(b[u].w)};
+            dws[r * 64 + q] = o;
+        }
     }
-    // the taps of w [d][k] written tap-major (each tap of 4 channels one
-    // float4): thread = channel c0 + tid, its k taps
     {
         float *tf = (float *)taps;
-        const float *wc = w + (size_t)(c0 + tid) * k;
-        for (int j = 0; j < k; j++) tf[j * 256 + tid] = wc[j];
+#pragma unroll
+        for (int j = 0; j < KT; j++)
+            if (j < k) tf[j * 256 + tid] = tv[j];
     }
-    __syncthreads();
     const int i = c0 + 4 * q;
     const float4 b0 = bias ? *(const float4 *)(bias + i) : float4{0.f, 0.f, 0.f, 0.f};
     float4 sc = {0.f, 0.f, 0.f, 0.f}, sh = sc;
@@ -284,33 +312,55 @@ __global__ __launch_bounds__(256) void k_dwconv_tile(const float *__restrict__ g
         sc = *(const float4 *)(scale + i);
         sh = *(const float4 *)(shift + i);
     }
+    __syncthreads();
     float *os = out + (size_t)blockIdx.z * T * d + i;
+    const int r0 = RW * wave;
+    float4 o[RW];
 #pragma unroll
-    for (int u = 0; u < DW_R / 4; u++) {
-        const int rr = (tid >> 6) + 4 * u, t = t0 + rr;
-        if (t >= T) break;
-        const int j0 = t - pc < 0 ? pc - t : 0, j1 = t - pc + k > T ? T - t + pc : k;
-        float4 o = b0;
-        for (int j = j0; j < j1; j++) {
-            const float4 src = dws[(rr + j) * 64 + q], wv = taps[j * 64 + q];
-            o.x = fmaf(wv.x, src.x, o.x);
-            o.y = fmaf(wv.y, src.y, o.y);
-            o.z = fmaf(wv.z, src.z, o.z);
-            o.w = fmaf(wv.w, src.w, o.w);
+    for (int u = 0; u < RW; u++) o[u] = b0;
+    auto tap = [](float4 &acc, const float4 &wv, const float4 &src) {
+        acc.x = fmaf(wv.x, src.x, acc.x);
+        acc.y = fmaf(wv.y, src.y, acc.y);
+        acc.z = fmaf(wv.z, src.z, acc.z);
+        acc.w = fmaf(wv.w, src.w, acc.w);
+    };
+    if (K && t0 >= pc && t0 + R - 1 - pc + k - 1 < T && t0 + R <= T) {
+        float4 wv[K ? K : 1];
+#pragma unroll
+        for (int j = 0; j < K; j++) wv[j] = taps[j * 64 + q];
+#pragma unroll
+        for (int r = 0; r < RW + K - 1; r++) {
+            const float4 src = dws[(r0 + r) * 64 + q];
+#pragma unroll
+            for (int u = 0; u < RW; u++)
+                if (r - u >= 0 && r - u < K) tap(o[u], wv[r - u], src);
         }
+    } else {
+#pragma unroll
+        for (int u = 0; u < RW; u++) {
+            const int t = t0 + r0 + u;
+            const int j0 = t - pc < 0 ? pc - t : 0, j1 = t - pc + k > T ? T - t + pc : k;
+            if (t < T)
+                for (int j = j0; j < j1; j++) tap(o[u], taps[j * 64 + q], dws[(r0 + u + j) * 64 + q]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < RW; u++) {
+        const int t = t0 + r0 + u;
+        if (t >= T) break;
         if (scale) {
-            o.x = silu_e(fmaf(o.x, sc.x, sh.x));
-            o.y = silu_e(fmaf(o.y, sc.y, sh.y));
-            o.z = silu_e(fmaf(o.z, sc.z, sh.z));
-            o.w = silu_e(fmaf(o.w, sc.w, sh.w));
+            o[u].x = silu_e(fmaf(o[u].x, sc.x, sh.x));
+            o[u].y = silu_e(fmaf(o[u].y, sc.y, sh.y));
+            o[u].z = silu_e(fmaf(o[u].z, sc.z, sh.z));
+            o[u].w = silu_e(fmaf(o[u].w, sc.w, sh.w));
         }
         if constexpr (PREP) {
             // lanes 32 cl .. 32 cl + 31 hold chunk cl's 128 channels of row t
-            float a = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fmaxf(fabsf(o.z), fabsf(o.w)));
+            float a = fmaxf(fmaxf(fabsf(o[u].x), fabsf(o[u].y)), fmaxf(fabsf(o[u].z), fabsf(o[u].w)));
 #pragma unroll
             for (int off = 16; off > 0; off >>= 1) a = fmaxf(a, __shfl_xor(a, off, 64));
             const int shf = chunk_shift(a);
-            const float xs[4] = {ldexpf(o.x, shf), ldexpf(o.y, shf), ldexpf(o.z, shf), ldexpf(o.w, shf)};
+            const float xs[4] = {ldexpf(o[u].x, shf), ldexpf(o[u].y, shf), ldexpf(o[u].z, shf), ldexpf(o[u].w, shf)};
             _Float16 hv[4], lv[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -321,18 +371,18 @@ __global__ __launch_bounds__(256) void k_dwconv_tile(const float *__restrict__ g
             __builtin_memcpy(&pl[u], lv, 8);
             pf[u] = ldexpf(1.0f, -shf);
         } else {
-            *(float4 *)(os + (size_t)t * d) = o;
+            *(float4 *)(os + (size_t)t * d) = o[u];
         }
     }
     if constexpr (PREP) {
         __syncthreads();   // every wave is done with the input rows and the taps
         float4 *stage = dws;
-        float *fold = (float *)taps;
+        float *fold = (float *)(dws + R * 64);
         {
             const int l32 = q & 31, cl = q >> 5, hu = l32 >> 2, hh = (l32 >> 1) & 1;
 #pragma unroll
-            for (int u = 0; u < DW_R / 4; u++) {
-                const int rr = (tid >> 6) + 4 * u;
+            for (int u = 0; u < RW; u++) {
+                const int rr = r0 + u;
                 if (t0 + rr >= T) break;
                 uint8_t *o8 = (uint8_t *)(stage + (((rr * 2 + cl) * 8 + hu) * 2) * 2 + hh) + 8 * (l32 & 1);
                 *(uint2 *)o8 = ph[u];
@@ -343,9 +393,9 @@ __global__ __launch_bounds__(256) void k_dwconv_tile(const float *__restrict__ g
         __syncthreads();
         const int Kc = d / 128;
         const size_t mb = (size_t)blockIdx.z * T;
-        // 2048 slots; consecutive threads run along the 32 rows
-        for (int p = tid; p < DW_R * 64; p += 256) {
-            const int rr = p & 31, rest = p >> 5;
+        // 64 slots per row; consecutive threads run along the rows
+        for (int p = tid; p < R * 64; p += 256) {
+            const int rr = p % R, rest = p / R;
             const int cl = rest >> 5, hu = (rest >> 2) & 7, term = (rest >> 1) & 1, hh = rest & 1;
             const int t = t0 + rr;
             if (t < T) {
@@ -355,8 +405,8 @@ __global__ __launch_bounds__(256) void k_dwconv_tile(const float *__restrict__ g
                     stage[(((rr * 2 + cl) * 8 + hu) * 2 + term) * 2 + hh];
             }
         }
-        if (tid < 64) {
-            const int rr = tid & 31, cl = tid >> 5, t = t0 + rr;
+        if (tid < 2 * R) {
+            const int rr = tid % R, cl = tid / R, t = t0 + rr;
             if (t < T) {
                 const size_t m = mb + t;
                 xpf[((m >> 5) * Kc + 2 * blockIdx.y + cl) * 32 + (m & 31)] = fold[rr * 2 + cl];
@@ -597,8 +647,43 @@ hipError_t mh_launch_glu(const float *h, float *g, size_t rows, int d, hipStream
     return hipGetLastError();
 }
 
+constexpr int DW_R = 32;   // rows of a large tile
+
 bool mh_glu_dwconv_supported(int d, int k) {
     return d > 0 && d % 256 == 0 && k > 0 && sizeof(float4) * 64 * (size_t)(DW_R + 2 * k - 1) <= 64 * 1024;
+}
+
+// odd widths up to 15 with the width known at compile time, the rest (even
+// widths and 1) at run time; 8-row tiles when 32-row ones are fewer than the CUs
+template <bool PREP, int R>
+static hipError_t dwconv_tile(const float *g, const float *w, const float *bias, const float *scale, const float *shift,
+                              float *out, int T, int nseq, int d, int k, int pc, uint8_t *xp, float *xpf,
+                              hipStream_t st) {
+    // (>= the staged slots and folds: R rows and 2 R floats, which the taps' rows cover only for k > 1)
+    const size_t lds = sizeof(float4) * 64 * (size_t)(R + 2 * k - 1);
+    const dim3 grid((unsigned)((T + R - 1) / R), d / 256, nseq);
+    switch (k) {
+#define DWK(K)                                                                                                        \
+    case K:                                                                                                           \
+        hipLaunchKernelGGL((k_dwconv_tile<PREP, R, K>), grid, dim3(256), lds, st, g, w, bias, scale, shift, out, \
+                           T, d, k, pc, xp, xpf);                                                                     \
+        break;
+        DWK(3) DWK(5) DWK(7) DWK(9) DWK(11) DWK(13) DWK(15)
+#undef DWK
+    default:
+        hipLaunchKernelGGL((k_dwconv_tile<PREP, R, 0>), grid, dim3(256), lds, st, g, w, bias, scale, shift, out, T, d,
+                           k, pc, xp, xpf);
+    }
+    return hipGetLastError();
+}
+
+template <bool PREP>
+static hipError_t dwconv_rows(const float *g, const float *w, const float *bias, const float *scale, const float *shift,
+                              float *out, int T, int nseq, int d, int k, int pc, uint8_t *xp, float *xpf,
+                              hipStream_t st) {
+    if ((long)((T + DW_R - 1) / DW_R) * (d / 256) * nseq < 256)
+        return dwconv_tile<PREP, 8>(g, w, bias, scale, shift, out, T, nseq, d, k, pc, xp, xpf, st);
+    return dwconv_tile<PREP, DW_R>(g, w, bias, scale, shift, out, T, nseq, d, k, pc, xp, xpf, st);
 }
 
 hipError_t mh_launch_glu_dwconv(const float *h, const float *w, const float *bias, const float *scale,
@@ -607,16 +692,8 @@ hipError_t mh_launch_glu_dwconv(const float *h, const float *w, const float *bia
     if (T <= 0 || nseq <= 0) return hipSuccess;
     if (!mh_glu_dwconv_supported(d, k)) return hipErrorInvalidValue;
     const int pc = causal ? k - 1 : (k - 1) / 2;
-    const size_t lds = sizeof(float4) * 64 * (size_t)(DW_R + 2 * k - 1);   // >= the staged slots and folds
-    const dim3 grid((unsigned)((T + DW_R - 1) / DW_R), d / 256, nseq);
-    if (xp) {
-        hipLaunchKernelGGL((k_dwconv_tile<true, true>), grid, dim3(256), lds, st, h, w, bias, scale, shift, out, T, d,
-                           k, pc, xp, xpf);
-    } else {
-        hipLaunchKernelGGL((k_dwconv_tile<true, false>), grid, dim3(256), lds, st, h, w, bias, scale, shift, out, T, d,
-                           k, pc, nullptr, nullptr);
-    }
-    return hipGetLastError();
+    if (xp) return dwconv_rows<true>(h, w, bias, scale, shift, out, T, nseq, d, k, pc, xp, xpf, st);
+    return dwconv_rows<false>(h, w, bias, scale, shift, out, T, nseq, d, k, pc, nullptr, nullptr, st);
 }
 
 hipError_t mh_launch_dwconv(const float *g, const float *w, const float *bias, const float *scale,
@@ -625,12 +702,6 @@ hipError_t mh_launch_dwconv(const float *g, const float *w, const float *bias, c
     if (T <= 0 || nseq <= 0) return hipSuccess;
     if (d % 4 || k <= 0) return hipErrorInvalidValue;
     const int pc = causal ? k - 1 : (k - 1) / 2;
-    if (mh_glu_dwconv_supported(d, k)) {
-        const size_t lds = sizeof(float4) * 64 * (size_t)(DW_R + 2 * k - 1);
-        hipLaunchKernelGGL((k_dwconv_tile<false, false>), dim3((unsigned)((T + DW_R - 1) / DW_R), d / 256, nseq),
-                           dim3(256), lds, st, g, w, bias, scale, shift, out, T, d, k, pc, nullptr, nullptr);
-        return hipGetLastError();
-    }
     const size_t n = (size_t)nseq * T * (d / 4);
     hipLaunchKernelGGL(k_dwconv, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, w, bias, scale, shift, out,
                        T, nseq, d, k, pc);

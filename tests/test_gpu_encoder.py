@@ -267,3 +267,29 @@ def test_encoder_layer_in_other_numerics(gpu, mode):
     finally:
         gpu.set_numerics(M.EXACT)
         dev.close()
+
+
+@pytest.mark.parametrize("k", [1, 3, 8, 9, 15, 16])
+@pytest.mark.parametrize("T,nseq", [(7, 2), (8, 1), (33, 1), (97, 1), (66, 96)],
+                         ids=["T7x2", "T8", "T33", "T97", "T66x96"])
+def test_conv_tiles_match_oracle(gpu, orc, k, T, nseq):
+    """The tiled depthwise conv at both tile heights, its compiled and run-time
+    widths, tiles at a segment's ends and tiles within one; the tests' bar."""
+    import torch
+    d, H, f = 256, 2, 256
+    say("conv tiles", k, T, nseq)
+    p = make_params(17, d, f, k, False, True)
+    dev = M.DeviceEncoderLayer(gpu, p, M.Q8_0)
+    try:
+        x = np.random.default_rng(18).standard_normal((nseq * T, d)).astype(np.float32)
+        pe = E.pos_emb(T, d).astype(np.float32)
+        xd, ped = torch.from_numpy(x).cuda(), torch.from_numpy(pe).cuda()
+        dev.run(xd.data_ptr(), T, nseq, ped.data_ptr(), d, H, k, 0)
+        torch.cuda.synchronize()
+        keep = np.r_[0:T, (nseq - 1) * T:nseq * T] if nseq > 2 else np.arange(nseq * T)
+        segs = 2 if nseq > 2 else nseq
+        ref = E.encoder_layer(x[keep], oracle_params(orc, dev, p, M.Q8_0), T, segs, pe, H, k, 0, -1, 0)
+        err = np.abs(xd.cpu().numpy()[keep] - ref)
+        assert (err <= 2e-6 * (1 + np.abs(ref))).all()
+    finally:
+        dev.close()
