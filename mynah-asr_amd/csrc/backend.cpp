@@ -919,7 +919,7 @@ int encoder_layer_dev(Ctx *c, const mynah_asr_hip_enc_layer *L, float *x, int T,
         if (gemm_dev(c, L->relk_w, pe, rk, P, 0, st)) return -1;
     }
     {
-        const size_t wb = mh_attn_ws_bytes(T, d, H, nseq, left);
+        const size_t wb = mh_attn_ws_bytes(T, d, H, nseq, left, right);
         void *ws = wb ? c->attw.get(wb) : nullptr;
         if (wb && !ws) return fail("device buffer allocation failed");
         // the context as the output projection's prepared input (tagged ctx),
@@ -927,7 +927,7 @@ int encoder_layer_dev(Ctx *c, const mynah_asr_hip_enc_layer *L, float *x, int T,
         uint8_t *xp = nullptr;
         float *xpf = nullptr;
         c->pa.src = nullptr;
-        if (mh_attn_preps_out(d, H, left) && ln_preps(&L->o_w, 1, M, d)) {
+        if (mh_attn_preps_out(d, H) && ln_preps(&L->o_w, 1, M, d)) {
             size_t bs[3];
             prep_sizes(0, mh_mpad(M), d, bs);
             xp = (uint8_t *)c->pa.xp.get(bs[0]);
@@ -1236,7 +1236,7 @@ int mynah_asr_hip_relpos_attention_dev(const float *q, const float *k, const flo
     if (ctx == q || ctx == k || ctx == v) return fail("ctx may not alias q, k or v");
     if ((size_t)2 * T * d >= 0x7fffffffu) return fail("attention: 2 T d must stay below 2^31");
     if (T == 0 || nseq == 0) return 0;
-    const size_t wb = mh_attn_ws_bytes(T, d, H, nseq, left);
+    const size_t wb = mh_attn_ws_bytes(T, d, H, nseq, left, right);
     void *ws = wb ? c->attw.get(wb) : nullptr;
     if (wb && !ws) return fail("device buffer allocation failed");
     hipError_t e = mh_launch_relpos_attn(q, k, v, rk, bias_u, bias_v, ctx, T, d, H, left, right, nseq, ws,

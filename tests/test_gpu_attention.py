@@ -159,3 +159,15 @@ def test_relpos_attention_rejects_bad_arguments(gpu):
         M.relpos_attention_dev(gpu, p, p, p, p, p, p, x[1:].data_ptr(), 1, 128, 2, 4, -1)
     with pytest.raises(RuntimeError, match="alias"):
         M.relpos_attention_dev(gpu, p, p, p, p, p, p, p, 1, 128, 2)
+
+
+@pytest.mark.parametrize("T", [1, 31, 32, 33, 64, 65, 129, 257])
+@pytest.mark.parametrize("d,H", [(128, 2), (256, 2)], ids=["dk64", "dk128"])
+@pytest.mark.parametrize("left,right", [(-1, 0), (0, 0), (3, 1), (64, 31), (70, 13), (100000, 0)])
+def test_relpos_attention_tile_edges(gpu, T, d, H, left, right):
+    """Lengths around the 32-row tiles; windows narrower than a tile, as wide as
+    one, and wider than the segment (fewer key tiles than waves, one wave's
+    tiles, waves with none)."""
+    say("attention tile edges", T, d, H, left, right)
+    arrs = make(1000 + T, T, d, 2)
+    check(run_gpu(gpu, arrs, T, d, H, left, right, 2), arrs, H, left, right)
