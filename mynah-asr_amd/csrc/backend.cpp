@@ -277,22 +277,29 @@ bool fits(const PrepBuf &P, const mynah_asr_hip_weight *W, int T) {
 bool prep_fits(const Ctx *c, const mynah_asr_hip_weight *W, int T) { return fits(c->pa, W, T); }
 
 // the product on a prepared input
-// act: 0 none, 1 SiLU; 2 and 3 (internal, the EXACT GEMM path only) add the
-// product, or half of it, into dy (the encoder layer's residual adds)
-int run_from(Ctx *c, const PrepBuf &P, const mynah_asr_hip_weight *W, float *dy, int T, int act, hipStream_t st) {
+// act: 0 none, 1 SiLU, both on the product + bias (or null); 2 and 3 (internal,
+// the EXACT GEMM path only) add that, or half of it, into dy (the encoder
+// layer's residual adds)
+int run_from(Ctx *c, const PrepBuf &P, const mynah_asr_hip_weight *W, float *dy, int T, int act, const float *bias,
+             hipStream_t st) {
     hipError_t e;
     if (act >= 2 && P.i8 != 0) return fail("internal: a residual epilogue outside the EXACT GEMM path");
     if (P.i8 == MH_I8_QMAT) {
-        e = mh_launch_gemm_i8(W->qtype, W->dw, (const uint8_t *)P.xp.p, (const float *)P.xs16.p, dy, T, act, st);
+        // (its epilogue has no bias)
+        const size_t n = W->dw.n;
+        e = mh_launch_gemm_i8(W->qtype, W->dw, (const uint8_t *)P.xp.p, (const float *)P.xs16.p, dy, T, bias ? 0 : act,
+                              st);
+        if (e == hipSuccess && bias) e = mh_launch_bias_rows(dy, bias, T, (int)n, st);
+        if (e == hipSuccess && bias && act == 1) e = mh_launch_silu(dy, T * n, st);
     } else {
         e = mh_launch_gemm(W->qtype, W->dw, (const uint8_t *)P.xp.p, (const float *)P.xs16.p,
-                           (const float *)P.xpf.p, dy, T, act, st, P.i8 != 0);
+                           (const float *)P.xpf.p, dy, T, act, bias, st, P.i8 != 0);
     }
     if (e != hipSuccess) return fail("gemm launch failed", hipGetErrorString(e));
     return 0;
 }
-int run_prepped(Ctx *c, const mynah_asr_hip_weight *W, float *dy, int T, int act, hipStream_t st) {
-    return run_from(c, c->pa, W, dy, T, act, st);
+int run_prepped(Ctx *c, const mynah_asr_hip_weight *W, float *dy, int T, int act, const float *bias, hipStream_t st) {
+    return run_from(c, c->pa, W, dy, T, act, bias, st);
 }
 
 // the calling thread's split-K GEMV workspace for W (null: the one-launch GEMV)
@@ -301,17 +308,17 @@ float *gemv_ws(Ctx *c, const mynah_asr_hip_weight *W) {
     return n ? (float *)c->gs.get(n * sizeof(float)) : nullptr;
 }
 
-int gemm_dev(Ctx *c, const mynah_asr_hip_weight *W, const float *dx, float *dy, int T, int act,
-             hipStream_t st) {
+int gemm_dev(Ctx *c, const mynah_asr_hip_weight *W, const float *dx, float *dy, int T, int act, hipStream_t st,
+             const float *bias = nullptr) {
     if (num_now() == MYNAH_ASR_HIP_EXACT && mh_use_gemv(W->dw, T)) {
         if (act >= 2) return fail("internal: a residual epilogue outside the EXACT GEMM path");
         const int vec = (W->dw.k % 8 == 0) && (((uintptr_t)dx & 15) == 0);
-        hipError_t e = mh_launch_gemv(W->qtype, W->dw, dx, T, vec, dy, act, gemv_ws(c, W), st);
+        hipError_t e = mh_launch_gemv_epi(W->qtype, W->dw, dx, T, vec, dy, GEpi{act, bias, nullptr}, gemv_ws(c, W), st);
         if (e != hipSuccess) return fail("gemv launch failed", hipGetErrorString(e));
         return 0;
     }
     if (prep_for(c, W, dx, T, st)) return -1;
-    return run_prepped(c, W, dy, T, act, st);
+    return run_prepped(c, W, dy, T, act, bias, st);
 }
 
 // out = SiLU(x . W1^T) . W2^T on device buffers (dx may alias dy). In EXACT
@@ -319,7 +326,7 @@ int gemm_dev(Ctx *c, const mynah_asr_hip_weight *W, const float *dx, float *dy, 
 // first product prepares the intermediate for the second in its epilogue
 // (no f32 intermediate, no preparation pass); otherwise two products.
 int ffn_dev(Ctx *c, const mynah_asr_hip_weight *W1, const mynah_asr_hip_weight *W2, const float *dx, float *dy,
-            int T, hipStream_t st, int act2 = 0) {
+            int T, hipStream_t st, int act2 = 0, const float *b1 = nullptr, const float *b2 = nullptr) {
     const int n1 = eff_num(W1->qtype, W1->dw.k, T), n2 = eff_num(W2->qtype, W2->dw.k, T);
     if (n1 != n2) {
         // (QMAT numerics: each product in its own mode, as qmat_ffn's two qmat_mul calls)
@@ -327,10 +334,10 @@ int ffn_dev(Ctx *c, const mynah_asr_hip_weight *W1, const mynah_asr_hip_weight *
         if (!dh) return fail("device buffer allocation failed");
         {
             NumScope s1(n1);
-            if (gemm_dev(c, W1, dx, dh, T, 1, st)) return -1;
+            if (gemm_dev(c, W1, dx, dh, T, 1, st, b1)) return -1;
         }
         NumScope s2(n2);
-        return gemm_dev(c, W2, dh, dy, T, act2, st);
+        return gemm_dev(c, W2, dh, dy, T, act2, st, b2);
     }
     NumScope sc(n1);
     const bool fuse = num_now() == MYNAH_ASR_HIP_EXACT && !mh_use_gemv(W1->dw, T) &&
@@ -345,30 +352,31 @@ int ffn_dev(Ctx *c, const mynah_asr_hip_weight *W1, const mynah_asr_hip_weight *
         float *xpf = (float *)P.xpf.get((size_t)Mpad * (Kp / 128) * sizeof(float));
         if (!xp || !xs16 || !xpf) return fail("workspace allocation failed");
         hipError_t e = mh_launch_gemm_prep_out(W1->qtype, W1->dw, (const uint8_t *)c->pa.xp.p,
-                                               (const float *)c->pa.xs16.p, (const float *)c->pa.xpf.p, T, xp, xs16,
-                                               xpf, Kp / 128, xsum, st);
+                                               (const float *)c->pa.xs16.p, (const float *)c->pa.xpf.p, T, b1, xp,
+                                               xs16, xpf, Kp / 128, xsum, st);
         if (e != hipSuccess) return fail("gemm launch failed", hipGetErrorString(e));
         P.T = T;
         P.Kp = Kp;
         P.xsum = xsum;
         P.i8 = 0;
-        return run_from(c, P, W2, dy, T, act2, st);
+        return run_from(c, P, W2, dy, T, act2, b2, st);
     }
     float *dh = (float *)c->h.get((size_t)T * W1->dw.n * sizeof(float));
     if (!dh) return fail("device buffer allocation failed");
-    if (gemm_dev(c, W1, dx, dh, T, 1, st)) return -1;
-    return gemm_dev(c, W2, dh, dy, T, act2, st);
+    if (gemm_dev(c, W1, dx, dh, T, 1, st, b1)) return -1;
+    return gemm_dev(c, W2, dh, dy, T, act2, st, b2);
 }
 
 // three products of one input: prepared once whenever it fits them all
 int qkv_dev(Ctx *c, const mynah_asr_hip_weight *const W[3], const float *dx, float *const dy[3], int T,
-            hipStream_t st) {
+            hipStream_t st, const float *const *bias = nullptr) {
+    auto b = [&](int i) { return bias ? bias[i] : nullptr; };
     const int nq = eff_num(W[0]->qtype, W[0]->dw.k, T);
     if (eff_num(W[1]->qtype, W[1]->dw.k, T) != nq || eff_num(W[2]->qtype, W[2]->dw.k, T) != nq) {
         // (QMAT numerics: each product in its own mode, as qmat_qkv's three qmat_mul calls)
         for (int i = 0; i < 3; i++) {
             NumScope si(eff_num(W[i]->qtype, W[i]->dw.k, T));
-            if (gemm_dev(c, W[i], dx, dy[i], T, 0, st)) return -1;
+            if (gemm_dev(c, W[i], dx, dy[i], T, 0, st, b(i))) return -1;
         }
         return 0;
     }
@@ -382,13 +390,14 @@ int qkv_dev(Ctx *c, const mynah_asr_hip_weight *const W[3], const float *dx, flo
         if (prep_for(c, W[0], dx, T, st)) return -1;
         if (c->pa.i8 == MH_I8_QMAT) {
             for (int i = 0; i < 3; i++)
-                if (run_prepped(c, W[i], dy[i], T, 0, st)) return -1;
+                if (run_prepped(c, W[i], dy[i], T, 0, b(i), st)) return -1;
             return 0;
         }
         GemmJobs J{};
         for (int i = 0; i < 3; i++) {
             J.W[i] = W[i]->dw;
             J.y[i] = dy[i];
+            J.bias[i] = b(i);
         }
         J.n = 3;
         const PrepBuf &P = c->pa;
@@ -400,13 +409,13 @@ int qkv_dev(Ctx *c, const mynah_asr_hip_weight *const W[3], const float *dx, flo
     bool prepared = false;
     for (int i = 0; i < 3; i++) {
         if (num_now() == MYNAH_ASR_HIP_EXACT && mh_use_gemv(W[i]->dw, T)) {
-            if (gemm_dev(c, W[i], dx, dy[i], T, 0, st)) return -1;
+            if (gemm_dev(c, W[i], dx, dy[i], T, 0, st, b(i))) return -1;
             continue;
         }
         if (!prepared || !prep_fits(c, W[i], T))
             if (prep_for(c, W[i], dx, T, st)) return -1;
         prepared = true;
-        if (run_prepped(c, W[i], dy[i], T, 0, st)) return -1;
+        if (run_prepped(c, W[i], dy[i], T, 0, b(i), st)) return -1;
     }
     return 0;
 }
@@ -616,15 +625,13 @@ int aed_run(Ctx *c, const mynah_asr_hip_aed *a, const float *enc, int T, const i
 
     // encoder projection and the per-layer cross K/V (decoder_aed.c:150-175)
     if (a->proj) {
-        if (gemm_dev(c, a->proj, enc, b.encp, T, 0, st)) return -1;
-        if (a->proj_b) AED_TRY(mh_launch_bias_rows(b.encp, a->proj_b, T, d, st));
+        if (gemm_dev(c, a->proj, enc, b.encp, T, 0, st, a->proj_b)) return -1;
     }
     for (int li = 0; li < nl; li++) {
         const mynah_asr_hip_aed_layer *L = &a->layers[li];
         float *CK = b.ckv + 2 * (size_t)li * td, *CV = CK + td;
-        if (gemm_dev(c, L->ck, b.encp, CK, T, 0, st) || gemm_dev(c, L->cv, b.encp, CV, T, 0, st)) return -1;
-        AED_TRY(mh_launch_bias_rows(CK, L->ck_b, T, d, st));
-        AED_TRY(mh_launch_bias_rows(CV, L->cv_b, T, d, st));
+        if (gemm_dev(c, L->ck, b.encp, CK, T, 0, st, L->ck_b) || gemm_dev(c, L->cv, b.encp, CV, T, 0, st, L->cv_b))
+            return -1;
     }
     if (hipMemcpyAsync(b.prompt, prompt, n_prompt * sizeof(int), hipMemcpyHostToDevice, st) != hipSuccess)
         return fail("H2D copy failed");
@@ -755,7 +762,7 @@ int gemm_noalloc(const mynah_asr_hip_weight *W, const float *dx, float *dy, int 
     e = launch_prep(kind, W, dx, T, xp, xs16, xpf, st);
     if (e == hipSuccess) {
         if (kind == MH_I8_QMAT) e = mh_launch_gemm_i8(W->qtype, W->dw, xp, xs16, dy, T, act, st);
-        else e = mh_launch_gemm(W->qtype, W->dw, xp, xs16, xpf, dy, T, act, st, kind != 0);
+        else e = mh_launch_gemm(W->qtype, W->dw, xp, xs16, xpf, dy, T, act, nullptr, st, kind != 0);
     }
     return e == hipSuccess ? 0 : fail("launch failed", hipGetErrorString(e));
 }
@@ -789,32 +796,6 @@ int enc_check(const mynah_asr_hip_enc_layer *L, int T, int nseq, int d, int H, i
     return 0;
 }
 
-int bias_add(float *y, const float *b, size_t rows, int n, hipStream_t st) {
-    if (!b) return 0;
-    hipError_t e = mh_launch_bias_rows(y, b, rows, n, st);
-    return e == hipSuccess ? 0 : fail("bias launch failed", hipGetErrorString(e));
-}
-
-// half_ffn (encoder.c:464-483) on xn: the fused FFN when both biases are
-// absent, else product, bias, SiLU, product, bias
-int enc_half_ffn(Ctx *c, const mynah_asr_hip_weight *w1, const mynah_asr_hip_weight *w2, const float *b1,
-                 const float *b2, const float *xn, float *out, float *h, int M, hipStream_t st, int act2 = 0) {
-    if (!b1 && !b2) return ffn_dev(c, w1, w2, xn, out, M, st, act2);
-    const int f = w1->dw.n;
-    {
-        NumScope s1(eff_num(w1->qtype, w1->dw.k, M));
-        if (gemm_dev(c, w1, xn, h, M, 0, st)) return -1;
-    }
-    if (bias_add(h, b1, M, f, st)) return -1;
-    hipError_t e = mh_launch_silu(h, (size_t)M * f, st);
-    if (e != hipSuccess) return fail("silu launch failed", hipGetErrorString(e));
-    {
-        NumScope s2(eff_num(w2->qtype, w2->dw.k, M));
-        if (gemm_dev(c, w2, h, out, M, 0, st)) return -1;
-    }
-    return bias_add(out, b2, M, w2->dw.n, st);
-}
-
 // Whether the products W[0..n) of one layer-norm output xn all read it as
 // the EXACT GEMM path's prepared input (no GEMV, no row sums, K = Kp = d):
 // then the layer norm writes that input directly.
@@ -839,7 +820,7 @@ bool ln_preps(const mynah_asr_hip_weight *const *W, int n, int M, int d) {
 // (c->pa, tagged xn; xn itself is then not written) when ln_preps allows,
 // else as f32 rows
 int enc_add_ln(Ctx *c, float *x, const float *res, float alpha, const float *w, const float *b, float *xn, int M,
-               int d, const mynah_asr_hip_weight *const *W, int n, hipStream_t st) {
+               int d, const mynah_asr_hip_weight *const *W, int n, hipStream_t st, bool silu = false) {
     hipError_t e;
     c->pa.src = nullptr;
     if (ln_preps(W, n, M, d)) {
@@ -850,7 +831,7 @@ int enc_add_ln(Ctx *c, float *x, const float *res, float alpha, const float *w, 
         float *xs16 = (float *)c->pa.xs16.get(bs[1]);
         float *xpf = (float *)c->pa.xpf.get(bs[2]);
         if (!xp || !xs16 || !xpf) return fail("workspace allocation failed");
-        e = mh_launch_add_ln_prep(x, res, alpha, w, b, M, d, xp, xpf, st);
+        e = mh_launch_add_ln_prep(x, res, alpha, w, b, M, d, silu, xp, xpf, st);
         if (e != hipSuccess) return fail("encoder layer launch failed", hipGetErrorString(e));
         c->pa.T = M;
         c->pa.Kp = d;
@@ -859,7 +840,7 @@ int enc_add_ln(Ctx *c, float *x, const float *res, float alpha, const float *w, 
         c->pa.src = xn;
         return 0;
     }
-    e = mh_launch_add_ln(x, res, alpha, w, b, xn, M, d, st);
+    e = mh_launch_add_ln(x, res, alpha, w, b, xn, M, d, silu, st);
     return e == hipSuccess ? 0 : fail("encoder layer launch failed", hipGetErrorString(e));
 }
 
@@ -871,16 +852,13 @@ int encoder_layer_dev(Ctx *c, const mynah_asr_hip_enc_layer *L, float *x, int T,
         PrepBuf &pa;
         ~TagClear() { pa.src = nullptr; }
     } tag_clear{c->pa};
-    const int f = L->ff1_w1->dw.n > L->ff2_w1->dw.n ? L->ff1_w1->dw.n : L->ff2_w1->dw.n;
-    const bool biased_ffn = L->ff1_b1 || L->ff1_b2 || L->ff2_b1 || L->ff2_b2;
     const size_t md = (size_t)M * d;
-    // xn, tmp, q, k, v, ctx [M, d]; h [M, 2d] (pw1, GLU); rk [P, d]; the FFN
-    // intermediate [M, f] only with FFN biases
-    const size_t need = 6 * md + 2 * md + (size_t)P * d + (biased_ffn ? (size_t)M * f : 0);
+    // xn, tmp, q, k, v, ctx [M, d]; h [M, 2d] (pw1, GLU); rk [P, d]
+    const size_t need = 6 * md + 2 * md + (size_t)P * d;
     float *base = (float *)c->enc.get(need * sizeof(float));
     if (!base) return fail("device buffer allocation failed");
     float *xn = base, *tmp = xn + md, *q = tmp + md, *k = q + md, *v = k + md, *ctx = v + md, *h = ctx + md,
-          *rk = h + 2 * md, *hf = rk + (size_t)P * d;
+          *rk = h + 2 * md;
     hipError_t e;
 #define ENC_TRY(expr)                                                                   \
     do {                                                                                \
@@ -891,26 +869,25 @@ int encoder_layer_dev(Ctx *c, const mynah_asr_hip_enc_layer *L, float *x, int T,
     // (each layer norm whose output only feeds products tags the prepared
     // input with xn; the tag is cleared once those products have run)
     //
-    // A product with no bias on the EXACT GEMM path adds its output into x
+    // A product on the EXACT GEMM path adds its output (and bias) into x
     // itself (x += tmp or x += tmp / 2, the same operations as the layer
     // norm's residual add), and the next layer norm reads x alone.
-    auto res_ok = [&](const mynah_asr_hip_weight *W, bool biased) {
-        return !biased && enc_fused() && eff_num(W->qtype, W->dw.k, M) == MYNAH_ASR_HIP_EXACT &&
+    auto res_ok = [&](const mynah_asr_hip_weight *W) {
+        return enc_fused() && eff_num(W->qtype, W->dw.k, M) == MYNAH_ASR_HIP_EXACT &&
                !mh_use_gemv(W->dw, M);
     };
     if (enc_add_ln(c, x, nullptr, 0.0f, L->ln_ff1_w, L->ln_ff1_b, xn, M, d, &L->ff1_w1, 1, st)) return -1;
-    const bool r1 = res_ok(L->ff1_w2, L->ff1_b1 || L->ff1_b2);
-    if (enc_half_ffn(c, L->ff1_w1, L->ff1_w2, L->ff1_b1, L->ff1_b2, xn, r1 ? x : tmp, hf, M, st, r1 ? 3 : 0))
-        return -1;
+    const bool r1 = res_ok(L->ff1_w2);
+    if (ffn_dev(c, L->ff1_w1, L->ff1_w2, xn, r1 ? x : tmp, M, st, r1 ? 3 : 0, L->ff1_b1, L->ff1_b2)) return -1;
     c->pa.src = nullptr;
     // x += 0.5 tmp; MHSA on LN(x) (:495-502)
     const mynah_asr_hip_weight *W3[3] = {L->q_w, L->k_w, L->v_w};
     if (enc_add_ln(c, x, r1 ? nullptr : tmp, r1 ? 0.0f : 0.5f, L->ln_att_w, L->ln_att_b, xn, M, d, W3, 3, st))
         return -1;
     float *const y3[3] = {q, k, v};
-    if (qkv_dev(c, W3, xn, y3, M, st)) return -1;
+    const float *const b3[3] = {L->q_b, L->k_b, L->v_b};
+    if (qkv_dev(c, W3, xn, y3, M, st, b3)) return -1;
     c->pa.src = nullptr;
-    if (bias_add(q, L->q_b, M, d, st) || bias_add(k, L->k_b, M, d, st) || bias_add(v, L->v_b, M, d, st)) return -1;
     {
         // rk = pe . relk^T (:336): the segments share T, so one product serves
         // them all; in f32 arithmetic whatever the mode (relk_w stays f32 in
@@ -945,23 +922,21 @@ int encoder_layer_dev(Ctx *c, const mynah_asr_hip_enc_layer *L, float *x, int T,
             c->pa.src = ctx;
         }
     }
-    const bool r2 = res_ok(L->o_w, L->o_b != nullptr);
+    const bool r2 = res_ok(L->o_w);
     {
         NumScope so(eff_num(L->o_w->qtype, d, M));
-        if (gemm_dev(c, L->o_w, ctx, r2 ? x : tmp, M, r2 ? 2 : 0, st)) return -1;
+        if (gemm_dev(c, L->o_w, ctx, r2 ? x : tmp, M, r2 ? 2 : 0, st, L->o_b)) return -1;
     }
     c->pa.src = nullptr;
-    if (bias_add(tmp, L->o_b, M, d, st)) return -1;
     // x += tmp; conv module on LN(x) (:503-507, 413-462)
     if (enc_add_ln(c, x, r2 ? nullptr : tmp, r2 ? 0.0f : 1.0f, L->ln_conv_w, L->ln_conv_b, xn, M, d, &L->pw1_w, 1,
                    st))
         return -1;
     {
         NumScope s1(eff_num(L->pw1_w->qtype, d, M));
-        if (gemm_dev(c, L->pw1_w, xn, h, M, 0, st)) return -1;
+        if (gemm_dev(c, L->pw1_w, xn, h, M, 0, st, L->pw1_b)) return -1;
     }
     c->pa.src = nullptr;
-    if (bias_add(h, L->pw1_b, M, 2 * d, st)) return -1;
     // the GLU (g = q, free now) folded into the depthwise conv where it can be
     const bool glu_dw = mh_glu_dwconv_supported(d, conv_k);
     if (!glu_dw) ENC_TRY(mh_launch_glu(h, q, M, d, st));
@@ -993,26 +968,23 @@ int encoder_layer_dev(Ctx *c, const mynah_asr_hip_enc_layer *L, float *x, int T,
         }
     } else {
         ENC_TRY(dwconv(nullptr, nullptr, v, nullptr, nullptr));
-        ENC_TRY(mh_launch_add_ln(v, nullptr, 0.0f, L->cnorm_w, L->cnorm_b, k, M, d, st));
-        ENC_TRY(mh_launch_silu(k, md, st));
+        if (enc_add_ln(c, v, nullptr, 0.0f, L->cnorm_w, L->cnorm_b, k, M, d, &L->pw2_w, 1, st, true)) return -1;
     }
-    const bool r3 = res_ok(L->pw2_w, L->pw2_b != nullptr);
+    const bool r3 = res_ok(L->pw2_w);
     {
         NumScope s2(eff_num(L->pw2_w->qtype, d, M));
-        if (gemm_dev(c, L->pw2_w, k, r3 ? x : tmp, M, r3 ? 2 : 0, st)) return -1;
+        if (gemm_dev(c, L->pw2_w, k, r3 ? x : tmp, M, r3 ? 2 : 0, st, L->pw2_b)) return -1;
     }
     c->pa.src = nullptr;
-    if (bias_add(tmp, L->pw2_b, M, d, st)) return -1;
     // x += tmp; 1/2 FFN2 on LN(x) (:508-511)
     if (enc_add_ln(c, x, r3 ? nullptr : tmp, r3 ? 0.0f : 1.0f, L->ln_ff2_w, L->ln_ff2_b, xn, M, d, &L->ff2_w1, 1,
                    st))
         return -1;
-    const bool r4 = res_ok(L->ff2_w2, L->ff2_b1 || L->ff2_b2);
-    if (enc_half_ffn(c, L->ff2_w1, L->ff2_w2, L->ff2_b1, L->ff2_b2, xn, r4 ? x : tmp, hf, M, st, r4 ? 3 : 0))
-        return -1;
+    const bool r4 = res_ok(L->ff2_w2);
+    if (ffn_dev(c, L->ff2_w1, L->ff2_w2, xn, r4 ? x : tmp, M, st, r4 ? 3 : 0, L->ff2_b1, L->ff2_b2)) return -1;
     c->pa.src = nullptr;
     // x += 0.5 tmp; x = LN_out(x) (:511-515)
-    ENC_TRY(mh_launch_add_ln(x, r4 ? nullptr : tmp, r4 ? 0.0f : 0.5f, L->ln_out_w, L->ln_out_b, x, M, d, st));
+    ENC_TRY(mh_launch_add_ln(x, r4 ? nullptr : tmp, r4 ? 0.0f : 0.5f, L->ln_out_w, L->ln_out_b, x, M, d, false, st));
 #undef ENC_TRY
     return 0;
 }
@@ -1170,7 +1142,7 @@ int mynah_asr_hip_qgemm_prepped_dev(const mynah_asr_hip_weight *w, float *dy, in
     if (check_numerics_supported(w->qtype, w->dw.k, T)) return -1;
     NumScope sc(eff_num(w->qtype, w->dw.k, T));
     if (!prep_fits(c, w, T)) return fail("the prepared input does not fit this weight");
-    return run_prepped(c, w, dy, T, act, pick_stream(stream));
+    return run_prepped(c, w, dy, T, act, nullptr, pick_stream(stream));
 }
 
 int mynah_asr_hip_qffn_dev(const mynah_asr_hip_weight *w1, const mynah_asr_hip_weight *w2, const float *dx,
@@ -1412,7 +1384,7 @@ int mynah_asr_hip_qqkv(const mynah_asr_hip_wdesc *wq, const mynah_asr_hip_wdesc 
             if (!prepared || !prep_fits(c, W[i], T))
                 if (prep_for(c, W[i], dx, T, c->st)) return -1;
             prepared = true;
-            if (run_prepped(c, W[i], dy, T, 0, c->st)) return -1;
+            if (run_prepped(c, W[i], dy, T, 0, nullptr, c->st)) return -1;
         }
         if (d2h_sync(c, outs[i], dy, (size_t)T * ws[i]->n)) return -1;
     }

@@ -30,8 +30,7 @@
 #include <math.h>
 #include <stdint.h>
 
-#include "fmt.h"
-#include "launch.h"
+#include "product.h"
 
 namespace {
 
@@ -51,7 +50,7 @@ __device__ __forceinline__ float sigmoid_f(float x) {
 // * inv) * w + b in f32.
 template <int V4>
 __device__ __forceinline__ void add_ln_row(float *xr, const float *__restrict__ rr, float alpha,
-                                           const float *__restrict__ w, const float *__restrict__ b, int lane,
+                                           const float *__restrict__ w, const float *__restrict__ b, int silu, int lane,
                                            float4 (&v)[V4]) {
     constexpr int d = 256 * V4;
     float4 wv[V4], bv[V4];
@@ -94,6 +93,7 @@ __device__ __forceinline__ void add_ln_row(float *xr, const float *__restrict__ 
         v[u].y = ((v[u].y - muf) * inv) * wv[u].y + bv[u].y;
         v[u].z = ((v[u].z - muf) * inv) * wv[u].z + bv[u].z;
         v[u].w = ((v[u].w - muf) * inv) * wv[u].w + bv[u].w;
+        if (silu) v[u] = float4{silu_f(v[u].x), silu_f(v[u].y), silu_f(v[u].z), silu_f(v[u].w)};
     }
 }
 
@@ -101,12 +101,12 @@ __device__ __forceinline__ void add_ln_row(float *xr, const float *__restrict__ 
 template <int V4>
 __global__ __launch_bounds__(256) void k_add_ln(float *x, const float *__restrict__ res, float alpha,
                                                 const float *__restrict__ w, const float *__restrict__ b,
-                                                float *out, int rows) {
+                                                float *out, int rows, int silu) {
     constexpr int d = 256 * V4;
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (r >= rows) return;
     float4 v[V4];
-    add_ln_row<V4>(x + (size_t)r * d, res ? res + (size_t)r * d : nullptr, alpha, w, b, lane, v);
+    add_ln_row<V4>(x + (size_t)r * d, res ? res + (size_t)r * d : nullptr, alpha, w, b, silu, lane, v);
     float *orow = out + (size_t)r * d;
 #pragma unroll
     for (int u = 0; u < V4; u++) *(float4 *)(orow + 4 * lane + 256 * u) = v[u];
@@ -130,14 +130,15 @@ __global__ __launch_bounds__(256) void k_add_ln(float *x, const float *__restric
 template <int V4>
 __global__ __launch_bounds__(512) void k_add_ln_prep(float *x, const float *__restrict__ res, float alpha,
                                                      const float *__restrict__ w, const float *__restrict__ b,
-                                                     int rows, uint8_t *__restrict__ xp, float *__restrict__ xpf) {
+                                                     int rows, int silu, uint8_t *__restrict__ xp,
+                                                     float *__restrict__ xpf) {
     constexpr int d = 256 * V4, Kc = d / 128, NL = Kc * 32;   // lines of the workgroup
     __shared__ uint4 stage[NL * 8];
     const int wave = threadIdx.x >> 6, m = blockIdx.x * 8 + wave, lane = threadIdx.x & 63;
     const int G = m >> 5, r = m & 31, l32 = lane & 31;
     float4 v[V4];
     if (m < rows) {
-        add_ln_row<V4>(x + (size_t)m * d, res ? res + (size_t)m * d : nullptr, alpha, w, b, lane, v);
+        add_ln_row<V4>(x + (size_t)m * d, res ? res + (size_t)m * d : nullptr, alpha, w, b, silu, lane, v);
     } else {
 #pragma unroll
         for (int u = 0; u < V4; u++) v[u] = float4{0.f, 0.f, 0.f, 0.f};
@@ -601,21 +602,21 @@ bool mh_enc_d_supported(int d) {
 }
 
 hipError_t mh_launch_add_ln(float *x, const float *res, float alpha, const float *w, const float *b, float *out,
-                            int rows, int d, hipStream_t st) {
+                            int rows, int d, bool silu, hipStream_t st) {
     if (rows <= 0) return hipSuccess;
     if (!mh_enc_d_supported(d)) return hipErrorInvalidValue;
     const dim3 grid((rows + 3) / 4), blk(256);
     switch (d / 256) {
-    case 1: hipLaunchKernelGGL(k_add_ln<1>, grid, blk, 0, st, x, res, alpha, w, b, out, rows); break;
-    case 2: hipLaunchKernelGGL(k_add_ln<2>, grid, blk, 0, st, x, res, alpha, w, b, out, rows); break;
-    case 3: hipLaunchKernelGGL(k_add_ln<3>, grid, blk, 0, st, x, res, alpha, w, b, out, rows); break;
-    case 4: hipLaunchKernelGGL(k_add_ln<4>, grid, blk, 0, st, x, res, alpha, w, b, out, rows); break;
-    case 5: hipLaunchKernelGGL(k_add_ln<5>, grid, blk, 0, st, x, res, alpha, w, b, out, rows); break;
-    case 6: hipLaunchKernelGGL(k_add_ln<6>, grid, blk, 0, st, x, res, alpha, w, b, out, rows); break;
-    case 7: hipLaunchKernelGGL(k_add_ln<7>, grid, blk, 0, st, x, res, alpha, w, b, out, rows); break;
-    case 8: hipLaunchKernelGGL(k_add_ln<8>, grid, blk, 0, st, x, res, alpha, w, b, out, rows); break;
-    case 12: hipLaunchKernelGGL(k_add_ln<12>, grid, blk, 0, st, x, res, alpha, w, b, out, rows); break;
-    case 16: hipLaunchKernelGGL(k_add_ln<16>, grid, blk, 0, st, x, res, alpha, w, b, out, rows); break;
+    case 1: hipLaunchKernelGGL(k_add_ln<1>, grid, blk, 0, st, x, res, alpha, w, b, out, rows, silu); break;
+    case 2: hipLaunchKernelGGL(k_add_ln<2>, grid, blk, 0, st, x, res, alpha, w, b, out, rows, silu); break;
+    case 3: hipLaunchKernelGGL(k_add_ln<3>, grid, blk, 0, st, x, res, alpha, w, b, out, rows, silu); break;
+    case 4: hipLaunchKernelGGL(k_add_ln<4>, grid, blk, 0, st, x, res, alpha, w, b, out, rows, silu); break;
+    case 5: hipLaunchKernelGGL(k_add_ln<5>, grid, blk, 0, st, x, res, alpha, w, b, out, rows, silu); break;
+    case 6: hipLaunchKernelGGL(k_add_ln<6>, grid, blk, 0, st, x, res, alpha, w, b, out, rows, silu); break;
+    case 7: hipLaunchKernelGGL(k_add_ln<7>, grid, blk, 0, st, x, res, alpha, w, b, out, rows, silu); break;
+    case 8: hipLaunchKernelGGL(k_add_ln<8>, grid, blk, 0, st, x, res, alpha, w, b, out, rows, silu); break;
+    case 12: hipLaunchKernelGGL(k_add_ln<12>, grid, blk, 0, st, x, res, alpha, w, b, out, rows, silu); break;
+    case 16: hipLaunchKernelGGL(k_add_ln<16>, grid, blk, 0, st, x, res, alpha, w, b, out, rows, silu); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -625,13 +626,13 @@ hipError_t mh_launch_add_ln(float *x, const float *res, float alpha, const float
 bool mh_add_ln_prep_supported(int d) { return d > 0 && d % 256 == 0 && d / 256 <= 8; }
 
 hipError_t mh_launch_add_ln_prep(float *x, const float *res, float alpha, const float *w, const float *b, int rows,
-                                 int d, uint8_t *xp, float *xpf, hipStream_t st) {
+                                 int d, bool silu, uint8_t *xp, float *xpf, hipStream_t st) {
     if (rows <= 0) return hipSuccess;
     if (!mh_add_ln_prep_supported(d)) return hipErrorInvalidValue;
     const dim3 grid(mh_mpad(rows) / 8), blk(512);
     switch (d / 256) {
 #define LNP(V) \
-    case V: hipLaunchKernelGGL(k_add_ln_prep<V>, grid, blk, 0, st, x, res, alpha, w, b, rows, xp, xpf); break;
+    case V: hipLaunchKernelGGL(k_add_ln_prep<V>, grid, blk, 0, st, x, res, alpha, w, b, rows, silu, xp, xpf); break;
     LNP(1) LNP(2) LNP(3) LNP(4) LNP(5) LNP(6) LNP(7) LNP(8)
 #undef LNP
     default: return hipErrorInvalidValue;

@@ -58,6 +58,7 @@ __global__ __launch_bounds__(512, (WM * WN == 1 ? 4 : 2)) void k_gemm_ks(GemmJob
     const int job = tr / tilesN, tn = tr - job * tilesN;
     const DevW W = job == 0 ? J.W[0] : (job == 1 ? J.W[1] : J.W[2]);
     float *__restrict__ y = job == 0 ? J.y[0] : (job == 1 ? J.y[1] : J.y[2]);
+    const float *__restrict__ bias = job == 0 ? J.bias[0] : (job == 1 ? J.bias[1] : J.bias[2]);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hh = lane >> 5, col = lane & 31;
     const int pcI = wave % PC, s = wave / PC;
@@ -202,7 +203,9 @@ __global__ __launch_bounds__(512, (WM * WN == 1 ? 4 : 2)) void k_gemm_ks(GemmJob
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 float t = total[v][j];
-                if constexpr (QT == QT_F32) t = ldexpf(t, -wshift<QT>(W, TC * tn + 4 * l32 + j));
+                const int n = TC * tn + 4 * l32 + j;
+                if constexpr (QT == QT_F32) t = ldexpf(t, -wshift<QT>(W, n));
+                if (bias && n < W.n) t = t + bias[n];
                 xs[j] = silu_f(t);
                 amax = fmaxf(amax, fabsf(xs[j]));
             }
@@ -256,23 +259,22 @@ __global__ __launch_bounds__(512, (WM * WN == 1 ? 4 : 2)) void k_gemm_ks(GemmJob
 #pragma unroll
         for (int j = 0; j < V; j++) {
             o[j] = total[v][j];
-            if constexpr (QT == QT_F32) o[j] = ldexpf(o[j], -wshift<QT>(W, min(n + j, W.n - 1)));
+            const int nj = min(n + j, W.n - 1);
+            if constexpr (QT == QT_F32) o[j] = ldexpf(o[j], -wshift<QT>(W, nj));
+            if (bias) o[j] = o[j] + bias[nj];
         }
         if (vec) {
             typedef float fv __attribute__((ext_vector_type(V)));
             fv r = {};
-            if (act >= 2) r = *(const fv *)yp;
+            if (act_res(act)) r = *(const fv *)yp;
             fv w;
 #pragma unroll
-            for (int j = 0; j < V; j++) {
-                const float ry = r[j];
-                w[j] = epi_out(act, o[j], &ry);
-            }
+            for (int j = 0; j < V; j++) w[j] = epi_out(act, o[j], r[j]);
             *(fv *)yp = w;
         } else {
 #pragma unroll
             for (int j = 0; j < V; j++)
-                if (n + j < W.n) yp[j] = epi_out(act, o[j], yp + j);
+                if (n + j < W.n) yp[j] = epi_out(act, o[j], act_res(act) ? yp[j] : 0.0f);
         }
     }
 }

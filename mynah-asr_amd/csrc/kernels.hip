@@ -178,6 +178,7 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
     const int job = tr / tilesN, tn = tr - job * tilesN;
     const DevW W = job == 0 ? J.W[0] : (job == 1 ? J.W[1] : J.W[2]);
     float *__restrict__ y = job == 0 ? J.y[0] : (job == 1 ? J.y[1] : J.y[2]);
+    const float *__restrict__ bias = job == 0 ? J.bias[0] : (job == 1 ? J.bias[1] : J.bias[2]);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int hh = lane >> 5, col = lane & 31;
@@ -350,7 +351,9 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
         static_assert(2 * L::BYTES >= (64 * RS + 128) * 4, "LDS tile");
         float *T = (float *)&sbuf[0][0];
         float *amx = T + 64 * RS;  // [2 row groups][2 halves][32 rows]
-        const int shw = wshift<QT>(W, 32 * (GC0 + wave) + col);  // (the pad columns hold 0)
+        const int np = 32 * (GC0 + wave) + col, shw = wshift<QT>(W, np);  // (the pad columns hold 0)
+        const bool hb = bias && np < W.n;
+        const float bn = hb ? bias[np] : 0.0f;
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < WM; i++)
@@ -358,6 +361,7 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
             for (int e = 0; e < 16; e++) {
                 float v = total[i][0][e];
                 if constexpr (QT == QT_F32) v = ldexpf(v, -shw);
+                if (hb) v = v + bn;
                 T[(32 * i + drow(e, hh)) * RS + 32 * wave + col] = silu_f(v);
             }
         __syncthreads();
@@ -412,8 +416,21 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
     for (int j = 0; j < WN; j++) {
         const int n = 32 * (GC0 + WN * wave + j) + col;
         if (n >= W.n) continue;
-        const int shw = wshift<QT>(W, n);
-        if (act >= 2) {
+        if constexpr (QT == QT_F32) {
+            const int shw = wshift<QT>(W, n);
+#pragma unroll
+            for (int i = 0; i < WM; i++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) total[i][j][e] = ldexpf(total[i][j][e], -shw);
+        }
+        if (bias) {
+            const float bn = bias[n];
+#pragma unroll
+            for (int i = 0; i < WM; i++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) total[i][j][e] = total[i][j][e] + bn;
+        }
+        if (act_res(act)) {
             // the residual adds: every value of y this lane adds to is loaded
             // first, so the loads are in flight together
             float r[WM][16];
@@ -430,23 +447,23 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
 #pragma unroll
                 for (int e = 0; e < 16; e++) {
                     const int m = 32 * (G0 + i) + drow(e, hh);
-                    if (m >= M) continue;
-                    float v = total[i][j][e];
-                    if constexpr (QT == QT_F32) v = ldexpf(v, -shw);
-                    y[(size_t)m * W.n + n] = fmaf(a, v, r[i][e]);
+                    if (m < M) y[(size_t)m * W.n + n] = fmaf(a, total[i][j][e], r[i][e]);
                 }
             continue;
         }
+        // (one branch on act, not one per element)
+        auto put = [&](auto f) {
 #pragma unroll
-        for (int i = 0; i < WM; i++)
+            for (int i = 0; i < WM; i++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const int m = 32 * (G0 + i) + drow(e, hh);
-                if (m >= M) continue;
-                float v = total[i][j][e];
-                if constexpr (QT == QT_F32) v = ldexpf(v, -shw);
-                y[(size_t)m * W.n + n] = act ? silu_f(v) : v;
-            }
+                for (int e = 0; e < 16; e++) {
+                    const int m = 32 * (G0 + i) + drow(e, hh);
+                    if (m < M) y[(size_t)m * W.n + n] = f(total[i][j][e]);
+                }
+        };
+        if (act == 1) put([](float v) { return silu_f(v); });
+        else if (act == 4) put([](float v) { return v < 0.0f ? 0.0f : v; });
+        else put([](float v) { return v; });
     }
 }
 
@@ -1851,10 +1868,11 @@ hipError_t mh_launch_gemv(int qtype, const DevW &W, const float *x, int M, int v
 }
 
 hipError_t mh_launch_gemm(int qtype, const DevW &W, const uint8_t *xp, const float *xs16,
-                          const float *xpf, float *y, int M, int act, hipStream_t st, bool a1) {
+                          const float *xpf, float *y, int M, int act, const float *bias, hipStream_t st, bool a1) {
     GemmJobs J{};
     J.W[0] = J.W[1] = J.W[2] = W;
     J.y[0] = J.y[1] = J.y[2] = y;
+    J.bias[0] = bias;
     J.n = 1;
     MH_DISPATCH(gemm_t, qtype, J, xp, xs16, xpf, M, act, nullptr, st, a1)
 }
@@ -1865,11 +1883,12 @@ hipError_t mh_launch_gemm_jobs(int qtype, const GemmJobs &J, const uint8_t *xp, 
 }
 
 hipError_t mh_launch_gemm_prep_out(int qtype, const DevW &W, const uint8_t *xp, const float *xs16,
-                                   const float *xpf, int M, uint8_t *oxp, float *oxs16, float *oxpf, int oKc,
-                                   int oxsum, hipStream_t st) {
+                                   const float *xpf, int M, const float *bias, uint8_t *oxp, float *oxs16, float *oxpf,
+                                   int oKc, int oxsum, hipStream_t st) {
     const PrepOut po{oxp, (uint8_t *)oxs16, oxpf, oKc, oxsum};
     GemmJobs J{};
     J.W[0] = J.W[1] = J.W[2] = W;
+    J.bias[0] = bias;
     J.n = 1;
     MH_DISPATCH(gemm_t, qtype, J, xp, xs16, xpf, M, 1, &po, st)
 }

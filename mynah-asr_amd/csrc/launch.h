@@ -57,13 +57,16 @@ hipError_t mh_launch_gemv_jobs(int qtype, const GJobs &J, const float *x, int M,
 // keys per attention split of the decoder step
 constexpr int MH_ATT_KC = 64;
 __host__ __device__ inline int mh_att_splits_dev(int n) { return (n + MH_ATT_KC - 1) / MH_ATT_KC; }
-// a1: the INT8ACT form of the product, on activations prepared by mh_launch_prep_a1
+// y = epilogue(x W^T + bias): bias [n] or null, act 0 none, 1 SiLU, 2 / 3 added (or
+// half of it) into y, 4 ReLU. a1: the INT8ACT form of the product, on activations
+// prepared by mh_launch_prep_a1
 hipError_t mh_launch_gemm(int qtype, const DevW &W, const uint8_t *xp, const float *xs16,
-                          const float *xpf, float *y, int M, int act, hipStream_t st, bool a1 = false);
+                          const float *xpf, float *y, int M, int act, const float *bias, hipStream_t st, bool a1 = false);
 // up to three products (same shape) of one prepared input in one launch
 struct GemmJobs {
     DevW W[3];
     float *y[3];
+    const float *bias[3];   // [n] or null
     int n;
 };
 hipError_t mh_launch_gemm_jobs(int qtype, const GemmJobs &J, const uint8_t *xp, const float *xs16,
@@ -72,8 +75,8 @@ hipError_t mh_launch_gemm_jobs(int qtype, const GemmJobs &J, const uint8_t *xp, 
 // product with Kp = 128 * oKc (oKc = the first product's column tiles):
 // (oxp, oxs16, oxpf) as mh_launch_prep would write them.
 hipError_t mh_launch_gemm_prep_out(int qtype, const DevW &W, const uint8_t *xp, const float *xs16,
-                                   const float *xpf, int M, uint8_t *oxp, float *oxs16, float *oxpf, int oKc,
-                                   int oxsum, hipStream_t st);
+                                   const float *xpf, int M, const float *bias, uint8_t *oxp, float *oxs16, float *oxpf,
+                                   int oKc, int oxsum, hipStream_t st);
 hipError_t mh_launch_dequant(int qtype, const DevW &W, float *out, hipStream_t st);
 // a plain streaming read of `bytes` (16-byte aligned), nothing written
 hipError_t mh_launch_read_floor(const void *p, size_t bytes, hipStream_t st);
@@ -117,16 +120,16 @@ hipError_t mh_launch_relpos_attn(const float *q, const float *k, const float *v,
 // Encoder layer steps around the products (encoder.hip). d: 256 * {1..8, 12,
 // 16} for the layer norm (mh_enc_d_supported), a multiple of 4 for the rest.
 bool mh_enc_d_supported(int d);
-// x += alpha * res (res may be null: no add), then out = LN(x) (w, b) per row;
-// out may be x
+// x += alpha * res (res may be null: no add), then out = LN(x) (w, b) per row,
+// then SiLU of it with silu; out may be x
 hipError_t mh_launch_add_ln(float *x, const float *res, float alpha, const float *w, const float *b, float *out,
-                            int rows, int d, hipStream_t st);
+                            int rows, int d, bool silu, hipStream_t st);
 // the same, its output as the EXACT products' prepared input (xp: mh_mpad(rows)
 // * d * 4 bytes, xpf: mh_mpad(rows) * d / 128 floats) in place of f32 rows;
 // for d a multiple of 256 up to 2048
 bool mh_add_ln_prep_supported(int d);
 hipError_t mh_launch_add_ln_prep(float *x, const float *res, float alpha, const float *w, const float *b, int rows,
-                                 int d, uint8_t *xp, float *xpf, hipStream_t st);
+                                 int d, bool silu, uint8_t *xp, float *xpf, hipStream_t st);
 // g [rows, d] = h[:, :d] * sigmoid(h[:, d:]) for h [rows, 2d]
 hipError_t mh_launch_glu(const float *h, float *g, size_t rows, int d, hipStream_t st);
 // depthwise conv over time in each of nseq segments of T rows (w: the taps

@@ -329,13 +329,15 @@ struct PrepOut {
     int Kc, xsum;   // mins A operands (xm_frag): 0 none, 1 of 8 sub-blocks, 2 of 4
 };
 
-// The products' output epilogue (k_gemm spells it out): act
-// 1 SiLU; act 2 and 3 accumulate into y, y = fmaf(1 or 1/2, v, y) (the
-// residual adds x += tmp and x += tmp / 2 of the encoder layer, with their
-// operations); otherwise v.
-__device__ __forceinline__ float epi_out(int act, float v, const float *yp) {
+// The products' output epilogue on v = the product (+ its bias): act 1 SiLU, 4
+// ReLU; act 2 and 3 accumulate into y, y = fmaf(1 or 1/2, v, y) (the residual
+// adds x += tmp and x += tmp / 2 of the encoder layer, with their operations);
+// 0 v. yv: what y holds (for act 2 and 3).
+__device__ __forceinline__ bool act_res(int act) { return act == 2 || act == 3; }
+__device__ __forceinline__ float epi_out(int act, float v, float yv) {
     if (act == 1) return silu_f(v);
-    if (act >= 2) return fmaf(act == 3 ? 0.5f : 1.0f, v, *yp);
+    if (act == 4) return v < 0.0f ? 0.0f : v;
+    if (act_res(act)) return fmaf(act == 3 ? 0.5f : 1.0f, v, yv);
     return v;
 }
 
