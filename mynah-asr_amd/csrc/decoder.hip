@@ -1,22 +1,24 @@
 // decoder.hip — the non-GEMV kernels of the AED (Canary) decoder step
 // (the reference's src/decoder_aed.c:139-232), device-resident:
 //
-//   k_embed_ln   x = LN(emb[token] + pos[p])                  decoder_aed.c:183-186
+//   k_embed_ln   x = LN(emb[token] + pos[p]), a row per position  decoder_aed.c:183-186
+//   k_ln_rows    y = LN(x) per row                             decoder_aed.c:21-28
 //   k_att_part   one query against a split of KC keys, per head: running max,
 //                sum of exponentials and the weighted sum of V rows; with
 //                `append`, the split holding key p first stores this step's
 //                k and v rows into the self-attention cache  decoder_aed.c:124-137, 195-198
-//   k_att_combine the splits of each head merged (the decoder step merges them
-//                instead in the prologue of the GEMV that reads the result)
+//   k_att_combine the splits of each head merged (for given tokens; the decoder
+//                step merges them in the prologue of the GEMV that reads the result)
 //   k_argmax     first maximum of the logits, the next token; advances p and
-//                forms the next position's x as k_embed_ln would (so only
-//                the first position launches k_embed_ln)   decoder_aed.c:217-222
+//                forms the next position's x as k_embed_ln would  decoder_aed.c:217-222
 //   k_bias_rows  y[t] += b                                    decoder_aed.c:132-136
 //
-// The step's position p and its token live in device memory (`st`: st[0] = p,
-// st[1] = the last argmax), so one captured launch sequence serves every
-// step: position p reads prompt[p] while p < n_prompt, else the argmax of the
-// step before (decoder_aed.c:213-222 chooses the same tokens).
+// Positions whose tokens are given (the prompt; all of them when tokens are
+// scored) run as rows of one batch: a row of the products carries the bits of
+// the row alone, and row p attends to the keys up to p.
+// A decoded position p and its token live in device memory (`st`: st[0] = p,
+// st[1] = the last argmax), so one captured launch sequence serves every step
+// (decoder_aed.c:213-222 chooses the same tokens).
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -80,24 +82,37 @@ __device__ void ln_store(float (&v)[V], int d, const float *w, const float *b, f
     }
 }
 
+// row r: position p0 + r
 __global__ __launch_bounds__(LN_T) void k_embed_ln(const float *__restrict__ emb, const float *__restrict__ pos,
-                                                   const int *__restrict__ prompt, int n_prompt,
-                                                   const int *__restrict__ st, const float *__restrict__ w,
-                                                   const float *__restrict__ b, float *__restrict__ x, int d) {
-    const int p = st[0];
-    const int tok = p < n_prompt ? prompt[p] : st[1];
-    const float *e = emb + (size_t)tok * d, *pe = pos + (size_t)p * d;
+                                                   const int *__restrict__ tokens, int p0,
+                                                   const float *__restrict__ w, const float *__restrict__ b,
+                                                   float *__restrict__ x, int d) {
+    const int p = p0 + blockIdx.x;
+    const float *e = emb + (size_t)tokens[p] * d, *pe = pos + (size_t)p * d;
     float v[LN_V];
 #pragma unroll
     for (int u = 0; u < LN_V; u++) {
         const int i = threadIdx.x + LN_T * u;
         v[u] = i < d ? e[i] + pe[i] : 0.0f;
     }
-    ln_store<LN_T, LN_V>(v, d, w, b, x);
+    ln_store<LN_T, LN_V>(v, d, w, b, x + (size_t)blockIdx.x * d);
 }
 
-// Workgroup (head h, split s) over keys [s*KC, min((s+1)*KC, n)), n = n_fixed,
-// or p + 1 for self attention (n_fixed = 0). Four waves, wave w the keys
+__global__ __launch_bounds__(LN_T) void k_ln_rows(const float *__restrict__ x, const float *__restrict__ w,
+                                                  const float *__restrict__ b, float *__restrict__ y, int d) {
+    const float *xr = x + (size_t)blockIdx.x * d;
+    float v[LN_V];
+#pragma unroll
+    for (int u = 0; u < LN_V; u++) {
+        const int i = threadIdx.x + LN_T * u;
+        v[u] = i < d ? xr[i] : 0.0f;
+    }
+    ln_store<LN_T, LN_V>(v, d, w, b, y + (size_t)blockIdx.x * d);
+}
+
+// Workgroup (head h, split s, row z) over keys [s*KC, min((s+1)*KC, n)), n =
+// n_fixed, or p + 1 for self attention (n_fixed = 0): p = st[0], or p0 + z of
+// given tokens (st null), whose keys are all in the cache. Four waves, wave w the keys
 // 16w .. 16w+15 of the split: for the scores 4 lanes per key (DK/4 features
 // each, q read by every lane from global); for the values lane = features
 // DK/64 per lane over the wave's 16 keys. Two workgroup barriers: the waves'
@@ -106,7 +121,7 @@ __global__ __launch_bounds__(LN_T) void k_embed_ln(const float *__restrict__ emb
 template <int DK>
 __global__ __launch_bounds__(256) void k_att_part(const float *__restrict__ q, float *K, float *V,
                                                   const float *__restrict__ kn, const float *__restrict__ vn,
-                                                  const int *__restrict__ st, int n_fixed, int d, float scale,
+                                                  const int *__restrict__ st, int p0, int n_fixed, int d, float scale,
                                                   float *__restrict__ o_part, float *__restrict__ ml_part,
                                                   int nsplit) {
     static_assert(KC == 64, "four waves of 16 keys");
@@ -115,17 +130,20 @@ __global__ __launch_bounds__(256) void k_att_part(const float *__restrict__ q, f
     __shared__ float wo[4][DK];
     const int h = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int ho = h * DK;
-    const int p = n_fixed > 0 ? -1 : st[0];   // (cross attention does not wait for st)
+    // (cross attention does not wait for st)
+    const int p = n_fixed > 0 ? -1 : st ? st[0] : p0 + (int)blockIdx.z;
+    const size_t hs = (size_t)blockIdx.z * gridDim.x + h;   // (row, head)
+    q += (size_t)blockIdx.z * d;
     const int n = n_fixed > 0 ? n_fixed : p + 1;
     const int j0 = s * KC, j1 = min(j0 + KC, n);
-    float *op = o_part + ((size_t)h * nsplit + s) * DK;
-    float *mlp = ml_part + ((size_t)h * nsplit + s) * 2;
+    float *op = o_part + (hs * nsplit + s) * DK;
+    float *mlp = ml_part + (hs * nsplit + s) * 2;
     if (j0 >= j1) {   // nothing in this split (uniform per workgroup)
         if (tid < DK) op[tid] = 0.0f;
         if (tid == 0) mlp[0] = -INFINITY, mlp[1] = 0.0f;
         return;
     }
-    const bool append = n_fixed == 0 && p >= j0 && p < j1;
+    const bool append = n_fixed == 0 && kn && p >= j0 && p < j1;
     if (append && tid < DK) {   // this step's k, v rows join the cache (read below from kn, vn)
         K[(size_t)p * d + ho + tid] = kn[ho + tid];
         V[(size_t)p * d + ho + tid] = vn[ho + tid];
@@ -198,45 +216,42 @@ __global__ __launch_bounds__(256) void k_att_part(const float *__restrict__ q, f
 // out[h] = sum_s o_s e^(m_s - M) / sum_s l_s e^(m_s - M) over the used splits
 template <int DK>
 __global__ __launch_bounds__(DK) void k_att_combine(const float *__restrict__ o_part,
-                                                    const float *__restrict__ ml_part, const int *__restrict__ st,
-                                                    int n_fixed, float *__restrict__ out, int nsplit) {
-    const int h = blockIdx.x, f = threadIdx.x;
-    const int n = n_fixed > 0 ? n_fixed : st[0] + 1;
+                                                    const float *__restrict__ ml_part, int p0, int n_fixed,
+                                                    float *__restrict__ out, int nsplit) {
+    const int h = blockIdx.x, z = blockIdx.y, f = threadIdx.x;
+    const size_t hs = (size_t)z * gridDim.x + h;
+    const int n = n_fixed > 0 ? n_fixed : p0 + z + 1;
     const int ns = min((n + KC - 1) / KC, nsplit);
-    const float *ml = ml_part + (size_t)h * nsplit * 2;
+    const float *ml = ml_part + hs * nsplit * 2;
     float M = -INFINITY;
     for (int s = 0; s < ns; s++) M = fmaxf(M, ml[2 * s]);
     float L = 0.0f, o = 0.0f;
     for (int s = 0; s < ns; s++) {
         const float c = expf(ml[2 * s] - M);
         L += ml[2 * s + 1] * c;
-        o += o_part[((size_t)h * nsplit + s) * DK + f] * c;
+        o += o_part[(hs * nsplit + s) * DK + f] * c;
     }
-    out[h * DK + f] = o / L;
+    out[hs * DK + f] = o / L;
 }
 
 // First maximum of logits[0..vocab) (the reference's strict > scan) -> st[1];
-// optionally the logits to logits_out[p]; then p + 1 -> st[0].
-__global__ __launch_bounds__(1024) void k_argmax(const float *__restrict__ logits, int vocab, int *st,
-                                                 float *__restrict__ logits_out, MhEmbNext en) {
+// then p + 1 -> st[0] and the next position's input row, while there is one.
+__global__ __launch_bounds__(1024) void k_argmax(const float *__restrict__ logits, int vocab, int *st, MhEmbNext en) {
     __shared__ float bv[16];
     __shared__ int bi[16];
     __shared__ int nxt;
     constexpr int AV = 16;   // logits per thread per batch: all of them go out at once
     const int tid = threadIdx.x, p = st[0];
-    // the next position's rows that do not depend on this argmax go out first
+    // the next position's row that does not depend on this argmax goes out first
     const int q = p + 1;
-    const bool next = en.emb && q < en.max_pos;   // (uniform)
-    float pv[4], ev[4];   // d <= 4096
-    const bool in_prompt = next && q < en.n_prompt;
+    const bool next = q < en.max_pos;   // (uniform)
+    float pv[4];   // d <= 4096
     if (next) {
         const float *pe = en.pos + (size_t)q * en.d;
-        const float *e = in_prompt ? en.emb + (size_t)en.prompt[q] * en.d : nullptr;
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const int i = tid + 1024 * u;
             pv[u] = i < en.d ? pe[i] : 0.0f;
-            ev[u] = in_prompt && i < en.d ? e[i] : 0.0f;
         }
     }
     float best = -INFINITY;
@@ -251,10 +266,7 @@ __global__ __launch_bounds__(1024) void k_argmax(const float *__restrict__ logit
 #pragma unroll
         for (int u = 0; u < AV; u++) {
             const int i = i0 + tid + 1024 * u;
-            if (i < vocab) {
-                if (v[u] > best) best = v[u], idx = i;   // i grows: a tie keeps the earlier index
-                if (logits_out) logits_out[(size_t)p * vocab + i] = v[u];
-            }
+            if (i < vocab && v[u] > best) best = v[u], idx = i;   // i grows: a tie keeps the earlier index
         }
     }
     for (int o = 32; o > 0; o >>= 1) {
@@ -274,17 +286,13 @@ __global__ __launch_bounds__(1024) void k_argmax(const float *__restrict__ logit
     // the next position's input row, as k_embed_ln would form it
     if (!next) return;
     __syncthreads();
-    if (!in_prompt) {
-        const float *e = en.emb + (size_t)nxt * en.d;
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int i = tid + 1024 * u;
-            ev[u] = i < en.d ? e[i] : 0.0f;
-        }
-    }
+    const float *e = en.emb + (size_t)nxt * en.d;
     float v[4];
 #pragma unroll
-    for (int u = 0; u < 4; u++) v[u] = ev[u] + pv[u];
+    for (int u = 0; u < 4; u++) {
+        const int i = tid + 1024 * u;
+        v[u] = (i < en.d ? e[i] : 0.0f) + pv[u];
+    }
     ln_store<1024, 4>(v, en.d, en.w, en.b, en.x);
 }
 
@@ -302,38 +310,56 @@ __global__ void k_set_state(int *st, int p, int cur) {
 
 int mh_att_splits(int n) { return mh_att_splits_dev(n); }
 
-hipError_t mh_launch_embed_ln(const float *emb, const float *pos, const int *prompt, int n_prompt, const int *st,
-                              const float *w, const float *b, float *x, int d, hipStream_t s) {
+hipError_t mh_launch_embed_ln(const float *emb, const float *pos, const int *tokens, int p0, int rows, const float *w,
+                              const float *b, float *x, int d, hipStream_t s) {
     if (d > LN_T * LN_V) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_embed_ln, dim3(1), dim3(LN_T), 0, s, emb, pos, prompt, n_prompt, st, w, b, x, d);
+    hipLaunchKernelGGL(k_embed_ln, dim3(rows), dim3(LN_T), 0, s, emb, pos, tokens, p0, w, b, x, d);
+    return hipGetLastError();
+}
+
+hipError_t mh_launch_ln_rows(const float *x, const float *w, const float *b, float *y, int rows, int d, hipStream_t s) {
+    if (d > LN_T * LN_V) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_ln_rows, dim3(rows), dim3(LN_T), 0, s, x, w, b, y, d);
     return hipGetLastError();
 }
 
 hipError_t mh_launch_attend1(const float *q, float *K, float *V, const float *kn, const float *vn, const int *st,
-                             int n_fixed, int d, int H, float *o_part, float *ml_part, int nsplit, float *out,
-                             hipStream_t s) {
+                             int n_fixed, int d, int H, float *o_part, float *ml_part, int nsplit, hipStream_t s) {
     const int dk = d / H;
     const float scale = 1.0f / sqrtf((float)dk);
-    if (dk == 128) {
-        hipLaunchKernelGGL(k_att_part<128>, dim3(H, nsplit), dim3(256), 0, s, q, K, V, kn, vn, st, n_fixed, d, scale,
+    if (dk == 128)
+        hipLaunchKernelGGL(k_att_part<128>, dim3(H, nsplit), dim3(256), 0, s, q, K, V, kn, vn, st, 0, n_fixed, d, scale,
                            o_part, ml_part, nsplit);
-        if (out)
-            hipLaunchKernelGGL(k_att_combine<128>, dim3(H), dim3(128), 0, s, o_part, ml_part, st, n_fixed, out, nsplit);
-    } else if (dk == 64) {
-        hipLaunchKernelGGL(k_att_part<64>, dim3(H, nsplit), dim3(256), 0, s, q, K, V, kn, vn, st, n_fixed, d, scale,
+    else if (dk == 64)
+        hipLaunchKernelGGL(k_att_part<64>, dim3(H, nsplit), dim3(256), 0, s, q, K, V, kn, vn, st, 0, n_fixed, d, scale,
                            o_part, ml_part, nsplit);
-        if (out)
-            hipLaunchKernelGGL(k_att_combine<64>, dim3(H), dim3(64), 0, s, o_part, ml_part, st, n_fixed, out, nsplit);
-    } else {
+    else
         return hipErrorInvalidValue;
-    }
     return hipGetLastError();
 }
 
-hipError_t mh_launch_argmax(const float *logits, int vocab, int *st, float *logits_out, const MhEmbNext *en,
-                            hipStream_t s) {
-    if (en && en->emb && en->d > 4096) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_argmax, dim3(1), dim3(1024), 0, s, logits, vocab, st, logits_out, en ? *en : MhEmbNext{});
+template <int DK>
+static void attend_rows(const float *q, float *K, float *V, int p0, int rows, int n_fixed, int d, int H, float *o_part,
+                        float *ml_part, int nsplit, float *out, hipStream_t s) {
+    const float scale = 1.0f / sqrtf((float)DK);
+    hipLaunchKernelGGL(k_att_part<DK>, dim3(H, nsplit, rows), dim3(256), 0, s, q, K, V, nullptr, nullptr, nullptr, p0,
+                       n_fixed, d, scale, o_part, ml_part, nsplit);
+    hipLaunchKernelGGL(k_att_combine<DK>, dim3(H, rows), dim3(DK), 0, s, o_part, ml_part, p0, n_fixed, out, nsplit);
+}
+
+hipError_t mh_launch_attend_rows(const float *q, float *K, float *V, int p0, int rows, int n_fixed, int d, int H,
+                                 float *o_part, float *ml_part, int nsplit, float *out, hipStream_t s) {
+    const int ns = mh_att_splits(n_fixed > 0 ? n_fixed : p0 + rows);   // (the last row's)
+    if (ns > nsplit) return hipErrorInvalidValue;
+    if (d / H == 128) attend_rows<128>(q, K, V, p0, rows, n_fixed, d, H, o_part, ml_part, ns, out, s);
+    else if (d / H == 64) attend_rows<64>(q, K, V, p0, rows, n_fixed, d, H, o_part, ml_part, ns, out, s);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+hipError_t mh_launch_argmax(const float *logits, int vocab, int *st, const MhEmbNext &en, hipStream_t s) {
+    if (en.d > 4096) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_argmax, dim3(1), dim3(1024), 0, s, logits, vocab, st, en);
     return hipGetLastError();
 }
 

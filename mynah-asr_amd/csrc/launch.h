@@ -171,28 +171,29 @@ hipError_t mh_launch_bias_scale(float *y, const float *b, size_t rows, int d, fl
 
 // AED decoder step kernels (decoder.hip); st = device int[2]: position p, last argmax
 int mh_att_splits(int n);   // attention splits for n keys
-hipError_t mh_launch_embed_ln(const float *emb, const float *pos, const int *prompt, int n_prompt, const int *st,
-                              const float *w, const float *b, float *x, int d, hipStream_t s);
-// out = attention of q over n keys (n_fixed, or p + 1 with the cache append of kn, vn when n_fixed == 0);
-// out == NULL: the splits only (merged by a GPRO_COMB prologue);
-// o_part [H][nsplit][dk], ml_part [H][nsplit][2]
+// x [rows, d] = LN(emb[tokens[p]] + pos[p]) for positions p = p0 .. p0 + rows - 1
+hipError_t mh_launch_embed_ln(const float *emb, const float *pos, const int *tokens, int p0, int rows, const float *w,
+                              const float *b, float *x, int d, hipStream_t s);
+// y = LN(x) per row, as the decoder's layer norms (d <= 4096)
+hipError_t mh_launch_ln_rows(const float *x, const float *w, const float *b, float *y, int rows, int d, hipStream_t s);
+// one position's attention of q over n keys (n_fixed, or p + 1 with the cache append of kn, vn when n_fixed == 0),
+// as splits merged by a GPRO_COMB prologue: o_part [H][nsplit][dk], ml_part [H][nsplit][2]
 hipError_t mh_launch_attend1(const float *q, float *K, float *V, const float *kn, const float *vn, const int *st,
-                             int n_fixed, int d, int H, float *o_part, float *ml_part, int nsplit, float *out,
-                             hipStream_t s);
+                             int n_fixed, int d, int H, float *o_part, float *ml_part, int nsplit, hipStream_t s);
+// out [rows, d] = attention of positions p0 .. p0 + rows - 1 over n_fixed keys, or row p over the p + 1 keys of the
+// cache (n_fixed == 0); o_part [rows][H][nsplit][dk], ml_part [rows][H][nsplit][2] with nsplit splits at least
+hipError_t mh_launch_attend_rows(const float *q, float *K, float *V, int p0, int rows, int n_fixed, int d, int H,
+                                 float *o_part, float *ml_part, int nsplit, float *out, hipStream_t s);
 // The next position's input row, formed by the argmax kernel once it has the
-// token: x = LN(emb[tok] + pos[q]) for q = p + 1 < max_pos, tok = prompt[q]
-// while q < n_prompt, else the argmax (d <= 4096)
+// token: x = LN(emb[tok] + pos[q]) for q = p + 1 < max_pos (d <= 4096)
 struct MhEmbNext {
     const float *emb, *pos;
-    const int *prompt;
-    int n_prompt, max_pos;
+    int max_pos;
     const float *w, *b;
     float *x;
     int d;
 };
-// first maximum of the logits into st[1], st[0] advanced; logits_out (if not
-// null) receives row p of the logits; en (if not null) as above
-hipError_t mh_launch_argmax(const float *logits, int vocab, int *st, float *logits_out, const MhEmbNext *en,
-                            hipStream_t s);
+// first maximum of the logits into st[1], st[0] advanced; en as above
+hipError_t mh_launch_argmax(const float *logits, int vocab, int *st, const MhEmbNext &en, hipStream_t s);
 hipError_t mh_launch_bias_rows(float *y, const float *b, size_t rows, int d, hipStream_t s);
 hipError_t mh_launch_set_state(int *st, int p, int cur, hipStream_t s);

@@ -142,6 +142,36 @@ def test_aed_greedy_tokens(gpu, orc, d, H, ffn, vocab, nl, T, qt, d_enc):
     dev.close()
 
 
+# given tokens run in batches of 64 rows: one row, the GEMV's rows (up to 16,
+# and 8 where K = 2048 splits), the GEMM from 17, an exact batch, one over, and
+# a batch that starts inside the second split of keys
+@pytest.mark.parametrize("qt,ffn", [(M.Q8_0, 512), (M.Q4_K, 2048), (M.F32, 256)])
+@pytest.mark.parametrize("n", [1, 2, 16, 17, 64, 65, 150])
+def test_aed_given_tokens(gpu, orc, qt, ffn, n):
+    """n scored tokens against the oracle, and greedy decoding after a prompt of
+    n tokens against the oracle's choice (its margin decides a near tie)."""
+    import torch
+    say("aed given", M.NAMES[qt], ffn, n)
+    d, H, vocab, T = 256, 4, 300, 70
+    params = make_params(d + ffn, d, H, ffn, vocab, 2, n + 3)
+    dev = M.DeviceAed(gpu, params, H, qt)
+    enc = np.random.default_rng(17).standard_normal((T, d)).astype(np.float32)
+    denc = torch.from_numpy(enc).cuda()
+    toks = [int(t) for t in np.random.default_rng(18 + n).integers(0, vocab, n)]
+    om = oracle_model(orc, dev, params, H)
+    check_logits(dev.forced(denc.data_ptr(), T, toks), om.forced(enc, toks), f"given {M.NAMES[qt]} n={n}")
+    for cap in (0, 1, 5):   # 5: the length limit n + 3 ends it
+        ref, margins = om.decode(enc, toks, eos=-1, cap=cap, max_seq=n + 3)
+        got = dev.decode(denc.data_ptr(), T, toks, eos=-1, cap=cap)
+        assert len(got) == len(ref)
+        for i, (a, b) in enumerate(zip(got, ref)):
+            if a != b:
+                lg = om.forced(enc, toks + ref[:i])[-1]
+                assert margins[i] <= 1e-4 * np.abs(lg).max() + 1e-5 * np.sqrt((lg ** 2).mean()), (cap, i, a, b)
+                break
+    dev.close()
+
+
 def test_aed_rejects_unsupported(gpu):
     import torch
     params = make_params(1, 96, 1, 128, 100, 1, 8)   # head size 96
