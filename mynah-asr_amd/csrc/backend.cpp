@@ -538,10 +538,10 @@ int aed_gemv(const mynah_asr_hip_weight *const *Ws, float *const *ys, const GEpi
     return e == hipSuccess ? 0 : fail("gemv launch failed", hipGetErrorString(e));
 }
 
-GPro pro_ln(const float *x, const float *w, const float *b) {
+GPro pro_ln(const float *x, const float *w, const float *b, int k) {
     GPro p{};
     p.kind = GPRO_LN;
-    p.x = x, p.w = w, p.b = b;
+    p.x = x, p.w = w, p.b = b, p.rk = 1.0 / k;
     return p;
 }
 
@@ -605,7 +605,7 @@ int aed_rows(Ctx *c, const mynah_asr_hip_aed *a, const AedBufs &b, int T, int ma
 // The final layer norm, the head and the argmax of the row x at position st[0]:
 // st advances and the next position's input row is formed in b.x.
 int aed_sample(const mynah_asr_hip_aed *a, const AedBufs &b, const float *x, int max_len, hipStream_t st) {
-    if (aed_one(a->head, b.logits, GEpi{0, a->head_b, nullptr}, pro_ln(x, a->fin_w, a->fin_b), st)) return -1;
+    if (aed_one(a->head, b.logits, GEpi{0, a->head_b, nullptr}, pro_ln(x, a->fin_w, a->fin_b, a->d), st)) return -1;
     const MhEmbNext en{a->emb, a->pos, max_len, a->embln_w, a->embln_b, b.x, a->d};
     AED_TRY(mh_launch_argmax(b.logits, a->vocab, b.st, en, st));
     return 0;
@@ -625,7 +625,7 @@ int aed_step(const mynah_asr_hip_aed *a, const AedBufs &b, int T, int max_len, h
         float *const qkv_y[3] = {b.q, b.kn, b.vn};
         const GEpi qkv_ep[3] = {{0, L->sq_b, nullptr}, {0, L->sk_b, nullptr}, {0, L->sv_b, nullptr}};
         const bool same = L->sk->qtype == L->sq->qtype && L->sv->qtype == L->sq->qtype;
-        const GPro ln_self = pro_ln(b.x, L->ln_self_w, L->ln_self_b);
+        const GPro ln_self = pro_ln(b.x, L->ln_self_w, L->ln_self_b, d);
         if (same) {
             if (aed_gemv(qkv, qkv_y, qkv_ep, 3, ln_self, nullptr, st)) return -1;
         } else {
@@ -635,12 +635,12 @@ int aed_step(const mynah_asr_hip_aed *a, const AedBufs &b, int T, int max_len, h
         AED_TRY(mh_launch_attend1(b.q, SK, SV, b.kn, b.vn, b.st, 0, d, H, b.opart, b.ml, b.nsplit, st));
         if (aed_one(L->so, b.x, GEpi{0, L->so_b, b.x}, pro_comb(b, 0, H), st)) return -1;
         // cross attention over the projected encoder output
-        if (aed_one(L->cq, b.q, GEpi{0, L->cq_b, nullptr}, pro_ln(b.x, L->ln_cross_w, L->ln_cross_b), st)) return -1;
+        if (aed_one(L->cq, b.q, GEpi{0, L->cq_b, nullptr}, pro_ln(b.x, L->ln_cross_w, L->ln_cross_b, d), st)) return -1;
         AED_TRY(mh_launch_attend1(b.q, CK, CV, nullptr, nullptr, b.st, T, d, H, b.opart, b.ml, b.nsplit, st));
         if (aed_one(L->co, b.x, GEpi{0, L->co_b, b.x}, pro_comb(b, T, H), st)) return -1;
         // ReLU FFN
         const GEpi ff2_ep{0, L->ff2_b, b.x};
-        if (aed_one(L->ff1, b.ff, GEpi{2, L->ff1_b, nullptr}, pro_ln(b.x, L->ln_ffn_w, L->ln_ffn_b), st) ||
+        if (aed_one(L->ff1, b.ff, GEpi{2, L->ff1_b, nullptr}, pro_ln(b.x, L->ln_ffn_w, L->ln_ffn_b, d), st) ||
             aed_gemv(&L->ff2, &b.x, &ff2_ep, 1, GPro{}, b.ff, st))
             return -1;
     }

@@ -490,7 +490,7 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
 //
 //   GPRO_LN   (float)(((double)x - mean) * (double)inv) * w + b with inv =
 //             (float)(1 / sqrt(var + 1e-5)), mean and var over the K values in
-//             double, two passes (decoder_aed.c:21-28)
+//             double (decoder_aed.c:21-28)
 //   GPRO_COMB the attention splits of the element's head merged:
 //             sum_s o_s e^(m_s - M) / sum_s l_s e^(m_s - M), in split order
 constexpr int PRO_XB = 8;   // chunks of x per batch of the layer-norm sums (1024 values)
@@ -501,8 +501,7 @@ struct WaveRow {
     // then mu and inv; GPRO_COMB: n = the keys, a / b = (m, l) and the lane's
     // two partial outputs of the chunk's first PRO_MB splits
     float2 a[PRO_MB], b[PRO_MB];
-    double mu;
-    float inv;
+    double mu, inv;
     bool have;
     int n;
     float2 xc, wc, bc;   // (GPRO_LN) this chunk's own operands
@@ -573,41 +572,46 @@ __device__ __forceinline__ float2 wave_row_values(const GPro &pro, int K, int c,
     const bool live = e < K;
     if (pro.kind == GPRO_LN) {
         if (!r.have) {
-            // two passes in double, as ln(): the mean, then the sum of (x - mean)^2
-            double s = 0.0;
-#pragma unroll
-            for (int u = 0; u < PRO_XB; u++) s += (double)r.a[u].x + (double)r.a[u].y;
-            for (int c0 = PRO_XB; 128 * c0 < K; c0 += PRO_XB)   // K > 1024: further batches
-#pragma unroll
-                for (int u = 0; u < PRO_XB; u++) {
-                    const int ee = 128 * (c0 + u) + 2 * lane;
-                    const float2 v = ee < K ? ld2(pro.x + ee) : float2{0.0f, 0.0f};
-                    s += (double)v.x + (double)v.y;
-                }
-            r.mu = wave_sum(s) / K;
-            double q = 0.0;
+            // Mean and variance over the row in double in one pass, of the
+            // differences to x[0]: (x[0] - mean)^2 <= K var, so what cancels
+            // in the variance is at most K^2 2^-53 of it. 1/sqrt by the
+            // hardware's estimate (about 24 bits) and two Newton steps. (Two
+            // passes with their divisions and square root are a chain of about
+            // 2300 cycles.)
+            const double x0 = (double)__shfl(r.a[0].x, 0, 64);
+            double s = 0.0, q = 0.0;
+            auto add = [&](float2 v) {
+                const double d0 = (double)v.x - x0, d1 = (double)v.y - x0;
+                s += d0 + d1;
+                q += d0 * d0 + d1 * d1;
+            };
 #pragma unroll
             for (int u = 0; u < PRO_XB; u++)
-                if (128 * u + 2 * lane < K) {
-                    const double d0 = (double)r.a[u].x - r.mu, d1 = (double)r.a[u].y - r.mu;
-                    q += d0 * d0 + d1 * d1;
-                }
-            for (int c0 = PRO_XB; 128 * c0 < K; c0 += PRO_XB)
+                if (128 * u + 2 * lane < K) add(r.a[u]);
+            for (int c0 = PRO_XB; 128 * c0 < K; c0 += PRO_XB) {   // K > 1024: further batches
+                float2 v[PRO_XB];
 #pragma unroll
                 for (int u = 0; u < PRO_XB; u++) {
                     const int ee = 128 * (c0 + u) + 2 * lane;
-                    if (ee < K) {
-                        const float2 v = ld2(pro.x + ee);
-                        const double d0 = (double)v.x - r.mu, d1 = (double)v.y - r.mu;
-                        q += d0 * d0 + d1 * d1;
-                    }
+                    if (ee < K) v[u] = ld2(pro.x + ee);
                 }
-            r.inv = (float)(1.0 / sqrt(wave_sum(q) / K + 1e-5));
+#pragma unroll
+                for (int u = 0; u < PRO_XB; u++)
+                    if (128 * (c0 + u) + 2 * lane < K) add(v[u]);
+            }
+            s = wave_sum(s);
+            q = wave_sum(q);
+            const double rk = pro.rk, m = s * rk, var = q * rk - m * m + 1e-5;
+            r.mu = x0 + m;
+            double y = __builtin_amdgcn_rsq(var);
+#pragma unroll
+            for (int i = 0; i < 2; i++) y = y * (1.5 - 0.5 * var * y * y);
+            r.inv = (double)(float)y;
             r.have = true;
         }
         if (!live) return float2{0.0f, 0.0f};
-        const float t0 = (float)(((double)r.xc.x - r.mu) * (double)r.inv);
-        const float t1 = (float)(((double)r.xc.y - r.mu) * (double)r.inv);
+        const float t0 = (float)(((double)r.xc.x - r.mu) * r.inv);
+        const float t1 = (float)(((double)r.xc.y - r.mu) * r.inv);
         return float2{t0 * r.wc.x + r.bc.x, t1 * r.wc.y + r.bc.y};
     }
     const int dk = K / pro.H, h = live ? e / dk : 0, f = live ? e - h * dk : 0;
@@ -646,6 +650,69 @@ __device__ __forceinline__ float2 wave_row_values(const GPro &pro, int K, int c,
     }
     if (!live) return float2{0.0f, 0.0f};
     return float2{o0 / L, o1 / L};
+}
+
+// The split of one row's chunk by a whole wave (M = 1): lane l holds elements
+// 2l, 2l+1 and splits them as split_vals would (the maximum is the chunk's, the
+// sub-block sums run in element order), then the 128 (hi, lo) pairs go through
+// the wave's 128 words of LDS to the A-fragment layout. Every lane reads the
+// row's fragment, so all 32 rows of A hold it; only row 0 of the result is
+// used. Two lanes splitting 64 values each took about 250 VALU instructions
+// per chunk, 0.3 us of a GEMV's 4.5 to 7.
+__device__ __forceinline__ float dpp_max(float v) {
+    auto step = [&](auto ctrl) {
+        v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xF, 0xF,
+                                                                false)));
+    };
+    step(std::integral_constant<int, 0xB1>{});    // (the steps of wave_sum)
+    step(std::integral_constant<int, 0x4E>{});
+    step(std::integral_constant<int, 0x141>{});
+    step(std::integral_constant<int, 0x140>{});
+    v = fmaxf(v, __shfl_xor(v, 16, 64));
+    return fmaxf(v, __shfl_xor(v, 32, 64));
+}
+template <int I>
+__device__ __forceinline__ float quad_lane(float v) {   // lane I of the lane's four
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), I * 0x55, 0xF, 0xF, false));
+}
+template <bool MINS>
+__device__ __forceinline__ void split_row(float2 v, int lane, int hh, uint32_t *lds, XChunk &o) {
+    const int sh = chunk_shift(dpp_max(fmaxf(fabsf(v.x), fabsf(v.y))));
+    o.p = ldexpf(1.0f, -sh);
+    const float x0 = ldexpf(v.x, sh), x1 = ldexpf(v.y, sh);
+    const half2v h = {(_Float16)x0, (_Float16)x1};
+    uint32_t hw;
+    __builtin_memcpy(&hw, &h, 4);
+    lds[lane] = hw;
+    lds[64 + lane] = lo_pair(hw, x0, x1);
+    if constexpr (MINS) {
+        // lanes 4t .. 4t+3 hold the eight values of half-step t >> 1, half t & 1
+        float s = 0.0f + quad_lane<0>(x0);
+        s += quad_lane<0>(x1);
+        s += quad_lane<1>(x0);
+        s += quad_lane<1>(x1);
+        s += quad_lane<2>(x0);
+        s += quad_lane<2>(x1);
+        s += quad_lane<3>(x0);
+        s += quad_lane<3>(x1);
+#pragma unroll
+        for (int u = 0; u < HSTEPS; u++) o.s8[u] = __shfl(s, 4 * (2 * u + hh), 64);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int u = 0; u < HSTEPS; u++) {
+        o.h[u] = *(const half8 *)(lds + 8 * u + 4 * hh);
+        o.l[u] = *(const half8 *)(lds + 64 + 8 * u + 4 * hh);
+    }
+}
+// the lane's two elements of chunk c of x (zero past K); VEC as load_chunk
+template <bool VEC>
+__device__ __forceinline__ float2 load_row2(const float *__restrict__ x, int K, int c, int lane) {
+    const int e = 128 * c + 2 * lane;
+    if constexpr (VEC) return e < K ? ld2(x + e) : float2{0.0f, 0.0f};
+    return float2{e < K ? x[e] : 0.0f, e + 1 < K ? x[e + 1] : 0.0f};
 }
 
 // The epilogue operands of a one-row product (the decoder's), loaded when the
@@ -690,12 +757,13 @@ __device__ __forceinline__ void gemv_store(const DevW &W, int n, int M, int hh, 
 template <int QT, int NW, int WNG, bool VEC, bool PRO, int NE>
 __device__ __forceinline__ void gemv_body(const DevW &W, const float *__restrict__ x, int M, float *y,
                                           const GEpi &ep, const GPro &pro, int bx) {
-    extern __shared__ float part[];  // [Kc][WNG][8][64] chunk results, pf [Kc][16], prologue row [Kp]
+    // [Kc][WNG][NE][64] chunk results, pf [Kc][16], M = 1: the row's (hi, lo) pairs [Kp]
+    extern __shared__ __align__(16) float part[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int hh = lane >> 5, col = lane & 31;
     const int Kc = W.Kp / 128;
-    float *pf = part + (size_t)Kc * WNG * 8 * 64;
-    float *xs = pf + (size_t)Kc * 16;
+    float *pf = part + (size_t)Kc * WNG * NE * 64;
+    uint32_t *xs = (uint32_t *)(pf + (size_t)Kc * 16);
     int gn[WNG];
 #pragma unroll
     for (int j = 0; j < WNG; j++) gn[j] = bx * WNG + j;
@@ -715,26 +783,17 @@ __device__ __forceinline__ void gemv_body(const DevW &W, const float *__restrict
         // loads complete in issue order, so the split can start as soon as
         // x lands, while the weight bytes are still on their way
         float xv[HSTEPS][8];
-        if constexpr (!PRO) load_chunk<VEC>(x, M, W.k, col, c, hh, xv);
-        else wave_row_issue(pro, W.k, c, lane, wr);
+        float2 x2;
+        if constexpr (PRO) wave_row_issue(pro, W.k, c, lane, wr);
+        else if constexpr (NE == 1) x2 = load_row2<VEC>(x, W.k, c, lane);
+        else load_chunk<VEC>(x, M, W.k, col, c, hh, xv);
         __builtin_amdgcn_sched_barrier(0);
         load(c);
         __builtin_amdgcn_sched_barrier(0);
         XChunk xc;
-        if constexpr (PRO) {
-            // M = 1: row 0, formed by this wave; its 128 values go to the
-            // A-fragment layout (lanes 0 and 32) through the chunk's own LDS
-            const float2 val = wave_row_values(pro, W.k, c, lane, wr);
-            *(float2 *)(xs + 128 * c + 2 * lane) = val;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            float v[HSTEPS][8];
-#pragma unroll
-            for (int u = 0; u < HSTEPS; u++)
-#pragma unroll
-                for (int j = 0; j < 8; j++) v[u][j] = col == 0 ? xs[128 * c + 16 * u + 8 * hh + j] : 0.0f;
-            split_vals(v, xc);
+        if constexpr (NE == 1) {
+            if constexpr (PRO) x2 = wave_row_values(pro, W.k, c, lane, wr);
+            split_row<Fmt<QT>::MINS>(x2, lane, hh, xs + 128 * c, xc);
         } else {
             split_vals(xv, xc);
         }
@@ -762,7 +821,7 @@ __device__ __forceinline__ void gemv_body(const DevW &W, const float *__restrict
 #pragma unroll
         for (int j = 0; j < WNG; j++)
 #pragma unroll
-            for (int e = 0; e < NE; e++) part[((c * WNG + j) * 8 + e) * 64 + lane] = acc[0][j][e];
+            for (int e = 0; e < NE; e++) part[((c * WNG + j) * NE + e) * 64 + lane] = acc[0][j][e];
     }
     __syncthreads();
     for (int j = wave; j < WNG; j += NW) {
@@ -772,7 +831,7 @@ __device__ __forceinline__ void gemv_body(const DevW &W, const float *__restrict
         for (int c = 0; c < Kc; c++)
 #pragma unroll
             for (int e = 0; e < NE; e++)
-                total[e] = __builtin_fmaf(pf[c * 16 + drow(e, hh)], part[((c * WNG + j) * 8 + e) * 64 + lane], total[e]);
+                total[e] = __builtin_fmaf(pf[c * 16 + drow(e, hh)], part[((c * WNG + j) * NE + e) * 64 + lane], total[e]);
         gemv_store<QT, NE>(W, 32 * gn[j] + col, M, hh, total, ep, pre, y);
     }
 }
@@ -796,14 +855,21 @@ __global__ __launch_bounds__(NW * 64) void k_gemv_part(DevW W, const float *__re
     BK<QT, 1> bk[KSTEPS];
     // x first: its loads complete before the weights' (issue order)
     float xv[HSTEPS][8];
-    load_chunk<VEC>(x, M, W.k, col, c, hh, xv);
+    float2 x2;
+    if constexpr (NE == 1) x2 = load_row2<VEC>(x, W.k, c, lane);
+    else load_chunk<VEC>(x, M, W.k, col, c, hh, xv);
     __builtin_amdgcn_sched_barrier(0);
     load_bh<QT, 1>(W, Kc, gn, c, lane, hd);
 #pragma unroll
     for (int s = 0; s < KSTEPS; s++) load_bk<QT, 1>(W, Kc, gn, c, s, lane, bk[s]);
     __builtin_amdgcn_sched_barrier(0);
     XChunk xc;
-    split_vals(xv, xc);
+    if constexpr (NE == 1) {
+        __shared__ __align__(16) uint32_t xs[NW][128];
+        split_row<Fmt<QT>::MINS>(x2, lane, hh, xs[wave], xc);
+    } else {
+        split_vals(xv, xc);
+    }
     if (bx == 0 && hh == 0 && col < 16) pfg[c * 16 + col] = xc.p;
     f16v acc[1][1];
     acc[0][0] = zero16();
@@ -1620,7 +1686,9 @@ template <int QT, int NW, int WNG, bool VEC, bool PRO>
 static hipError_t launch_gemv1(const GJobs &J, const float *x, int M, const GPro &pro, hipStream_t st) {
     const DevW &W = J.W[0];
     const int Kc = W.Kp / 128;
-    const size_t lds = ((size_t)Kc * WNG * 8 * 64 + (size_t)Kc * 16 + (PRO ? (size_t)W.Kp : 0)) * sizeof(float);
+    // accumulator elements the M rows need (rows drow(e, hh) < M)
+    const int ne = M == 1 ? 1 : (M <= 8 ? 4 : 8);
+    const size_t lds = ((size_t)Kc * WNG * ne * 64 + (size_t)Kc * 16 + (M == 1 ? (size_t)W.Kp : 0)) * sizeof(float);
     // set once per instantiation; a function-local static's initialisation is
     // thread-safe, so concurrent first calls wait for the one that runs it
     static const hipError_t attr = []() {
@@ -1638,11 +1706,10 @@ static hipError_t launch_gemv1(const GJobs &J, const float *x, int M, const GPro
         hipLaunchKernelGGL((k_gemv_jobs<QT, NW, WNG>), dim3(W.Np / 32 / WNG * J.n), dim3(NW * 64), lds, st, J, pro);
     } else {
         if (J.n != 1) return hipErrorInvalidValue;
-        // accumulator elements the M rows need (rows drow(e, hh) < M)
-        if (M == 1)
+        if (ne == 1)
             hipLaunchKernelGGL((k_gemv<QT, NW, WNG, VEC, 1>), dim3(W.Np / 32 / WNG), dim3(NW * 64), lds, st, W, x, M,
                                J.y[0], J.ep[0]);
-        else if (M <= 8)
+        else if (ne == 4)
             hipLaunchKernelGGL((k_gemv<QT, NW, WNG, VEC, 4>), dim3(W.Np / 32 / WNG), dim3(NW * 64), lds, st, W, x, M,
                                J.y[0], J.ep[0]);
         else

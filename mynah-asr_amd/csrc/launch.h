@@ -41,6 +41,7 @@ enum { GPRO_NONE = 0, GPRO_LN = 1, GPRO_COMB = 2 };
 struct GPro {
     int kind;
     const float *x, *w, *b;
+    double rk;   // GPRO_LN: 1 / K
     const float *opart, *ml;
     const int *st;
     int n_fixed, nsplit, H;

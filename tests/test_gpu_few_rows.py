@@ -100,3 +100,33 @@ def test_ffn_hand_off(gpu, q1, q2):
     finally:
         w1.close()
         w2.close()
+
+
+@pytest.mark.parametrize("qt", FMTS, ids=lambda q: M.NAMES[q])
+def test_one_row_carries_the_larger_products_bits(gpu, qt):
+    """One row is split by its whole wave: one and several chunks per wave, two
+    column groups per workgroup, the split over workgroups, and the largest K."""
+    import torch
+    for n, k in [(1000, 1024), (8200, 512), (130, 1280), (1024, 4096), (2100, 4096), (96, 8192)]:
+        say("one row", M.NAMES[qt], n, k)
+        _check(gpu, qt, n, k, 40, [1])
+    # rows off the 16-byte grid, whose elements are loaded one by one
+    n, k = 200, 768
+    dw = M.DeviceWeight(gpu, M.Weight.make(gpu, qt, gpu.randn(3, 0.02, (n, k))))
+    x = torch.from_numpy(gpu.randn(4, 1.0, (1 + 40 * k,))).cuda()
+    y = torch.empty((40, n), device="cuda")
+    y1 = torch.empty((1, n), device="cuda")
+    torch.cuda.synchronize()
+    try:
+        dw.gemm(x.data_ptr() + 4, y.data_ptr(), 40, 0)
+        dw.gemm(x.data_ptr() + 4, y1.data_ptr(), 1, 0)
+        torch.cuda.synchronize()
+        assert np.array_equal(_bits(y1), _bits(y)[:1])
+    finally:
+        dw.close()
+
+
+@pytest.mark.parametrize("k", [1, 37, 129, 1027])
+def test_one_row_of_odd_length(gpu, k):
+    say("one row, K", k)
+    _check(gpu, M.F32, 70, k, 40, [1])
