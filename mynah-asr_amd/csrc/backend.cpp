@@ -1084,15 +1084,43 @@ int subsampling_dev(Ctx *c, const mynah_asr_hip_subsampling *ss, const float *fe
         if (e != hipSuccess) return fail("subsampling launch failed", hipGetErrorString(e)); \
     } while (0)
     NumScope sc(MYNAH_ASR_HIP_EXACT);
-    SS_TRY(mh_launch_transpose_taps(ss->conv_in_w, w0, C, 9, st));
-    SS_TRY(mh_launch_transpose_taps(ss->dw_w[0], w1, C, 9, st));
-    SS_TRY(mh_launch_transpose_taps(ss->dw_w[1], w2, C, 9, st));
-    SS_TRY(mh_launch_conv_in_dw(feats, w0, ss->conv_in_b, w1, ss->dw_b[0], B, nseq, T, F, C, cz, st));
-    if (gemm_dev(c, ss->pw_w[0], B, A, nseq * T2 * F2, 0, st)) return -1;
-    SS_TRY(mh_launch_dw_s2(A, ss->pw_b[0], w2, ss->dw_b[1], B, nseq, T2, F2, C, cz, st));
-    if (gemm_dev(c, ss->pw_w[1], B, A, nseq * T3 * F3, 0, st)) return -1;
-    SS_TRY(mh_launch_flatten(A, ss->pw_b[1], B, (size_t)nseq * T3, F3, C, st));
-    if (gemm_dev(c, ss->lin_w, B, out, nseq * T3, 0, st)) return -1;
+    // each product's input is written prepared by the step in front of it where
+    // the product reads it so (f32 weights and the formats without row sums, on
+    // the EXACT GEMM path), else as f32 rows: the same bits
+    const int M2 = nseq * T2 * F2, M3 = nseq * T3 * F3, M4 = nseq * T3;
+    const auto preps = [&](const mynah_asr_hip_weight *W, int M, int K) {
+        return C % 256 == 0 && enc_fused() && !mh_use_gemv(W->dw, M) && !wants_xsum(W->qtype) && W->dw.Kp == K;
+    };
+    const auto get_prep = [&](int M, int K) {
+        PrepBuf &P = c->pa;
+        P.src = nullptr;
+        size_t bs[3];
+        prep_sizes(0, mh_mpad(M), K, bs);
+        if (!P.xp.get(bs[0]) || !P.xs16.get(bs[1]) || !P.xpf.get(bs[2])) return fail("workspace allocation failed");
+        P.T = M, P.Kp = K, P.xsum = 0, P.i8 = 0;
+        return 0;
+    };
+    const bool p0 = preps(ss->pw_w[0], M2, C), p1 = preps(ss->pw_w[1], M3, C),
+               p2 = preps(ss->lin_w, M4, C * F3) && mh_flatten_prep_supported(F3, C);
+    const auto xp = [&](bool p) { return p ? (uint8_t *)c->pa.xp.p : nullptr; };
+    const auto xpf = [&](bool p) { return p ? (float *)c->pa.xpf.p : nullptr; };
+    const auto product = [&](bool p, const mynah_asr_hip_weight *W, float *y, int M) {
+        return p ? run_prepped(c, W, y, M, 0, nullptr, st) : gemm_dev(c, W, B, y, M, 0, st);
+    };
+    SS_TRY(mh_launch_transpose_taps(ss->conv_in_w, ss->dw_w[0], ss->dw_w[1], w0, C, st));
+    if (p0 && get_prep(M2, C)) return -1;
+    SS_TRY(mh_launch_conv_in_dw(feats, w0, ss->conv_in_b, w1, ss->dw_b[0], B, nseq, T, F, C, cz, xp(p0), xpf(p0), st));
+    if (product(p0, ss->pw_w[0], A, M2)) return -1;
+    if (p1 && get_prep(M3, C)) return -1;
+    SS_TRY(mh_launch_dw_s2(A, ss->pw_b[0], w2, ss->dw_b[1], B, nseq, T2, F2, C, cz, xp(p1), xpf(p1), st));
+    if (product(p1, ss->pw_w[1], A, M3)) return -1;
+    if (p2) {
+        if (get_prep(M4, C * F3)) return -1;
+        SS_TRY(mh_launch_flatten_prep(A, ss->pw_b[1], (size_t)M4, F3, C, xp(true), xpf(true), st));
+    } else {
+        SS_TRY(mh_launch_flatten(A, ss->pw_b[1], B, (size_t)M4, F3, C, st));
+    }
+    if (product(p2, ss->lin_w, out, M4)) return -1;
     SS_TRY(mh_launch_bias_scale(out, ss->lin_b, (size_t)nseq * T3, ss->d_model, xscale, st));
 #undef SS_TRY
     return 0;

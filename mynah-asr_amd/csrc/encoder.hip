@@ -97,6 +97,35 @@ __device__ __forceinline__ void add_ln_row(float *xr, const float *__restrict__ 
     }
 }
 
+// Four channels per lane of row m of an EXACT product's prepared input: the
+// lane's half wave holds chunk c, lane l of it elements 4l .. 4l+3. The
+// arithmetic of split_chunk; 8-byte stores, which the L2 joins with those of the
+// neighbouring rows (the wave's next ones).
+__device__ __forceinline__ void prep_store4(float4 v, int lane, size_t m, int c, int Kc, uint8_t *__restrict__ xp,
+                                            float *__restrict__ xpf) {
+    const int l32 = lane & 31, hu = l32 >> 2, hh = (l32 >> 1) & 1;
+    float a = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+    auto step = [&](auto ctrl) {   // (within each row of 16 lanes, symmetrically)
+        a = fmaxf(a, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), decltype(ctrl)::value, 0xF, 0xF,
+                                                                false)));
+    };
+    step(std::integral_constant<int, 0xB1>{});    // quad_perm [1,0,3,2]
+    step(std::integral_constant<int, 0x4E>{});    // quad_perm [2,3,0,1]
+    step(std::integral_constant<int, 0x141>{});   // row_half_mirror
+    step(std::integral_constant<int, 0x140>{});   // row_mirror
+    a = fmaxf(a, __shfl_xor(a, 16, 64));
+    const int sh = chunk_shift(a);
+    const float xs[4] = {ldexpf(v.x, sh), ldexpf(v.y, sh), ldexpf(v.z, sh), ldexpf(v.w, sh)};
+    const half4v h = {(_Float16)xs[0], (_Float16)xs[1], (_Float16)xs[2], (_Float16)xs[3]};
+    uint2 hw;
+    __builtin_memcpy(&hw, &h, 8);
+    const uint2 lw = {lo_pair(hw.x, xs[0], xs[1]), lo_pair(hw.y, xs[2], xs[3])};
+    uint8_t *o = xp + ((((m >> 5) * Kc + c) * 8 + hu) * 2 * 64 + (m & 31) + 32 * hh) * 16 + 8 * (lane & 1);
+    *(uint2 *)o = hw;
+    *(uint2 *)(o + 64 * 16) = lw;
+    if (l32 == 0) xpf[((m >> 5) * Kc + c) * 32 + (m & 31)] = ldexpf(1.0f, -sh);
+}
+
 // out = LN(x += alpha res), one wave per row. out may be x.
 template <int V4>
 __global__ __launch_bounds__(256) void k_add_ln(float *x, const float *__restrict__ res, float alpha,
@@ -440,21 +469,55 @@ __global__ __launch_bounds__(256) void k_dwconv_tile(const float *__restrict__ g
 // y's [T1, F1] reads zero (the depthwise conv's pad), and a mel sample
 // outside [T, F] reads zero (the first conv's pad).
 //
-// One wave per output row (s, to), its lanes over the channels 4 at a time,
-// sliding along fo: the 3 x 3 window of y a depthwise output reads stays in
-// registers, and each step forms y's two new columns (y column 2 of one
-// step is column 0 of the next). The mel samples are wave-uniform and read
-// through the scalar cache; each lane holds its channels' 2 x 9 taps.
+// One wave per output row (s, to) and run of FS columns fo, its lanes over the
+// channels 4 at a time, sliding along fo: the 3 x 3 window of y a depthwise
+// output reads stays in registers, and each step forms y's two new columns (y
+// column 2 of one step is column 0 of the next). Each lane holds its channels'
+// 2 x 9 taps. The 7 mel rows the wave reads lie in its own LDS with the pads as
+// zeros, column k at word k + 1, so that a step reads its four new columns of a
+// row as one 16-byte broadcast (the fifth is the last step's last). Loads of
+// single mel samples behind their bounds, through the scalar cache, made a step
+// a chain of about 30 waits: 138 us at 4 segments of 6000 frames (6000 rows of
+// 20 columns, 256 channels), where its fmas take 55.
+// PREP: the rows are written as the pointwise product's prepared input (waves
+// past the rows write the 64-row padding) instead of as f32.
 // Weights tap-major, w0[j][C] and w1[j][C].
+constexpr int CI_FS = 32;   // columns per wave at most
+template <bool PREP>
 __global__ __launch_bounds__(256) void k_conv_in_dw(const float *__restrict__ x, const float *__restrict__ w0,
                                                     const float *__restrict__ b0, const float *__restrict__ w1,
                                                     const float *__restrict__ b1, float *__restrict__ out, int nseq,
-                                                    int T, int F, int T1, int F1, int To, int Fo, int C, int pl) {
-    const int wrow = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6));
-    if (wrow >= nseq * To) return;
-    const int lane = threadIdx.x & 63;
-    const int to = wrow % To, s = wrow / To;
+                                                    int T, int F, int T1, int F1, int To, int Fo, int C, int pl,
+                                                    int FS, int parts, uint8_t *__restrict__ xp,
+                                                    float *__restrict__ xpf) {
+    constexpr int WC = 4 * CI_FS + 4;
+    __shared__ __align__(16) float win[4][7][WC];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + wave), wrow = wid / parts;
+    if (wrow >= nseq * To) {
+        if constexpr (PREP) {
+            const size_t M = (size_t)nseq * To * Fo, m = M + (wid - nseq * To * parts);
+            if (m < (M + 63) / 64 * 64)
+                for (int c = 4 * lane; c < C; c += 256)
+                    prep_store4(float4{0.f, 0.f, 0.f, 0.f}, lane, m, c >> 7, C / 128, xp, xpf);
+        }
+        return;   // (no workgroup barrier follows)
+    }
+    const int to = wrow % To, s = wrow / To, f0 = (wid - wrow * parts) * FS, f9 = min(f0 + FS, Fo);
     const float *xs = x + (size_t)s * T * F;
+    // window column k: mel f = 4 f0 - 3 pl + k; window row j: mel t = 4 to - 3 pl + j
+    const int cols = 4 * (f9 - f0) + 4;
+    for (int k = lane; k < cols; k += 64) {
+        const int f = 4 * f0 - 3 * pl + k - 1;
+#pragma unroll
+        for (int j = 0; j < 7; j++) {
+            const int t = 4 * to - 3 * pl + j;
+            win[wave][j][k] = t >= 0 && t < T && f >= 0 && f < F ? xs[(size_t)t * F + f] : 0.0f;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     for (int c = 4 * lane; c < C; c += 256) {
         float4 wa[9], wb[9];
 #pragma unroll
@@ -463,38 +526,51 @@ __global__ __launch_bounds__(256) void k_conv_in_dw(const float *__restrict__ x,
             wb[j] = *(const float4 *)(w1 + (size_t)j * C + c);
         }
         const float4 bb0 = *(const float4 *)(b0 + c), bb1 = *(const float4 *)(b1 + c);
-        // y at (t1 = 2 to - pl + r, f1): relu(b0 + conv_in), zero outside [T1, F1]
-        auto yat = [&](int r, int f1) {
+        float mel[7][5];   // columns 4i+2 .. 4i+6 of step i
+        // y at (t1 = 2 to - pl + r, f1): relu(b0 + conv_in) over the mel columns
+        // from m0 of the step, zero outside [T1, F1]
+        auto yat = [&](int r, int f1, int m0) {
             const int t1 = 2 * to - pl + r;
-            float4 y = {0.f, 0.f, 0.f, 0.f};
+            float4 ci = {0.f, 0.f, 0.f, 0.f};
             if (t1 >= 0 && t1 < T1 && f1 >= 0 && f1 < F1) {
-                float4 ci = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int dt = 0; dt < 3; dt++)
 #pragma unroll
                     for (int df = 0; df < 3; df++) {
-                        const int t = 2 * t1 - pl + dt, f = 2 * f1 - pl + df;
-                        const float v = t >= 0 && t < T && f >= 0 && f < F ? xs[(size_t)t * F + f] : 0.0f;
+                        const float v = mel[2 * r + dt][m0 + df];
                         const float4 wv = wa[3 * dt + df];
                         ci.x = fmaf(wv.x, v, ci.x);
                         ci.y = fmaf(wv.y, v, ci.y);
                         ci.z = fmaf(wv.z, v, ci.z);
                         ci.w = fmaf(wv.w, v, ci.w);
                     }
-                y = float4{fmaxf(ci.x + bb0.x, 0.0f), fmaxf(ci.y + bb0.y, 0.0f), fmaxf(ci.z + bb0.z, 0.0f),
-                           fmaxf(ci.w + bb0.w, 0.0f)};
+                ci = float4{fmaxf(ci.x + bb0.x, 0.0f), fmaxf(ci.y + bb0.y, 0.0f), fmaxf(ci.z + bb0.z, 0.0f),
+                            fmaxf(ci.w + bb0.w, 0.0f)};
             }
-            return y;
+            return ci;
         };
         float4 yw[3][3];
 #pragma unroll
-        for (int r = 0; r < 3; r++) yw[r][2] = yat(r, -pl);
-        for (int fo = 0; fo < Fo; fo++) {
+        for (int j = 0; j < 7; j++) {   // columns 0, 1, 2
+            const float4 a = *(const float4 *)&win[wave][j][0];
+            mel[j][0] = a.y, mel[j][1] = a.z, mel[j][2] = a.w;
+        }
+#pragma unroll
+        for (int r = 0; r < 3; r++) yw[r][2] = yat(r, 2 * f0 - pl, 0);
+#pragma unroll
+        for (int j = 0; j < 7; j++) mel[j][4] = mel[j][2];
+        for (int fo = f0; fo < f9; fo++) {
+#pragma unroll
+            for (int j = 0; j < 7; j++) {
+                mel[j][0] = mel[j][4];
+                const float4 a = *(const float4 *)&win[wave][j][4 * (fo - f0) + 4];
+                mel[j][1] = a.x, mel[j][2] = a.y, mel[j][3] = a.z, mel[j][4] = a.w;
+            }
 #pragma unroll
             for (int r = 0; r < 3; r++) {
                 yw[r][0] = yw[r][2];
-                yw[r][1] = yat(r, 2 * fo - pl + 1);
-                yw[r][2] = yat(r, 2 * fo - pl + 2);
+                yw[r][1] = yat(r, 2 * fo - pl + 1, 0);
+                yw[r][2] = yat(r, 2 * fo - pl + 2, 2);
             }
             float4 acc = {wb[0].x * yw[0][0].x, wb[0].y * yw[0][0].y, wb[0].z * yw[0][0].z, wb[0].w * yw[0][0].w};
 #pragma unroll
@@ -505,8 +581,10 @@ __global__ __launch_bounds__(256) void k_conv_in_dw(const float *__restrict__ x,
                 acc.z = fmaf(wv.z, y.z, acc.z);
                 acc.w = fmaf(wv.w, y.w, acc.w);
             }
-            *(float4 *)(out + ((size_t)wrow * Fo + fo) * C + c) =
-                float4{bb1.x + acc.x, bb1.y + acc.y, bb1.z + acc.z, bb1.w + acc.w};
+            acc = float4{bb1.x + acc.x, bb1.y + acc.y, bb1.z + acc.z, bb1.w + acc.w};
+            const size_t m = (size_t)wrow * Fo + fo;
+            if constexpr (PREP) prep_store4(acc, lane, m, c >> 7, C / 128, xp, xpf);
+            else *(float4 *)(out + m * C + c) = acc;
         }
     }
 }
@@ -515,15 +593,22 @@ __global__ __launch_bounds__(256) void k_conv_in_dw(const float *__restrict__ x,
 // in the reference's term order (the nine products summed left to right,
 // subsampling.c:96-98); with pb, each input value is relu(in + pb[c]) first.
 // The weights tap-major, wt[j][c].
+// PREP (C of 256: a wave is 256 channels of one row): as the next product's
+// prepared input, with its padding rows.
+template <bool PREP>
 __global__ __launch_bounds__(256) void k_dw_s2(const float *__restrict__ in, const float *__restrict__ pb,
                                                const float *__restrict__ wt, const float *__restrict__ b,
                                                float *__restrict__ out, int nseq, int T, int F, int To, int Fo,
-                                               int C, int pl) {
+                                               int C, int pl, uint8_t *__restrict__ xp, float *__restrict__ xpf) {
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const int C4 = C / 4;
-    if (idx >= (size_t)nseq * To * Fo * C4) return;
-    const size_t row = idx / C4;
+    const int C4 = C / 4, lane = threadIdx.x & 63;
+    const size_t row = idx / C4, rows = (size_t)nseq * To * Fo;
     const int c = 4 * (int)(idx - row * C4);
+    if (row >= rows) {
+        if constexpr (PREP)
+            if (row < (rows + 63) / 64 * 64) prep_store4(float4{0.f, 0.f, 0.f, 0.f}, lane, row, c >> 7, C / 128, xp, xpf);
+        return;
+    }
     const int fo = (int)(row % Fo), to = (int)((row / Fo) % To), s = (int)(row / ((size_t)Fo * To));
     const float *is = in + (size_t)s * T * F * C;
     const float4 pbv = pb ? *(const float4 *)(pb + c) : float4{0.f, 0.f, 0.f, 0.f};
@@ -556,7 +641,9 @@ __global__ __launch_bounds__(256) void k_dw_s2(const float *__restrict__ in, con
         acc.w = fmaf(wv.w, v[j].w, acc.w);
     }
     const float4 bb = *(const float4 *)(b + c);
-    *(float4 *)(out + row * C + c) = float4{bb.x + acc.x, bb.y + acc.y, bb.z + acc.z, bb.w + acc.w};
+    acc = float4{bb.x + acc.x, bb.y + acc.y, bb.z + acc.z, bb.w + acc.w};
+    if constexpr (PREP) prep_store4(acc, lane, row, c >> 7, C / 128, xp, xpf);
+    else *(float4 *)(out + row * C + c) = acc;
 }
 
 // flat[s * To + t][c * Fo + f] = relu(in[s][t][f][c] + pb[c]); thread = one
@@ -572,13 +659,44 @@ __global__ __launch_bounds__(256) void k_flatten(const float *__restrict__ in, c
     flat[idx] = v < 0.0f ? 0.0f : v;
 }
 
-// wt[j][c] = w[c][j] for w [C][k]: the per-channel taps tap-major
-__global__ __launch_bounds__(256) void k_transpose(const float *__restrict__ w, float *__restrict__ wt, int C,
-                                                   int k) {
-    const int idx = blockIdx.x * 256 + threadIdx.x;
-    if (idx >= C * k) return;
+// The same as the linear's prepared input (C of 256): a workgroup takes one row,
+// read along c into LDS and written along c * Fo + f by half waves of one
+// chunk each; the workgroups past the rows write the padding.
+__global__ __launch_bounds__(256) void k_flatten_prep(const float *__restrict__ in, const float *__restrict__ pb,
+                                                      int rows, int Fo, int C, uint8_t *__restrict__ xp,
+                                                      float *__restrict__ xpf) {
+    extern __shared__ float row[];   // [Fo][C + 1]
+    const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, CF = C * Fo;
+    if (r < rows) {
+        for (int i = 4 * tid; i < CF; i += 1024) {
+            const int f = i / C, c = i - f * C;
+            const float4 a = *(const float4 *)(in + (size_t)r * CF + i);
+            const float v[4] = {a.x + pb[c], a.y + pb[c + 1], a.z + pb[c + 2], a.w + pb[c + 3]};
+#pragma unroll
+            for (int j = 0; j < 4; j++) row[f * (C + 1) + c + j] = v[j] < 0.0f ? 0.0f : v[j];
+        }
+        __syncthreads();
+    }
+    for (int j = 4 * tid; j < CF; j += 1024) {   // (CF of 256: whole waves)
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int c = (j + u) / Fo, f = j + u - c * Fo;
+            v[u] = r < rows ? row[f * (C + 1) + c] : 0.0f;
+        }
+        prep_store4(float4{v[0], v[1], v[2], v[3]}, lane, (size_t)r, j >> 7, CF / 128, xp, xpf);
+    }
+}
+
+// wt[z][j][c] = w_z[c][j] for w_z [C][9]: the per-channel taps of the three
+// 3 x 3 convs tap-major, in one launch
+__global__ __launch_bounds__(256) void k_transpose(const float *__restrict__ wa, const float *__restrict__ wb,
+                                                   const float *__restrict__ wc, float *__restrict__ wt, int C) {
+    const int idx = blockIdx.x * 256 + threadIdx.x, z = blockIdx.y;
+    if (idx >= C * 9) return;
     const int j = idx / C, c = idx - j * C;
-    wt[idx] = w[(size_t)c * k + j];
+    const float *w = z == 0 ? wa : (z == 1 ? wb : wc);
+    wt[(size_t)z * C * 9 + idx] = w[(size_t)c * 9 + j];
 }
 
 // y[r][i] = (y[r][i] + b[i]) * scale (the subsampling's linear bias, then
@@ -716,27 +834,56 @@ int mh_ss_out_len(int n, int causal) {
 }
 
 hipError_t mh_launch_conv_in_dw(const float *x, const float *w0, const float *b0, const float *w1, const float *b1,
-                                float *out, int nseq, int T, int F, int C, int causal, hipStream_t st) {
-    if (C % 4) return hipErrorInvalidValue;
+                                float *out, int nseq, int T, int F, int C, int causal, uint8_t *xp, float *xpf,
+                                hipStream_t st) {
+    if (C % 4 || (xp && C % 256)) return hipErrorInvalidValue;
     const int T1 = mh_ss_out_len(T, causal), F1 = mh_ss_out_len(F, causal);
-    const int To = mh_ss_out_len(T1, causal), Fo = mh_ss_out_len(F1, causal);
+    const int To = mh_ss_out_len(T1, causal), Fo = mh_ss_out_len(F1, causal), pl = causal ? 2 : 1;
     if (T1 <= 0 || F1 <= 0 || To <= 0 || Fo <= 0) return hipSuccess;
-    const size_t rows = (size_t)nseq * To;   // one wave per output row (s, to)
+    const size_t rows = (size_t)nseq * To;   // output rows (s, to)
     if (!rows) return hipSuccess;
-    if (rows > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_conv_in_dw, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, x, w0, b0, w1, b1, out, nseq,
-                       T, F, T1, F1, To, Fo, C, causal ? 2 : 1);
+    // A wave takes whole rows while they fill the chip (1024 SIMDs, 3 waves
+    // each), else part of one: a part forms one column of y more
+    int FS = Fo < CI_FS ? Fo : CI_FS;
+    while (FS > 4 && rows * ((Fo + FS - 1) / FS) < 2048) FS = (FS + 1) / 2;
+    const int parts = (Fo + FS - 1) / FS;
+    if (rows * parts > 0x7fffff00) return hipErrorInvalidValue;
+    const size_t M = rows * Fo, waves = rows * parts + (xp ? (M + 63) / 64 * 64 - M : 0);
+    const dim3 grid((unsigned)((waves + 3) / 4));
+    if (xp)
+        hipLaunchKernelGGL(k_conv_in_dw<true>, grid, dim3(256), 0, st, x, w0, b0, w1, b1, out, nseq, T, F, T1, F1, To,
+                           Fo, C, pl, FS, parts, xp, xpf);
+    else
+        hipLaunchKernelGGL(k_conv_in_dw<false>, grid, dim3(256), 0, st, x, w0, b0, w1, b1, out, nseq, T, F, T1, F1, To,
+                           Fo, C, pl, FS, parts, xp, xpf);
     return hipGetLastError();
 }
 
 hipError_t mh_launch_dw_s2(const float *in, const float *pb, const float *w, const float *b, float *out, int nseq,
-                           int T, int F, int C, int causal, hipStream_t st) {
-    if (C % 4) return hipErrorInvalidValue;
-    const int To = mh_ss_out_len(T, causal), Fo = mh_ss_out_len(F, causal);
-    const size_t n = (size_t)nseq * To * Fo * (C / 4);
-    if (!n) return hipSuccess;
-    hipLaunchKernelGGL(k_dw_s2, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, in, pb, w, b, out, nseq, T, F, To,
-                       Fo, C, causal ? 2 : 1);
+                           int T, int F, int C, int causal, uint8_t *xp, float *xpf, hipStream_t st) {
+    if (C % 4 || (xp && C % 256)) return hipErrorInvalidValue;
+    const int To = mh_ss_out_len(T, causal), Fo = mh_ss_out_len(F, causal), pl = causal ? 2 : 1;
+    const size_t rows = (size_t)nseq * To * Fo;
+    if (!rows) return hipSuccess;
+    const size_t n = (xp ? (rows + 63) / 64 * 64 : rows) * (C / 4);
+    const dim3 grid((unsigned)((n + 255) / 256));
+    if (xp)
+        hipLaunchKernelGGL(k_dw_s2<true>, grid, dim3(256), 0, st, in, pb, w, b, out, nseq, T, F, To, Fo, C, pl, xp, xpf);
+    else
+        hipLaunchKernelGGL(k_dw_s2<false>, grid, dim3(256), 0, st, in, pb, w, b, out, nseq, T, F, To, Fo, C, pl, xp,
+                           xpf);
+    return hipGetLastError();
+}
+
+// the row k_flatten_prep holds in LDS, with its padding
+bool mh_flatten_prep_supported(int Fo, int C) { return C % 256 == 0 && (size_t)Fo * (C + 1) * 4 <= 65536; }
+
+hipError_t mh_launch_flatten_prep(const float *in, const float *pb, size_t rows, int Fo, int C, uint8_t *xp,
+                                  float *xpf, hipStream_t st) {
+    if (!mh_flatten_prep_supported(Fo, C) || rows > 0x7fffff00) return hipErrorInvalidValue;
+    if (!rows) return hipSuccess;
+    hipLaunchKernelGGL(k_flatten_prep, dim3((unsigned)((rows + 63) / 64 * 64)), dim3(256),
+                       (size_t)Fo * (C + 1) * sizeof(float), st, in, pb, (int)rows, Fo, C, xp, xpf);
     return hipGetLastError();
 }
 
@@ -755,8 +902,9 @@ hipError_t mh_launch_bias_scale(float *y, const float *b, size_t rows, int d, fl
     return hipGetLastError();
 }
 
-hipError_t mh_launch_transpose_taps(const float *w, float *wt, int C, int k, hipStream_t st) {
-    if (C * k <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_transpose, dim3((C * k + 255) / 256), dim3(256), 0, st, w, wt, C, k);
+hipError_t mh_launch_transpose_taps(const float *wa, const float *wb, const float *wc, float *wt, int C,
+                                    hipStream_t st) {
+    if (C <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_transpose, dim3((C * 9 + 255) / 256, 3), dim3(256), 0, st, wa, wb, wc, wt, C);
     return hipGetLastError();
 }

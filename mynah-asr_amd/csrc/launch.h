@@ -155,18 +155,26 @@ hipError_t mh_launch_glu_dwconv(const float *h, const float *w, const float *bia
 // [segment][time][freq][channel] (C a multiple of 4); causal pads (2, 1),
 // else (1, 1), in time and frequency alike.
 int mh_ss_out_len(int n, int causal);   // the length after one stride-2 stage
+// xp, xpf (or null; C a multiple of 256): the output as the EXACT products'
+// prepared input (mh_mpad(rows) * K * 4 bytes, mh_mpad(rows) * K / 128 floats)
+// in place of out.
 // the first conv (1 -> C, + b0, ReLU) and the first depthwise conv (+ b1) in
 // one pass: x [nseq][T][F] -> out [nseq][T2][F2][C]
 hipError_t mh_launch_conv_in_dw(const float *x, const float *w0, const float *b0, const float *w1, const float *b1,
-                                float *out, int nseq, int T, int F, int C, int causal, hipStream_t st);
+                                float *out, int nseq, int T, int F, int C, int causal, uint8_t *xp, float *xpf,
+                                hipStream_t st);
 // pb (or null): the previous pointwise conv's bias, applied with ReLU on load
 hipError_t mh_launch_dw_s2(const float *in, const float *pb, const float *w, const float *b, float *out, int nseq,
-                           int T, int F, int C, int causal, hipStream_t st);
+                           int T, int F, int C, int causal, uint8_t *xp, float *xpf, hipStream_t st);
 hipError_t mh_launch_flatten(const float *in, const float *pb, float *flat, size_t rows, int Fo, int C,
                              hipStream_t st);
-// wt [k][C] = the taps of w [C][k] tap-major (the layout k_conv_in_dw and
-// k_dw_s2 read: w, the argument of their launchers, is this copy)
-hipError_t mh_launch_transpose_taps(const float *w, float *wt, int C, int k, hipStream_t st);
+bool mh_flatten_prep_supported(int Fo, int C);
+hipError_t mh_launch_flatten_prep(const float *in, const float *pb, size_t rows, int Fo, int C, uint8_t *xp,
+                                  float *xpf, hipStream_t st);
+// wt [3][9][C] = the taps of wa, wb, wc [C][9] tap-major (the layout k_conv_in_dw
+// and k_dw_s2 read: w, the argument of their launchers, is such a copy)
+hipError_t mh_launch_transpose_taps(const float *wa, const float *wb, const float *wc, float *wt, int C,
+                                    hipStream_t st);
 // y = (y + b) * scale per row (scale 1: the bias alone)
 hipError_t mh_launch_bias_scale(float *y, const float *b, size_t rows, int d, float scale, hipStream_t st);
 

@@ -231,6 +231,43 @@ def test_subsampling_matches_oracle(gpu, causal, C):
         dev.close()
 
 
+@pytest.mark.parametrize("causal,C,mels,T,nseq", [
+    (0, 256, 80, 203, 3),     # rows split over waves, a ragged last 64-row block in every product
+    (1, 256, 80, 41, 1),      # the second product and the linear have few rows (no prepared input)
+    (1, 512, 128, 130, 2),    # two passes over the channels
+    (0, 256, 300, 67, 1),     # 75 columns: three parts of a row even when rows fill the chip
+    (0, 64, 80, 4500, 2),     # whole rows per wave, f32 hand-offs
+])
+def test_subsampling_handoffs(gpu, monkeypatch, causal, C, mels, T, nseq):
+    """The prepared hand-offs give the bits of the f32 ones, and both the
+    oracle's values (bar as above)."""
+    import torch
+    say("subsampling hand-offs", causal, C, mels, T, nseq)
+    d = 256
+    p = ss_params(14, C, mels, d, causal)
+    dev = M.DeviceSubsampling(gpu, p, causal)
+    try:
+        x = np.random.default_rng(15).standard_normal((nseq * T, mels)).astype(np.float32)
+        xd = torch.from_numpy(x).cuda()
+        To = T
+        for _ in range(3):
+            To = (To + (3 if causal else 2) - 3) // 2 + 1
+        outs = []
+        for flag in ("1", "0"):
+            monkeypatch.setenv("MYNAH_ASR_HIP_LN_PREP", flag)
+            out = torch.full((nseq * To, d), float("nan"), dtype=torch.float32, device="cuda")
+            assert dev.run(xd.data_ptr(), T, nseq, mels, out.data_ptr(), xscale=2.0) == To
+            torch.cuda.synchronize()
+            outs.append(out)
+        assert torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
+        pp = {k: (v.reshape(v.shape[0], -1) if k.startswith("pw_w") else v) for k, v in p.items()}
+        ref = np.concatenate([2.0 * E.subsampling(x[s * T:(s + 1) * T], pp, causal) for s in range(nseq)])
+        err = np.abs(outs[0].cpu().numpy() - ref)
+        assert (err <= 5e-6 * (np.abs(ref) + np.sqrt((ref ** 2).mean()))).all()
+    finally:
+        dev.close()
+
+
 @pytest.mark.parametrize("mode", [M.INT8ACT, M.QMAT], ids=["int8act", "qmat"])
 def test_encoder_layer_in_other_numerics(gpu, mode):
     """Each product of the layer runs in the current numerics mode (the
