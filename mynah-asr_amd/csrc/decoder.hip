@@ -23,7 +23,7 @@
 #include <math.h>
 #include <stdint.h>
 
-#include "launch.h"
+#include "product.h"
 
 namespace {
 
@@ -31,26 +31,16 @@ constexpr int LN_T = 256;   // threads of the one-workgroup row kernels
 constexpr int LN_V = 16;    // values per thread: d <= 4096
 constexpr int KC = MH_ATT_KC;   // keys per attention split
 
-// Sum over the NT threads of the workgroup in double (the reference's ln
-// accumulates in double).
-template <int NT>
-__device__ double block_sum(double v, double *red) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) red[w] = v;
-    __syncthreads();
-    double s = 0.0;
-    for (int i = 0; i < NT / 64; i++) s += red[i];
-    return s;
-}
-
 // y = LN(v) over d values held V per thread (i = tid + NT * u):
-// (float)((x - mean) * inv) * w + b with inv = (float)(1 / sqrt(var + 1e-5))
+// (float)((x - mean) * inv) * w + b with inv = (float)(1 / sqrt(var + 1e-5)),
+// the sums in double (as the reference's ln) in one pass, of the differences to
+// the row's first value: what cancels in the variance is at most d^2 2^-53 of it
 template <int NT, int V>
 __device__ void ln_store(float (&v)[V], int d, const float *w, const float *b, float *y) {
-    __shared__ double red[NT / 64];
+    __shared__ double rs[NT / 64], rq[NT / 64];
+    __shared__ float first;
     const int tid = threadIdx.x;
+    if (tid == 0) first = v[0];
     float lw[V], lb[V];   // loaded before the sums, so their latency overlaps them
 #pragma unroll
     for (int u = 0; u < V; u++) {
@@ -58,25 +48,29 @@ __device__ void ln_store(float (&v)[V], int d, const float *w, const float *b, f
         lw[u] = i < d ? w[i] : 0.0f;
         lb[u] = i < d ? b[i] : 0.0f;
     }
-    double s = 0.0;
-#pragma unroll
-    for (int u = 0; u < V; u++)
-        if (tid + NT * u < d) s += (double)v[u];
-    const double mu = block_sum<NT>(s, red) / d;
-    double q = 0.0;
+    __syncthreads();
+    const double x0 = (double)first;
+    double s = 0.0, q = 0.0;
 #pragma unroll
     for (int u = 0; u < V; u++)
         if (tid + NT * u < d) {
-            const double c = (double)v[u] - mu;
+            const double c = (double)v[u] - x0;
+            s += c;
             q += c * c;
         }
-    const double var = block_sum<NT>(q, red) / d;
-    const float inv = (float)(1.0 / sqrt(var + 1e-5));
+    s = wave_sum(s);
+    q = wave_sum(q);
+    if ((tid & 63) == 0) rs[tid >> 6] = s, rq[tid >> 6] = q;
+    __syncthreads();
+    s = q = 0.0;
+#pragma unroll
+    for (int i = 0; i < NT / 64; i++) s += rs[i], q += rq[i];
+    const double m = s / d, mu = x0 + m, inv = (double)(float)rsqrt_d(q / d - m * m + 1e-5);
 #pragma unroll
     for (int u = 0; u < V; u++) {
         const int i = tid + NT * u;
         if (i < d) {
-            const float t = (float)(((double)v[u] - mu) * (double)inv);
+            const float t = (float)(((double)v[u] - mu) * inv);
             y[i] = t * lw[u] + lb[u];
         }
     }

@@ -45,9 +45,13 @@ __device__ __forceinline__ float sigmoid_f(float x) {
 
 // One wave per row of d = 256 V4 floats (lane l holds elements 4l + 256u ..
 // +3): x += alpha res (stored; res may be null), then the layer norm into
-// v. Sums in double in two passes, as layer_norm_f: mean, then the sum of
-// (x - mean)^2; inv = (float)(1 / sqrt(var + 1e-5)); v = ((x - (float)mean)
-// * inv) * w + b in f32.
+// v: mean and var in double, inv = (float)(1 / sqrt(var + 1e-5)); v = ((x -
+// (float)mean) * inv) * w + b in f32, as layer_norm_f. One pass sums the
+// differences to the row's first element and their squares: (x[0] - mean)^2 <= d
+// var, so what cancels in the variance is at most d^2 2^-53 of it. Two passes
+// are twice the chain of double sums across the wave, which is most of the time
+// when rows are few (a layer of 63 x 1024, five of these: 118 -> 116 us; of 1004
+// x 1024, six: 290 -> 279 us).
 template <int V4>
 __device__ __forceinline__ void add_ln_row(float *xr, const float *__restrict__ rr, float alpha,
                                            const float *__restrict__ w, const float *__restrict__ b, int silu, int lane,
@@ -72,20 +76,20 @@ __device__ __forceinline__ void add_ln_row(float *xr, const float *__restrict__ 
             *(float4 *)(xr + 4 * lane + 256 * u) = v[u];
         }
     }
-    double s = 0.0;
-#pragma unroll
-    for (int u = 0; u < V4; u++) s += ((double)v[u].x + (double)v[u].y) + ((double)v[u].z + (double)v[u].w);
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    const double mu = s / d;
-    double q = 0.0;
+    const double x0 = (double)__int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v[0].x)));
+    double s = 0.0, q = 0.0;
 #pragma unroll
     for (int u = 0; u < V4; u++) {
-        const double c0 = (double)v[u].x - mu, c1 = (double)v[u].y - mu;
-        const double c2 = (double)v[u].z - mu, c3 = (double)v[u].w - mu;
+        const double c0 = (double)v[u].x - x0, c1 = (double)v[u].y - x0;
+        const double c2 = (double)v[u].z - x0, c3 = (double)v[u].w - x0;
+        s += (c0 + c1) + (c2 + c3);
         q += (c0 * c0 + c1 * c1) + (c2 * c2 + c3 * c3);
     }
-    for (int o = 32; o > 0; o >>= 1) q += __shfl_xor(q, o, 64);
-    const float inv = (float)(1.0 / sqrt(q / d + 1e-5));
+    s = wave_sum(s);
+    q = wave_sum(q);
+    constexpr double rd = 1.0 / d;
+    const double m = s * rd, mu = x0 + m;
+    const float inv = (float)rsqrt_d(q * rd - m * m + 1e-5);
     const float muf = (float)mu;
 #pragma unroll
     for (int u = 0; u < V4; u++) {
@@ -105,15 +109,7 @@ __device__ __forceinline__ void prep_store4(float4 v, int lane, size_t m, int c,
                                             float *__restrict__ xpf) {
     const int l32 = lane & 31, hu = l32 >> 2, hh = (l32 >> 1) & 1;
     float a = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-    auto step = [&](auto ctrl) {   // (within each row of 16 lanes, symmetrically)
-        a = fmaxf(a, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), decltype(ctrl)::value, 0xF, 0xF,
-                                                                false)));
-    };
-    step(std::integral_constant<int, 0xB1>{});    // quad_perm [1,0,3,2]
-    step(std::integral_constant<int, 0x4E>{});    // quad_perm [2,3,0,1]
-    step(std::integral_constant<int, 0x141>{});   // row_half_mirror
-    step(std::integral_constant<int, 0x140>{});   // row_mirror
-    a = fmaxf(a, __shfl_xor(a, 16, 64));
+    a = wave_max<32>(a);
     const int sh = chunk_shift(a);
     const float xs[4] = {ldexpf(v.x, sh), ldexpf(v.y, sh), ldexpf(v.z, sh), ldexpf(v.w, sh)};
     const half4v h = {(_Float16)xs[0], (_Float16)xs[1], (_Float16)xs[2], (_Float16)xs[3]};
@@ -177,9 +173,7 @@ __global__ __launch_bounds__(512) void k_add_ln_prep(float *x, const float *__re
     for (int u = 0; u < V4; u++) {
         const int c = 2 * u + (lane >> 5);
         float a = fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w)));
-#pragma unroll
-        for (int o = 16; o > 0; o >>= 1) a = fmaxf(a, __shfl_xor(a, o, 64));
-        const int sh = chunk_shift(a);
+        const int sh = chunk_shift(wave_max<32>(a));
         const float xs[4] = {ldexpf(v[u].x, sh), ldexpf(v[u].y, sh), ldexpf(v[u].z, sh), ldexpf(v[u].w, sh)};
         _Float16 hv[4], lv[4];
 #pragma unroll

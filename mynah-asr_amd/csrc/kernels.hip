@@ -544,28 +544,6 @@ __device__ __forceinline__ void wave_row_issue(const GPro &pro, int K, int c, in
     }
 }
 
-// a double moved between lanes by one DPP pattern (its two halves)
-template <int CTRL>
-__device__ __forceinline__ double dpp_d(double x) {
-    const long long b = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-// The wave's sum in every lane: within each row of 16 lanes by DPP (swap
-// neighbours, swap pairs, mirror within 8, mirror within 16: each step adds
-// two values symmetrically, so every lane holds the same sum), then across
-// the four rows.
-__device__ __forceinline__ double wave_sum(double v) {
-    v += dpp_d<0xB1>(v);    // quad_perm [1,0,3,2]
-    v += dpp_d<0x4E>(v);    // quad_perm [2,3,0,1]
-    v += dpp_d<0x141>(v);   // row_half_mirror
-    v += dpp_d<0x140>(v);   // row_mirror
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
-    return v;
-}
-
 // the lane's two elements of chunk c (zero past K)
 __device__ __forceinline__ float2 wave_row_values(const GPro &pro, int K, int c, int lane, WaveRow &r) {
     const int e = 128 * c + 2 * lane;
@@ -574,10 +552,9 @@ __device__ __forceinline__ float2 wave_row_values(const GPro &pro, int K, int c,
         if (!r.have) {
             // Mean and variance over the row in double in one pass, of the
             // differences to x[0]: (x[0] - mean)^2 <= K var, so what cancels
-            // in the variance is at most K^2 2^-53 of it. 1/sqrt by the
-            // hardware's estimate (about 24 bits) and two Newton steps. (Two
-            // passes with their divisions and square root are a chain of about
-            // 2300 cycles.)
+            // in the variance is at most K^2 2^-53 of it. (Two passes with
+            // their divisions and square root are a chain of about 2300
+            // cycles.)
             const double x0 = (double)__shfl(r.a[0].x, 0, 64);
             double s = 0.0, q = 0.0;
             auto add = [&](float2 v) {
@@ -603,10 +580,7 @@ __device__ __forceinline__ float2 wave_row_values(const GPro &pro, int K, int c,
             q = wave_sum(q);
             const double rk = pro.rk, m = s * rk, var = q * rk - m * m + 1e-5;
             r.mu = x0 + m;
-            double y = __builtin_amdgcn_rsq(var);
-#pragma unroll
-            for (int i = 0; i < 2; i++) y = y * (1.5 - 0.5 * var * y * y);
-            r.inv = (double)(float)y;
+            r.inv = (double)(float)rsqrt_d(var);
             r.have = true;
         }
         if (!live) return float2{0.0f, 0.0f};
@@ -659,25 +633,13 @@ __device__ __forceinline__ float2 wave_row_values(const GPro &pro, int K, int c,
 // row's fragment, so all 32 rows of A hold it; only row 0 of the result is
 // used. Two lanes splitting 64 values each took about 250 VALU instructions
 // per chunk, 0.3 us of a GEMV's 4.5 to 7.
-__device__ __forceinline__ float dpp_max(float v) {
-    auto step = [&](auto ctrl) {
-        v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xF, 0xF,
-                                                                false)));
-    };
-    step(std::integral_constant<int, 0xB1>{});    // (the steps of wave_sum)
-    step(std::integral_constant<int, 0x4E>{});
-    step(std::integral_constant<int, 0x141>{});
-    step(std::integral_constant<int, 0x140>{});
-    v = fmaxf(v, __shfl_xor(v, 16, 64));
-    return fmaxf(v, __shfl_xor(v, 32, 64));
-}
 template <int I>
 __device__ __forceinline__ float quad_lane(float v) {   // lane I of the lane's four
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), I * 0x55, 0xF, 0xF, false));
 }
 template <bool MINS>
 __device__ __forceinline__ void split_row(float2 v, int lane, int hh, uint32_t *lds, XChunk &o) {
-    const int sh = chunk_shift(dpp_max(fmaxf(fabsf(v.x), fabsf(v.y))));
+    const int sh = chunk_shift(wave_max<64>(fmaxf(fabsf(v.x), fabsf(v.y))));
     o.p = ldexpf(1.0f, -sh);
     const float x0 = ldexpf(v.x, sh), x1 = ldexpf(v.y, sh);
     const half2v h = {(_Float16)x0, (_Float16)x1};

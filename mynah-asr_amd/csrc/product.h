@@ -3,6 +3,8 @@
 // the operands of the affine formats. A row's bits are the same from every
 // kernel because they all run these functions in the same order.
 #pragma once
+#include <type_traits>
+
 #include "fmt.h"
 #include "launch.h"
 
@@ -31,6 +33,50 @@ __device__ __forceinline__ float silu_f(float v) {
     const float e = __expf(-fabsf(v));
     const float r = __builtin_amdgcn_rcpf(1.0f + e);
     return v * (v >= 0.0f ? r : e * r);
+}
+
+// a double moved between lanes by one DPP pattern (its two halves)
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double x) {
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// The wave's sum in every lane: within each row of 16 lanes by DPP (swap
+// neighbours, swap pairs, mirror within 8, mirror within 16: each step adds
+// two values symmetrically, so every lane holds the same sum), then across
+// the four rows.
+__device__ __forceinline__ double wave_sum(double v) {
+    v += dpp_d<0xB1>(v);    // quad_perm [1,0,3,2]
+    v += dpp_d<0x4E>(v);    // quad_perm [2,3,0,1]
+    v += dpp_d<0x141>(v);   // row_half_mirror
+    v += dpp_d<0x140>(v);   // row_mirror
+    v += __shfl_xor(v, 16, 64);
+    v += __shfl_xor(v, 32, 64);
+    return v;
+}
+// the maximum over the wave (N = 64) or over each half of it (32), in every lane
+template <int N>
+__device__ __forceinline__ float wave_max(float v) {
+    auto step = [&](auto ctrl) {
+        v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xF, 0xF,
+                                                                false)));
+    };
+    step(std::integral_constant<int, 0xB1>{});    // (the steps of wave_sum)
+    step(std::integral_constant<int, 0x4E>{});
+    step(std::integral_constant<int, 0x141>{});
+    step(std::integral_constant<int, 0x140>{});
+    v = fmaxf(v, __shfl_xor(v, 16, 64));
+    if (N == 64) v = fmaxf(v, __shfl_xor(v, 32, 64));
+    return v;
+}
+// 1/sqrt in double: the hardware's estimate (about 24 bits) and two Newton steps
+__device__ __forceinline__ double rsqrt_d(double v) {
+    double y = __builtin_amdgcn_rsq(v);
+#pragma unroll
+    for (int i = 0; i < 2; i++) y = y * (1.5 - 0.5 * v * y * y);
+    return y;
 }
 
 // ---------------------------------------------------------------------------
