@@ -21,7 +21,8 @@
 // final linear are this unit's products:
 //   k_conv_in_dw  the full 3x3 stride-2 conv of the mel features, 1 -> C
 //               channels, + bias, ReLU (:222-226), fused into the first
-//               depthwise 3x3 stride-2 conv, + bias (:231-236)
+//               depthwise 3x3 stride-2 conv, + bias (:231-236);
+//               k_conv_in_dw_mx is its form on the f32 MFMA
 //   k_dw_s2     the depthwise 3x3 stride-2 conv, + bias; its input takes
 //               the previous pointwise conv's bias and ReLU on load  :237-244
 //   k_flatten   the last pointwise conv's bias and ReLU, then the
@@ -473,30 +474,19 @@ __global__ __launch_bounds__(256) void k_dwconv_tile(const float *__restrict__ g
 // single mel samples behind their bounds, through the scalar cache, made a step
 // a chain of about 30 waits: 138 us at 4 segments of 6000 frames (6000 rows of
 // 20 columns, 256 channels), where its fmas take 55.
-// PREP: the rows are written as the pointwise product's prepared input (waves
-// past the rows write the 64-row padding) instead of as f32.
+// For channels that are no multiple of 128; the others take k_conv_in_dw_mx.
 // Weights tap-major, w0[j][C] and w1[j][C].
 constexpr int CI_FS = 32;   // columns per wave at most
-template <bool PREP>
 __global__ __launch_bounds__(256) void k_conv_in_dw(const float *__restrict__ x, const float *__restrict__ w0,
                                                     const float *__restrict__ b0, const float *__restrict__ w1,
                                                     const float *__restrict__ b1, float *__restrict__ out, int nseq,
                                                     int T, int F, int T1, int F1, int To, int Fo, int C, int pl,
-                                                    int FS, int parts, uint8_t *__restrict__ xp,
-                                                    float *__restrict__ xpf) {
+                                                    int FS, int parts) {
     constexpr int WC = 4 * CI_FS + 4;
     __shared__ __align__(16) float win[4][7][WC];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + wave), wrow = wid / parts;
-    if (wrow >= nseq * To) {
-        if constexpr (PREP) {
-            const size_t M = (size_t)nseq * To * Fo, m = M + (wid - nseq * To * parts);
-            if (m < (M + 63) / 64 * 64)
-                for (int c = 4 * lane; c < C; c += 256)
-                    prep_store4(float4{0.f, 0.f, 0.f, 0.f}, lane, m, c >> 7, C / 128, xp, xpf);
-        }
-        return;   // (no workgroup barrier follows)
-    }
+    if (wrow >= nseq * To) return;   // (no workgroup barrier follows)
     const int to = wrow % To, s = wrow / To, f0 = (wid - wrow * parts) * FS, f9 = min(f0 + FS, Fo);
     const float *xs = x + (size_t)s * T * F;
     // window column k: mel f = 4 f0 - 3 pl + k; window row j: mel t = 4 to - 3 pl + j
@@ -577,9 +567,139 @@ __global__ __launch_bounds__(256) void k_conv_in_dw(const float *__restrict__ x,
             }
             acc = float4{bb1.x + acc.x, bb1.y + acc.y, bb1.z + acc.z, bb1.w + acc.w};
             const size_t m = (size_t)wrow * Fo + fo;
-            if constexpr (PREP) prep_store4(acc, lane, m, c >> 7, C / 128, xp, xpf);
-            else *(float4 *)(out + m * C + c) = acc;
+            *(float4 *)(out + m * C + c) = acc;
         }
+    }
+}
+
+// The same for channels that are a multiple of 128, with the first conv on the
+// f32 MFMA. A workgroup is 32 consecutive output rows m = (s, to, fo) by 128
+// channels, wave w channels 32w .. 32w + 31: for each of the nine depthwise
+// taps y comes as five 32 x 32 x 2 MFMAs (rows = channels, columns = output
+// rows, K = the nine mel samples and a zero), starting from b0, and goes into
+// the tap's fma where it lies. Each lane holds 16 channels of one output row, so
+// nothing moves between lanes, and rows of any T and F fill the tiles. The mel
+// samples come to LDS once per workgroup in the B operand's order.
+// On the VALU the first conv's fmas alone are 216 of about 330 instructions per
+// wave and step, which bounds k_conv_in_dw: 95 us at 4 segments of 6000 frames of
+// 80 features, 256 channels, 87 here (both traced; the whole subsampling 330 ->
+// 314 us, other boxes within 1%). The 45 MFMAs of a tile are 35 us of it at the
+// f32 MFMA's nominal rate and the rows' 123 MB 25; what is left is the chain of
+// a tap (five dependent MFMAs, then their fmas). A neighbour's column would
+// save a third of the MFMAs but lies in other lanes.
+// PREP: the pointwise product's prepared input, its 64-row padding as zeros: the
+// arithmetic of prep_store4, the chunk's maximum over the four waves.
+template <bool PREP>
+__global__ __launch_bounds__(256, 4) void k_conv_in_dw_mx(const float *__restrict__ x, const float *__restrict__ w0,
+                                                       const float *__restrict__ b0, const float *__restrict__ w1,
+                                                       const float *__restrict__ b1, float *__restrict__ out, int M,
+                                                       int T, int F, int T1, int F1, int To, int Fo, int C, int pl,
+                                                       uint8_t *__restrict__ xp, float *__restrict__ xpf) {
+    __shared__ float win[7][7][32];   // mel rows 4 to - 3 pl .., columns 4 fo - 3 pl .. of each output row
+    __shared__ __align__(16) float wd[9][128];
+    __shared__ float wm[4][32];
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = (int)blockIdx.x * 32 + l32, c0 = 128 * (int)blockIdx.y, cw = c0 + 32 * wave;
+    const bool live = m < M;
+    const unsigned mm = live ? m : 0, row = mm / (unsigned)Fo, s = row / (unsigned)To;
+    const int fo = (int)(mm - row * Fo), to = (int)(row - s * To);
+    // half wave g takes window row g: all loads go out before the first is stored
+    const int g7 = 2 * wave + hh, t = 4 * to - 3 * pl + g7;
+    const bool tin = live && g7 < 7 && (unsigned)t < (unsigned)T;
+    const float *xr = x + (tin ? ((size_t)s * T + t) * F : 0);
+    float v[7];
+#pragma unroll
+    for (int u = 0; u < 7; u++) {
+        const int f = 4 * fo - 3 * pl + u;
+        const bool in = tin && (unsigned)f < (unsigned)F;
+        const float e = xr[in ? f : 0];
+        v[u] = in ? e : 0.0f;
+    }
+    float a[5];   // A operand: channel l32, sample 2j + hh
+#pragma unroll
+    for (int j = 0; j < 5; j++) a[j] = 2 * j + hh < 9 ? w0[(size_t)(2 * j + hh) * C + cw + l32] : 0.0f;
+    f16v bias;
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        const float4 b = *(const float4 *)(b0 + cw + 8 * g + 4 * hh);
+        bias[4 * g] = b.x, bias[4 * g + 1] = b.y, bias[4 * g + 2] = b.z, bias[4 * g + 3] = b.w;
+    }
+    for (int i = tid; i < 9 * 32; i += 256)
+        *(float4 *)&wd[i >> 5][4 * (i & 31)] = *(const float4 *)(w1 + (size_t)(i >> 5) * C + c0 + 4 * (i & 31));
+    if (g7 < 7)
+#pragma unroll
+        for (int u = 0; u < 7; u++) win[g7][u][l32] = v[u];
+    __syncthreads();
+    const float *bp[5];   // B operand: output row l32, sample 2j + hh of tap (0, 0)
+#pragma unroll
+    for (int j = 0; j < 5; j++) bp[j] = 2 * j + hh < 9 ? &win[(2 * j + hh) / 3][(2 * j + hh) % 3][l32] : &win[0][0][l32];
+    float4 o[4];
+#pragma unroll
+    for (int g = 0; g < 4; g++) o[g] = float4{0.f, 0.f, 0.f, 0.f};
+    // (unrolled, the compiler reads every tap ahead at one wave per SIMD: the whole
+    // subsampling 408 us; three taps unrolled at three waves: 323; rolled, the
+    // waves of a SIMD overlap each other's MFMAs and fmas)
+#pragma unroll 1
+    for (int y = 0; y < 9; y++) {
+        f16v acc = bias;
+        const int r = y / 3, cc = y - 3 * r, at = (2 * r * 7 + 2 * cc) * 32;
+        float bv[5];
+#pragma unroll
+        for (int j = 0; j < 5; j++) bv[j] = bp[j][at];
+        __builtin_amdgcn_sched_barrier(0);   // (one wait for all five, not one in front of each MFMA)
+        bv[4] = hh ? 0.0f : bv[4];   // (the tenth sample)
+#pragma unroll
+        for (int j = 0; j < 5; j++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], bv[j], acc, 0, 0, 0);
+        // ReLU; zero outside y's [T1, F1]
+        const bool yin = (unsigned)(2 * to - pl + r) < (unsigned)T1 && (unsigned)(2 * fo - pl + cc) < (unsigned)F1;
+        const float lim = yin ? INFINITY : 0.0f;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const float4 wv = *(const float4 *)&wd[y][32 * wave + 8 * g + 4 * hh];
+            const float4 yv = {__builtin_amdgcn_fmed3f(acc[4 * g], 0.0f, lim),
+                               __builtin_amdgcn_fmed3f(acc[4 * g + 1], 0.0f, lim),
+                               __builtin_amdgcn_fmed3f(acc[4 * g + 2], 0.0f, lim),
+                               __builtin_amdgcn_fmed3f(acc[4 * g + 3], 0.0f, lim)};
+            o[g].x = fmaf(wv.x, yv.x, o[g].x);
+            o[g].y = fmaf(wv.y, yv.y, o[g].y);
+            o[g].z = fmaf(wv.z, yv.z, o[g].z);
+            o[g].w = fmaf(wv.w, yv.w, o[g].w);
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        const float4 b = *(const float4 *)(b1 + cw + 8 * g + 4 * hh);
+        o[g] = float4{b.x + o[g].x, b.y + o[g].y, b.z + o[g].z, b.w + o[g].w};
+        if constexpr (!PREP)
+            if (live) *(float4 *)(out + (size_t)m * C + cw + 8 * g + 4 * hh) = o[g];
+    }
+    if constexpr (PREP) {
+        float am = 0.0f;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            if (!live) o[g] = float4{0.f, 0.f, 0.f, 0.f};
+            am = fmaxf(am, fmaxf(fmaxf(fabsf(o[g].x), fabsf(o[g].y)), fmaxf(fabsf(o[g].z), fabsf(o[g].w))));
+        }
+        am = fmaxf(am, __shfl_xor(am, 32, 64));
+        if (hh == 0) wm[wave][l32] = am;
+        __syncthreads();
+        am = fmaxf(fmaxf(wm[0][l32], wm[1][l32]), fmaxf(wm[2][l32], wm[3][l32]));
+        const int sh = chunk_shift(am), Kc = C / 128;
+        const size_t mc = (size_t)blockIdx.x * Kc + blockIdx.y;   // (32 rows, chunk)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const float xv[4] = {ldexpf(o[g].x, sh), ldexpf(o[g].y, sh), ldexpf(o[g].z, sh), ldexpf(o[g].w, sh)};
+            const half4v h = {(_Float16)xv[0], (_Float16)xv[1], (_Float16)xv[2], (_Float16)xv[3]};
+            uint2 hw;
+            __builtin_memcpy(&hw, &h, 8);
+            const uint2 lw = {lo_pair(hw.x, xv[0], xv[1]), lo_pair(hw.y, xv[2], xv[3])};
+            // channels 32 wave + 8 g + 4 hh ..: half-step 2 wave + g / 2, slot half g % 2
+            uint8_t *p = xp + ((mc * 8 + 2 * wave + (g >> 1)) * 2 * 64 + l32 + 32 * (g & 1)) * 16 + 8 * hh;
+            *(uint2 *)p = hw;
+            *(uint2 *)(p + 64 * 16) = lw;
+        }
+        if (tid < 32) xpf[mc * 32 + l32] = ldexpf(1.0f, -sh);
     }
 }
 
@@ -830,26 +950,32 @@ int mh_ss_out_len(int n, int causal) {
 hipError_t mh_launch_conv_in_dw(const float *x, const float *w0, const float *b0, const float *w1, const float *b1,
                                 float *out, int nseq, int T, int F, int C, int causal, uint8_t *xp, float *xpf,
                                 hipStream_t st) {
-    if (C % 4 || (xp && C % 256)) return hipErrorInvalidValue;
+    if (C % 4 || (xp && C % 128)) return hipErrorInvalidValue;
     const int T1 = mh_ss_out_len(T, causal), F1 = mh_ss_out_len(F, causal);
     const int To = mh_ss_out_len(T1, causal), Fo = mh_ss_out_len(F1, causal), pl = causal ? 2 : 1;
     if (T1 <= 0 || F1 <= 0 || To <= 0 || Fo <= 0) return hipSuccess;
-    const size_t rows = (size_t)nseq * To;   // output rows (s, to)
+    const size_t rows = (size_t)nseq * To, M = rows * Fo;   // output rows (s, to), and (s, to, fo)
     if (!rows) return hipSuccess;
+    if (M > 0x7fffff00) return hipErrorInvalidValue;
+    if (C % 128 == 0) {
+        if (C / 128 > 65535) return hipErrorInvalidValue;
+        const dim3 grid((unsigned)(xp ? (M + 63) / 64 * 2 : (M + 31) / 32), C / 128);
+        if (xp)
+            hipLaunchKernelGGL(k_conv_in_dw_mx<true>, grid, dim3(256), 0, st, x, w0, b0, w1, b1, out, (int)M, T, F, T1,
+                               F1, To, Fo, C, pl, xp, xpf);
+        else
+            hipLaunchKernelGGL(k_conv_in_dw_mx<false>, grid, dim3(256), 0, st, x, w0, b0, w1, b1, out, (int)M, T, F, T1,
+                               F1, To, Fo, C, pl, xp, xpf);
+        return hipGetLastError();
+    }
     // A wave takes whole rows while they fill the chip (1024 SIMDs, 3 waves
     // each), else part of one: a part forms one column of y more
     int FS = Fo < CI_FS ? Fo : CI_FS;
     while (FS > 4 && rows * ((Fo + FS - 1) / FS) < 2048) FS = (FS + 1) / 2;
     const int parts = (Fo + FS - 1) / FS;
     if (rows * parts > 0x7fffff00) return hipErrorInvalidValue;
-    const size_t M = rows * Fo, waves = rows * parts + (xp ? (M + 63) / 64 * 64 - M : 0);
-    const dim3 grid((unsigned)((waves + 3) / 4));
-    if (xp)
-        hipLaunchKernelGGL(k_conv_in_dw<true>, grid, dim3(256), 0, st, x, w0, b0, w1, b1, out, nseq, T, F, T1, F1, To,
-                           Fo, C, pl, FS, parts, xp, xpf);
-    else
-        hipLaunchKernelGGL(k_conv_in_dw<false>, grid, dim3(256), 0, st, x, w0, b0, w1, b1, out, nseq, T, F, T1, F1, To,
-                           Fo, C, pl, FS, parts, xp, xpf);
+    hipLaunchKernelGGL(k_conv_in_dw, dim3((unsigned)((rows * parts + 3) / 4)), dim3(256), 0, st, x, w0, b0, w1, b1, out,
+                       nseq, T, F, T1, F1, To, Fo, C, pl, FS, parts);
     return hipGetLastError();
 }
 

@@ -237,6 +237,8 @@ def test_subsampling_matches_oracle(gpu, causal, C):
     (1, 512, 128, 130, 2),    # two passes over the channels
     (0, 256, 300, 67, 1),     # 75 columns: three parts of a row even when rows fill the chip
     (0, 64, 80, 4500, 2),     # whole rows per wave, f32 hand-offs
+    (1, 384, 80, 99, 3),      # the first stage's MFMA tiles, f32 rows out (a ragged last tile)
+    (0, 128, 16, 17, 1),      # the same, one short tile: every row at an edge
 ])
 def test_subsampling_handoffs(gpu, monkeypatch, causal, C, mels, T, nseq):
     """The prepared hand-offs give the bits of the f32 ones, and both the
