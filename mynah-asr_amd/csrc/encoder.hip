@@ -583,7 +583,7 @@ __global__ __launch_bounds__(256) void k_conv_in_dw(const float *__restrict__ x,
 // On the VALU the first conv's fmas alone are 216 of about 330 instructions per
 // wave and step, which bounds k_conv_in_dw: 95 us at 4 segments of 6000 frames of
 // 80 features, 256 channels, 87 here (both traced; the whole subsampling 330 ->
-// 314 us, other boxes within 1%). The 45 MFMAs of a tile are 35 us of it at the
+// 314 us). The 45 MFMAs of a tile are 35 us of it at the
 // f32 MFMA's nominal rate and the rows' 123 MB 25; what is left is the chain of
 // a tap (five dependent MFMAs, then their fmas). A neighbour's column would
 // save a third of the MFMAs but lies in other lanes.
