@@ -215,12 +215,16 @@ int mynah_asr_hip_read_floor_dev(const void *p, size_t bytes, void *stream);
  * (head h at columns h*dk .. h*dk+dk-1, dk = d / H, 64 or 128). nseq > 1 runs
  * independent equal-length segments in one launch (the reference calls the
  * layer once per segment). All pointers 16-byte aligned. ctx may not alias
- * q, k or v. Outputs are f32 sums in another order than the reference's BLAS,
- * their products formed from f16 hi + lo splits scaled by powers of two (22 bits
- * of each row's, or V tile column's, maximum): equal within
- * |y - ref| <= 1e-4*|ref| + 1e-5*max|v|. K, rk and V are first split into the
- * calling thread's workspace (the size of K + V + rk, grown as needed, as the
- * other _dev calls' buffers are); 2T * d must stay below 2^31. */
+ * q, k or v. Outputs are f32 sums in another order than the reference's BLAS
+ * (full attention forms its products from f16 hi + lo splits scaled by powers of
+ * two, 22 bits of each row's, or V tile column's, maximum): equal within
+ * |y - ref| <= 1e-4*|ref| + 1e-5*max|v|. A row of chunked-limited attention
+ * depends on the keys of its window alone, bit for bit (the others finite). Full
+ * attention first splits K, rk and V into the calling thread's workspace (the
+ * size of K + V + rk, grown as needed, as the other _dev calls' buffers are): a
+ * thread's full-attention calls are ordered on one stream, or by events, and so
+ * are the replays of graphs that captured them. Chunked-limited attention uses
+ * no workspace. 2T * d must stay below 2^31. */
 /* The same on host buffers, one segment (the call encoder.c's attention() and
  * attention_banded() would make in place of their per-head loops, after rk is
  * formed): copies in, computes, copies ctx out. d must be a multiple of 4. */

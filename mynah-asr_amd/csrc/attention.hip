@@ -1,16 +1,13 @@
 // attention.hip — the relative-position self-attention core of the FastConformer
-// encoder layer (the reference's src/encoder.c:315-410 for full attention and
-// its banded twin encoder.c:220-313 for chunked-limited attention), on the f16
-// MFMA of gfx950 from split operands.
+// encoder layer over the full window (the reference's src/encoder.c:315-410), on
+// the f16 MFMA of gfx950 from split operands. Chunked-limited windows take
+// attention_window.hip.
 //
 // Per head h (columns h*DK .. h*DK+DK-1 of the [T, d] buffers):
 //   s[t, j] = ((q[t] + bias_u) . k[j] + (q[t] + bias_v) . rk[T-1 + j - t]) / sqrt(DK)
-//   ctx[t]  = sum_j softmax_j(s[t, j]) v[j],  j over the row's window
+//   ctx[t]  = sum_j softmax_j(s[t, j]) v[j],  j over [0, T)
 // rk = pe . relk_w^T is [2T-1, d] (the pos projection's output, shared by the
-// segments of one call). The window is all of [0, T) for left < 0, else
-// chunked-limited: chunk = right + 1, lc = left / chunk, row t (chunk t/chunk)
-// sees [(t/chunk - lc) * chunk, (t/chunk + 1) * chunk) clipped to [0, T)
-// (encoder.c:373-381).
+// segments of one call).
 //
 // Operands. Each row of q + bias, K and rk (per head) is scaled by the power of
 // two 2^e that puts its largest magnitude in [2^14, 2^15) and split into f16
@@ -45,11 +42,10 @@
 // about 400 VALU instructions; of a workgroup's 65 000 cycles at T = 750, 10 000
 // prepare the rows and load the first operands and 4500 join the contexts.
 // Measured, d 1024, 8 heads, full window, with the splits: 16 x 750 frames 430 ->
-// 275 us, 1 x 750 118 -> 36, 1 x 63 28 -> 13; [70, 13], 16 x 750: 173 -> 133 us
-// (before: 128-row blocks staging K, V and rk in LDS, f32 MFMA for the chunked
-// windows). No faster, each measured: eight waves per workgroup (15% slower at 16 x
-// 750), two query blocks per workgroup sharing K and V through L1, two MFMA
-// chains per product, the products' loads two phases ahead.
+// 275 us, 1 x 750 118 -> 36, 1 x 63 28 -> 13 (before: 128-row blocks staging K, V
+// and rk in LDS). No faster, each measured: eight waves per workgroup (15% slower
+// at 16 x 750), two query blocks per workgroup sharing K and V through L1, two
+// MFMA chains per product, the products' loads two phases ahead.
 //
 // MFMA 32x32x16 f16 operands (lane l, c = l & 31, hh = l >> 5): A row c, B column
 // c, k-slots 8 hh + j (j = 0..7); D column c, rows 8i + 4hh + jj in element 4i + jj.
@@ -96,8 +92,8 @@ __device__ __forceinline__ void split8(const float (&x)[8], int s, half8 &h, hal
 // [64 lanes][16 B]: lane (r, hh) of half-step u holds features 16u + 8hh .. +7
 // of row r.
 //   k   [segment][head][tile], keys 32 tile + r;  ke [..][32]: minus each row's e
-//   r   [head][nr blocks], block b = offsets' rows T + 32 (b + rb0) + r of rk
-//       (zeros outside [0, 2T-2]);                re [..][32] likewise
+//   r   [head][2 ntile blocks], block b = offsets' rows T + 32 (b - ntile) + r of
+//       rk (zeros outside [0, 2T-2]);             re [..][32] likewise
 //   v   [segment][head][tile] as [DK/32 feature groups][2 k-steps][hi, lo][64]
 //       [16 B]: lane (f, hh) of k-step u holds feature f of the group and keys 16u +
 //       8 (j >> 2) + 4hh + (j & 3) of the tile;   vs [..][DK]: 2^-(6 + e)
@@ -109,24 +105,9 @@ struct Planes {
     half8 *k, *r, *v;
     int *ke, *re;
     float *vs;
-    int ntile, nr, rb0;
+    int ntile;
     uint8_t *xp;
     float *xpf;
-};
-
-// Compiler-level ordering of a wave's own LDS writes and reads (the LDS
-// executes one wave's operations in issue order).
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-struct Window {
-    int lim, chunk, lc, T;
-    __device__ Window(int left, int right, int T_) : lim(left >= 0), chunk(lim ? right + 1 : 1), lc(lim ? left / chunk : 0), T(T_) {}
-    __device__ int j0(int t) const { return lim ? max((t / chunk - lc) * chunk, 0) : 0; }
-    __device__ int j1(int t) const { return lim ? min((t / chunk + 1) * chunk, T) : T; }
 };
 
 template <int DK> struct AttnLds {
@@ -145,7 +126,7 @@ template <int DK> struct AttnLds {
 template <int DK>
 __global__ __launch_bounds__(64 * NW, 2) void k_attn(const float *__restrict__ q, const float *__restrict__ bu,
                                                      const float *__restrict__ bv, float *__restrict__ ctx, int T,
-                                                     int d, int left, int right, float kscale, Planes P) {
+                                                     int d, float kscale, Planes P) {
     using L = AttnLds<DK>;
     constexpr int NU = L::NU, NF = DK / 32, NUW = (NU + NW - 1) / NW;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -160,20 +141,14 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn(const float *__restrict__ q
     // one head the same rk rows, so they run on one XCD and share its L2
     int bx, by, bz;
     xcd_order(bx, by, bz);
-    const int H = gridDim.y, ho = by * DK, t0 = 32 * bx;
-    const Window win(left, right, T);
-
-    // this wave's key tiles [ta, tb) of the block's [na, nb)
-    const int na = win.j0(t0) / KT, nb = (win.j1(min(t0 + 31, T - 1)) + KT - 1) / KT, n = nb - na;
-    const int ta = na + n * w / NW, tb = na + n * (w + 1) / NW;
-    const int tq = min(t0 + c, T - 1), rj0 = win.j0(tq), rj1 = win.j1(tq);   // this lane's query and its window
-    const int wj0 = win.j0(min(t0 + 31, T - 1)), wj1 = win.j1(t0);            // the keys that every row sees
+    const int H = gridDim.y, ho = by * DK, t0 = 32 * bx, n = P.ntile;
+    const int ta = n * w / NW, tb = n * (w + 1) / NW;   // this wave's key tiles [ta, tb)
     float *ring = (float *)(lds + L::Q + w * L::RING);
     const size_t bh = (size_t)bz * H + by;
     // (uniform bases and one 32-bit lane offset: scalar address arithmetic)
     const uint8_t *kp = (const uint8_t *)(P.k + bh * P.ntile * (DK * 8)), *vp = (const uint8_t *)(P.v + bh * P.ntile * (DK * 8));
-    const uint8_t *rp = (const uint8_t *)(P.r + (size_t)by * P.nr * (DK * 8));
-    const int *ke = P.ke + bh * P.ntile * 32, *re = P.re + (size_t)by * P.nr * 32;
+    const uint8_t *rp = (const uint8_t *)(P.r + (size_t)by * (2 * n) * (DK * 8));
+    const int *ke = P.ke + bh * P.ntile * 32, *re = P.re + (size_t)by * (2 * n) * 32;
     const float *vs = P.vs + bh * P.ntile * DK;
     const unsigned lo16 = lane * 16u;
     auto frag = [&](const uint8_t *base, size_t tile, int i) {   // fragment i of a tile
@@ -187,7 +162,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn(const float *__restrict__ q
 #pragma unroll
         for (int u = 0; u < HU; u++)
 #pragma unroll
-            for (int p = 0; p < 2; p++) rf[u0 + u][p] = frag(rp, (size_t)(t - bx - P.rb0), 2 * (u0 + u) + p);
+            for (int p = 0; p < 2; p++) rf[u0 + u][p] = frag(rp, (size_t)(t - bx + n), 2 * (u0 + u) + p);
     };
     // the rows' (q + bias_u), (q + bias_v), split, into LDS in B-operand order:
     // wave w forms half-steps w, w + NW, ... Loads return in order: the rows
@@ -213,7 +188,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn(const float *__restrict__ q
         if (ta < tb) {
             load_r(ta - 1, 0);
             load_r(ta - 1, HU);
-            er = re[(size_t)(ta - 1 - bx - P.rb0) * 32 + c];
+            er = re[(size_t)(ta - 1 - bx + n) * 32 + c];
 #pragma unroll
             for (int u = 0; u < NU; u++)
 #pragma unroll
@@ -322,7 +297,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn(const float *__restrict__ q
             }
             __builtin_amdgcn_sched_barrier(0);
             load_r(t, HU);
-            er = re[(size_t)(t - bx - P.rb0) * 32 + c];
+            er = re[(size_t)(t - bx + n) * 32 + c];
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int u = 0; u < NU; u++) bd_step(u, rf[u][0], rf[u][1], bd);
@@ -346,12 +321,10 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn(const float *__restrict__ q
                 sv[e] = (ldexpf(s[e], eqa + ee[e]) + rr[32 * (8 * (e >> 2) + (e & 3))]) * kscale;
             }
             wave_lds_order();   // (the next tile's ring writes come after these reads)
-            if (KT * t < wj0 || KT * t + KT > wj1) {
+            if (KT * t + KT > T) {
 #pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    const int j = KT * t + 8 * (e >> 2) + 4 * hh + (e & 3);
-                    if ((unsigned)(j - rj0) >= (unsigned)(rj1 - rj0)) sv[e] = -INFINITY;
-                }
+                for (int e = 0; e < 16; e++)
+                    if (KT * t + 8 * (e >> 2) + 4 * hh + (e & 3) >= T) sv[e] = -INFINITY;
             }
             // online softmax. The maxima move only when some query of the wave
             // would exceed its maximum by more than 2^8 (base 2): the
@@ -506,9 +479,9 @@ __global__ __launch_bounds__(256) void k_attn_split(SplitIn S, Planes P) {
         // rows: thread = row tid / 8, features DK/8 (tid % 8) .. of it
         constexpr int FPT = DK / 8;
         const bool isk = b < S.nk;
-        const unsigned tile = isk ? b : b - S.nk, per = isk ? P.ntile : P.nr;
+        const unsigned tile = isk ? b : b - S.nk, per = isk ? P.ntile : 2 * P.ntile;
         const int bh = (int)(tile / per), tt = (int)(tile % per), h = bh % H;
-        const int r = tid >> 3, row = isk ? 32 * tt + r : T + 32 * (tt + P.rb0) + r;
+        const int r = tid >> 3, row = isk ? 32 * tt + r : T + 32 * (tt - P.ntile) + r;
         const bool live = row >= 0 && row < (isk ? T : 2 * T - 1);
         const float *x = (isk ? S.k + (size_t)(bh / H) * T * d : S.rk) + (size_t)(live ? row : 0) * d + h * DK + FPT * (tid & 7);
         float y[FPT], a = 0.0f;
@@ -574,33 +547,18 @@ __global__ __launch_bounds__(256) void k_attn_split(SplitIn S, Planes P) {
 
 size_t al256(size_t b) { return (b + 255) / 256 * 256; }
 
-// the blocks of rk that the windows reach: offsets of query block bx and key
-// tile t are block t - bx (and the one before it)
-void rk_blocks(int T, int left, int right, int *rb0, int *nr) {
-    const int ntile = (T + KT - 1) / KT;
-    int lo = -ntile, hi = ntile - 1;
-    if (left >= 0) {
-        // a row t sees keys t - left - right .. t + right
-        const long a = ((long)left + right + KT - 1) / KT + 3, b = ((long)right + KT - 1) / KT + 2;
-        if (a < ntile) lo = (int)-a;
-        if (b < ntile - 1) hi = (int)b;
-    }
-    *rb0 = lo;
-    *nr = hi - lo + 1;
-}
-
-// the workspace: K planes and exponents, then rk's, then V's and scales
+// the workspace: K planes and exponents, then rk's (offsets of query block bx and
+// key tile t are block t - bx, and the one before it), then V's and scales
 struct SplitWs {
     size_t kp, ke, rp, re, vs, total;
-    int ntile, nr, rb0;
-    SplitWs(int T, int d, int H, int nseq, int left, int right) {
+    int ntile;
+    SplitWs(int T, int d, int H, int nseq) {
         ntile = (T + KT - 1) / KT;
-        rk_blocks(T, left, right, &rb0, &nr);
-        const size_t kt = (size_t)nseq * ntile;
+        const size_t kt = (size_t)nseq * ntile, nr = 2 * (size_t)ntile;
         kp = al256(kt * KT * d * 4);
         ke = al256(kt * KT * H * sizeof(int));
-        rp = al256((size_t)nr * KT * d * 4);
-        re = al256((size_t)nr * KT * H * sizeof(int));
+        rp = al256(nr * KT * d * 4);
+        re = al256(nr * KT * H * sizeof(int));
         vs = al256(kt * d * sizeof(float));
         total = 2 * kp + ke + rp + re + vs;
     }
@@ -608,10 +566,10 @@ struct SplitWs {
 
 template <int DK>
 hipError_t launch_dk(const float *q, const float *k, const float *v, const float *rk, const float *bu,
-                     const float *bv, float *ctx, int T, int d, int H, int left, int right, int nseq, void *ws,
-                     uint8_t *xp, float *xpf, hipStream_t st) {
+                     const float *bv, float *ctx, int T, int d, int H, int nseq, void *ws, uint8_t *xp, float *xpf,
+                     hipStream_t st) {
     if ((size_t)(2 * (size_t)T) * d >= 0x7fffffffu || !ws) return hipErrorInvalidValue;
-    const SplitWs W(T, d, H, nseq, left, right);
+    const SplitWs W(T, d, H, nseq);
     uint8_t *b = (uint8_t *)ws;
     Planes P{};
     P.k = (half8 *)b;
@@ -620,12 +578,12 @@ hipError_t launch_dk(const float *q, const float *k, const float *v, const float
     P.r = (half8 *)(b + 2 * W.kp + W.ke);
     P.re = (int *)(b + 2 * W.kp + W.ke + W.rp);
     P.vs = (float *)(b + 2 * W.kp + W.ke + W.rp + W.re);
-    P.ntile = W.ntile, P.nr = W.nr, P.rb0 = W.rb0;
+    P.ntile = W.ntile;
     P.xp = xp, P.xpf = xpf;
     SplitIn S{};
     S.k = k, S.rk = rk, S.v = v;
     S.T = T, S.d = d;
-    const size_t nk = (size_t)nseq * H * W.ntile, nrb = (size_t)H * W.nr;
+    const size_t nk = (size_t)nseq * H * W.ntile, nrb = (size_t)H * 2 * W.ntile;
     if (2 * nk + nrb > 0x7fffffffu) return hipErrorInvalidValue;
     S.nk = (unsigned)nk, S.nrb = (unsigned)nrb;
     hipLaunchKernelGGL(k_attn_split<DK>, dim3((unsigned)(2 * nk + nrb)), dim3(256), 0, st, S, P);
@@ -638,8 +596,8 @@ hipError_t launch_dk(const float *q, const float *k, const float *v, const float
     if (attr != hipSuccess) return attr;
     // exponentials are base 2: scores carry log2(e) / sqrt(DK)
     const float kscale = (1.0f / sqrtf((float)DK)) * 1.4426950408889634f;
-    hipLaunchKernelGGL((k_attn<DK>), dim3(P.ntile, H, nseq), dim3(64 * NW), bytes, st, q, bu, bv, ctx, T, d, left,
-                       right, kscale, P);
+    hipLaunchKernelGGL((k_attn<DK>), dim3(P.ntile, H, nseq), dim3(64 * NW), bytes, st, q, bu, bv, ctx, T, d, kscale,
+                       P);
     return hipGetLastError();
 }
 
@@ -647,9 +605,9 @@ hipError_t launch_dk(const float *q, const float *k, const float *v, const float
 
 bool mh_attn_supported(int dk) { return dk == 64 || dk == 128; }
 
-size_t mh_attn_ws_bytes(int T, int d, int H, int nseq, int left, int right) {
-    if (T <= 0 || nseq <= 0 || H <= 0) return 0;
-    return SplitWs(T, d, H, nseq, left, right).total;
+size_t mh_attn_ws_bytes(int T, int d, int H, int nseq, int left) {
+    if (left >= 0 || T <= 0 || nseq <= 0 || H <= 0) return 0;   // (chunked windows split nothing)
+    return SplitWs(T, d, H, nseq).total;
 }
 
 hipError_t mh_launch_relpos_attn(const float *q, const float *k, const float *v, const float *rk,
@@ -657,11 +615,13 @@ hipError_t mh_launch_relpos_attn(const float *q, const float *k, const float *v,
                                  int left, int right, int nseq, void *ws, uint8_t *xp, float *xpf,
                                  hipStream_t st) {
     const int dk = d / H;
-    if (dk == 128)
-        return launch_dk<128>(q, k, v, rk, bias_u, bias_v, ctx, T, d, H, left, right, nseq, ws, xp, xpf, st);
+    if (left >= 0)
+        return xp ? hipErrorInvalidValue
+                  : mh_launch_relpos_attn_win(q, k, v, rk, bias_u, bias_v, ctx, T, d, H, left, right, nseq, st);
+    if (dk == 128) return launch_dk<128>(q, k, v, rk, bias_u, bias_v, ctx, T, d, H, nseq, ws, xp, xpf, st);
     if (dk == 64 && !xp)
-        return launch_dk<64>(q, k, v, rk, bias_u, bias_v, ctx, T, d, H, left, right, nseq, ws, nullptr, nullptr, st);
+        return launch_dk<64>(q, k, v, rk, bias_u, bias_v, ctx, T, d, H, nseq, ws, nullptr, nullptr, st);
     return hipErrorInvalidValue;
 }
 
-bool mh_attn_preps_out(int d, int H) { return H > 0 && d / H == 128; }
+bool mh_attn_preps_out(int d, int H, int left) { return left < 0 && H > 0 && d / H == 128; }

@@ -103,7 +103,7 @@ struct Ctx {
     hipStream_t st = nullptr;
     DBuf x, y, h;
     DBuf att;    // the host-pointer attention call's q, k, v, rk, biases and ctx
-    DBuf attw;   // the attention core's workspace (K and rk split into f16 planes)
+    DBuf attw;   // full attention's workspace (K, rk and V split into f16 planes)
     DBuf aed;    // the AED decoder's caches and vectors
     DBuf enc;    // the encoder layer's activations
     DBuf ssb;    // the subsampling's activations
@@ -967,7 +967,7 @@ int encoder_layer_dev(Ctx *c, const mynah_asr_hip_enc_layer *L, float *x, int T,
         if (gemm_dev(c, L->relk_w, pe, rk, P, 0, st)) return -1;
     }
     {
-        const size_t wb = mh_attn_ws_bytes(T, d, H, nseq, left, right);
+        const size_t wb = mh_attn_ws_bytes(T, d, H, nseq, left);
         void *ws = wb ? c->attw.get(wb) : nullptr;
         if (wb && !ws) return fail("device buffer allocation failed");
         // the context as the output projection's prepared input (tagged ctx),
@@ -975,7 +975,7 @@ int encoder_layer_dev(Ctx *c, const mynah_asr_hip_enc_layer *L, float *x, int T,
         uint8_t *xp = nullptr;
         float *xpf = nullptr;
         c->pa.src = nullptr;
-        if (mh_attn_preps_out(d, H) && ln_preps(&L->o_w, 1, M, d)) {
+        if (mh_attn_preps_out(d, H, left) && ln_preps(&L->o_w, 1, M, d)) {
             size_t bs[3];
             prep_sizes(0, mh_mpad(M), d, bs);
             xp = (uint8_t *)c->pa.xp.get(bs[0]);
@@ -1295,7 +1295,7 @@ int mynah_asr_hip_relpos_attention_dev(const float *q, const float *k, const flo
                                        int H, int left, int right, int nseq, void *stream) {
     Ctx *c;
     if (begin(&c)) return -1;
-    note_capture(pick_stream(stream));   // the split workspace may grow
+    note_capture(pick_stream(stream));   // full attention's workspace may grow
     if (!q || !k || !v || !rk || !bias_u || !bias_v || !ctx || T < 0 || nseq < 0 || H <= 0 || d <= 0 ||
         d % H != 0)
         return fail("bad argument");
@@ -1307,7 +1307,7 @@ int mynah_asr_hip_relpos_attention_dev(const float *q, const float *k, const flo
     if (ctx == q || ctx == k || ctx == v) return fail("ctx may not alias q, k or v");
     if ((size_t)2 * T * d >= 0x7fffffffu) return fail("attention: 2 T d must stay below 2^31");
     if (T == 0 || nseq == 0) return 0;
-    const size_t wb = mh_attn_ws_bytes(T, d, H, nseq, left, right);
+    const size_t wb = mh_attn_ws_bytes(T, d, H, nseq, left);
     void *ws = wb ? c->attw.get(wb) : nullptr;
     if (wb && !ws) return fail("device buffer allocation failed");
     hipError_t e = mh_launch_relpos_attn(q, k, v, rk, bias_u, bias_v, ctx, T, d, H, left, right, nseq, ws,

@@ -394,6 +394,14 @@ template <int QT> constexpr float w_bpe() {
          : QT == QT_Q5_K ? 0.6875f : 0.82f;
 }
 
+// Compiler-level ordering of a wave's own LDS writes and reads (the LDS
+// executes one wave's operations in issue order).
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Products of few rows, K split over a workgroup's waves (gemm_ksplit.hip):
 // whether M rows of `jobs` products of W's shape take that form (prep: the
 // FFN's prepared output, as mh_launch_gemm_prep_out), and its launch

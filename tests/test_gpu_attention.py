@@ -2,12 +2,13 @@
 (mynah_asr_hip_relpos_attention_dev) against the oracle's float64 restatement
 of src/encoder.c:315-410 (full) and :220-313 (chunked-limited).
 
-Bar: |ctx - ref| <= 1e-4*|ref| + 1e-5*max|v| per element. The kernel computes
+Bar: |ctx - ref| <= 1e-4*|ref| + 1e-5*max|v| per element. The kernels compute
 in f32 like the reference, with another summation order and base-2
-exponentials (full attention forms its scores from f16 hi + lo splits of
-row-scaled operands, 22 bits of each row's maximum), so a context element near
-zero (a cancelling weighted sum of v) carries an absolute error of order
-1e-6 * max|v| — the scale term covers that.
+exponentials (full attention forms its products from f16 hi + lo splits of
+scaled operands, 22 bits of each row's, or V tile column's, maximum), so a
+context element near zero (a cancelling weighted sum of v) carries an absolute
+error of order 1e-6 * max|v| — the scale term covers that. A row of a chunked
+window depends on the keys it sees alone: bit for bit.
 Inputs: q, k, v, rk N(0, 1) and bias_u, bias_v N(0, 0.1), seeded.
 """
 import sys
@@ -86,7 +87,7 @@ def test_relpos_attention_fastconformer_segment(gpu):
 
 @pytest.mark.parametrize("d", [256, 128])
 def test_relpos_attention_many_segments(gpu, d):
-    """Enough segments for the eight-wave (128-row) kernel variant, dk 128 and 64."""
+    """More (query block, head, segment) workgroups than the chip holds at once, dk 128 and 64."""
     T, H, nseq = 200, 2, 128
     say("attention many segments", T, d, H, nseq)
     arrs = make(21 + d, T, d, nseq)
@@ -127,15 +128,123 @@ def test_relpos_attention_wide_row_scales(gpu, left, right):
     assert (err <= lim).all(), f"{int((err > lim).sum())} outside, worst ratio {(err / lim).max():.3g}"
 
 
-def test_relpos_attention_segments_independent(gpu):
+@pytest.mark.parametrize("left,right", [(-1, 0), (20, 6)])
+def test_relpos_attention_segments_independent(gpu, left, right):
     """A segment's context does not depend on the other segments of the call
     (bit-identical to running it alone)."""
     T, d, H = 97, 256, 2
-    for nseq in (3, 256):   # the four- and the eight-wave kernel
+    for nseq in (3, 256):   # fewer and more workgroups than the chip holds at once
         arrs = make(5, T, d, nseq)
-        many = run_gpu(gpu, arrs, T, d, H, -1, 0, nseq)
-        one = run_gpu(gpu, tuple(a[1:2] if a.ndim == 3 else a for a in arrs), T, d, H, -1, 0, 1)
+        many = run_gpu(gpu, arrs, T, d, H, left, right, nseq)
+        one = run_gpu(gpu, tuple(a[1:2] if a.ndim == 3 else a for a in arrs), T, d, H, left, right, 1)
         assert np.array_equal(many[1].view(np.uint32), one[0].view(np.uint32))
+
+
+@pytest.mark.parametrize("d,H", [(128, 2), (256, 2)], ids=["dk64", "dk128"])
+@pytest.mark.parametrize("left,right", [(0, 0), (4, 3), (70, 13), (0, 31)])
+def test_relpos_attention_hidden_keys(gpu, d, H, left, right):
+    """Keys outside a row's window, 2^20 (v) and 2^4 (k) times the visible ones,
+    in the same key tiles: the row's context keeps its bits, and its bar is
+    that of the values it sees."""
+    T, chunk = 150, right + 1
+    say("attention hidden keys", d, H, left, right)
+    arrs = make(91, T, d, 1)
+    plain = run_gpu(gpu, arrs, T, d, H, left, right, 1)[0]
+    for c in (0, (T // chunk) // 2, (T - 1) // chunk):
+        j0, j1 = max((c - left // chunk) * chunk, 0), min((c + 1) * chunk, T)
+        rows = slice(c * chunk, j1)
+        q, k, v, rk, bu, bv = (a.copy() for a in arrs)
+        hidden = np.ones(T, bool)
+        hidden[j0:j1] = False
+        v[0, hidden] *= np.float32(2.0 ** 20)
+        k[0, hidden] *= np.float32(16.0)
+        got = run_gpu(gpu, (q, k, v, rk, bu, bv), T, d, H, left, right, 1)[0]
+        assert np.array_equal(got[rows].view(np.uint32), plain[rows].view(np.uint32)), f"chunk {c}"
+        ref = relpos_attention(q[0], k[0], v[0], rk, bu, bv, H, left, right)[rows]
+        lim = RTOL * np.abs(ref) + VTOL * np.abs(v[0, j0:j1]).max()
+        assert (np.abs(got[rows] - ref) <= lim).all(), f"chunk {c}"
+
+
+def _window_calls(gpu, torch, n, T, d, H, nseq):
+    """n sets of inputs on the GPU, and the call of set i on a stream."""
+    sets, out = [], []
+    for i in range(n):
+        sets.append([torch.from_numpy(a).cuda() for a in make(200 + i, T, d, nseq)])
+        out.append(torch.zeros((nseq, T, d), dtype=torch.float32, device="cuda"))
+
+    def call(i, stream):
+        M.relpos_attention_dev(gpu, *(a.data_ptr() for a in sets[i]), out[i].data_ptr(), T, d, H, 70, 13, nseq,
+                               stream=stream.cuda_stream)
+    return call, out, sets
+
+
+def test_relpos_attention_window_on_two_streams(gpu):
+    """Chunked-window calls of one thread on two streams, not ordered with each
+    other, give the bits of the calls alone."""
+    import torch
+    say("attention windows on two streams")
+    call, out, _sets = _window_calls(gpu, torch, 2, 750, 1024, 8, 4)
+    ss = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    alone = []
+    for i in range(2):
+        call(i, ss[0])
+        torch.cuda.synchronize()
+        alone.append(out[i].clone())
+        out[i].zero_()
+    torch.cuda.synchronize()
+    for rep in range(10):
+        for i in range(2):
+            call(i, ss[i])
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert torch.equal(out[i].view(torch.int32), alone[i].view(torch.int32))
+
+
+def test_relpos_attention_window_captured(gpu):
+    """Chunked-window calls larger than any before them in their thread are
+    captured (nothing is allocated), and two such graphs replayed at once on two
+    streams give the eager calls' bits, replay after replay."""
+    import threading
+    import torch
+    say("attention windows captured")
+    call, out, _sets = _window_calls(gpu, torch, 2, 600, 512, 4, 4)
+    small, _o, _s = _window_calls(gpu, torch, 1, 1, 256, 2, 1)
+    graphs, errs = [], []
+    ss = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+
+    def capture():
+        try:
+            small(0, ss[0])   # (the thread's first call)
+            torch.cuda.synchronize()
+            for i in range(2):
+                g = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(g, stream=ss[i]):
+                    call(i, torch.cuda.current_stream())
+                graphs.append(g)
+        except Exception as e:   # (reported by the test's own thread)
+            errs.append(e)
+
+    t = threading.Thread(target=capture)
+    t.start()
+    t.join()
+    assert not errs, errs
+    eager = []
+    for i in range(2):
+        call(i, ss[0])
+        torch.cuda.synchronize()
+        eager.append(out[i].clone())
+    for rep in range(3):
+        for o in out:
+            o.zero_()
+        torch.cuda.synchronize()
+        for i in range(2):
+            with torch.cuda.stream(ss[i]):
+                graphs[i].replay()
+        torch.cuda.synchronize()
+        for i in range(2):
+            assert torch.equal(out[i].view(torch.int32), eager[i].view(torch.int32)), f"replay {rep}, graph {i}"
 
 
 def test_relpos_attention_host_entry(gpu):
