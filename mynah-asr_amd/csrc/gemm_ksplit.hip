@@ -328,21 +328,39 @@ hipError_t ks_dispatch(const GemmJobs &J, const uint8_t *xp, const float *xs16, 
 
 }  // namespace
 
-// By the number of 32 x 32 output tiles. Q8_0, this form against k_gemm (us):
-//   1024 -> 1024   250 rows (256 tiles) 4.9 / 12.2   1004 (1024) 10.3 / 11.2   1500 (1504) 14.6 / 14.0
-//   1024 -> 4096    64 rows (256 tiles) 4.9 / 12.8    250 (1024) 10.3 / 11.1    384 (1536) 14.3 / 14.5
-//    512 -> 2048   384 rows (768 tiles) 6.7 / 7.5     512 (1024) 7.8 / 7.7      750 (1536) 10.3 / 9.2
-//   4096 -> 1024    64 rows (64 tiles) 10.5 / 32.2   1004 (1024) 31.8 / 39.8   1500 (1504) 44.4 / 43.8
-//   2048 -> 512   1500 rows (752 tiles) 13.3 / 18.3  2200 (1104) 19.7 / 23.3   3000 (1504) 23.8 / 24.9
-// so up to 1024 tiles, and up to 1408 for K of 16 chunks or more, where
-// k_gemm's chains are longest. The prepared output (32 x 128 tiles, SiLU and
-// split as the epilogue) wins up to 128 such workgroups: 1024 -> 4096 at 64 rows
-// 14 / 18 us with its preparation, at 128 rows 15.1 / 16.2, at 192 rows 16.9 / 14.9.
-bool mh_use_gemm_ks(const DevW &W, int M, int jobs, bool prep) {
+// By the number of 32 x 32 output tiles, the chunks of K and the format. A CU
+// runs tiles two at a time, so the time steps every 256 tiles; K of fewer than
+// eight chunks leaves waves idle, and of ten leaves most of them idle every second
+// round. Where an element costs the most instructions k_gemm's chains are longest:
+// the super-block formats leave later than the others (with one term per element,
+// INT8ACT, so do the rest from eight chunks on; so do f32 weights of 8 to 15 chunks
+// when they are more than two XCDs' L2 or of a chunk count that is no power of
+// two, where k_gemm waits for their planes). This form / k_gemm, us, Q8_0 and Q6_K:
+//    256 -> 1024   251 rows (256 tiles)  3.7 / 4.5   4.0 / 5.2     763 (768)  6.2 / 4.9   6.7 / 5.5
+//    512 -> 2048   251 rows (512 tiles)  5.2 / 6.6   5.6 / 7.7     379 (768)  7.0 / 6.9   7.5 / 8.0
+//                  507 rows (1024)       8.2 / 7.2   8.9 / 8.1
+//   1024 -> 1024   763 rows (768 tiles)  9.6 / 10.4  10.4 / 12.7  1019 (1024) 11.0 / 10.6 12.3 / 12.8
+//   1280 -> 1280   507 rows (640 tiles)  0.90 / 1    0.85 / 1      660 (840)  1.03 / 1    0.99 / 1
+//   2048 -> 512   2555 rows (1280)      21.4 / 23.0  24.2 / 29.9  2811 (1408) 24.1 / 23.6 27.2 / 30.2
+//   4096 -> 1024  1275 rows (1280)      39.8 / 43.2  44.4 / 56.3  1403 (1408) 49.5 / 44.0 51.4 / 56.3
+// The other formats of each kind lie within 8% of these ratios. f32 weights: 1024 ->
+// 4096 at 251 rows (1024 tiles) 13.8 / 18.6, 1280 -> 1280 at 660 (840) 16.3 / 22.0,
+// but 1024 -> 2048 at 507 (1024) 13.2 / 12.6, 1024 -> 1024 at 1019 (1024) 13.8 / 12.9.
+// The prepared output (32 x 128 tiles, SiLU and split as the epilogue) wins while a
+// CU has one such workgroup: the whole FFN 1024 -> 4096 at 125 rows (128) 25.3 /
+// 30.1, at 253 rows (256) 28.2 / 32.9, at 317 rows (320) 41.1 / 38.1; 0.77 to 0.93
+// of it in every format up to 256.
+bool mh_use_gemm_ks(int qtype, const DevW &W, int M, int jobs, bool prep, bool a1) {
     const long rows = (M + 31) / 32, Kc = W.Kp / 128;
-    if (prep) return mh_mpad(M) / 32 * (W.Np / 128) <= 128;
-    const long tiles = rows * (W.Np / 32) * jobs;
-    return tiles <= 1024 || (Kc >= 16 && tiles <= 1408);
+    if (prep) return mh_mpad(M) / 32 * (W.Np / 128) <= 256;
+    const bool super_blocks = qtype == QT_Q2_K || qtype == QT_Q3_K || qtype == QT_Q4_K || qtype == QT_Q5_K || qtype == QT_Q6_K;
+    const bool late = super_blocks || (a1 && Kc >= 8);
+    const bool f32_late = qtype == QT_F32 && (Kc > 8 || 4L * W.Np * W.Kp * jobs > 9000000);
+    const long most = Kc < 4   ? 256
+                      : Kc < 8 ? (late ? 768 : 512)
+                      : Kc < 16 ? (late || f32_late ? 1024 : Kc == 10 ? 640 : 768)
+                                : (late ? 1408 : 1280);
+    return rows * (W.Np / 32) * jobs <= most;
 }
 
 hipError_t mh_launch_gemm_ks(int qtype, const GemmJobs &J, const uint8_t *xp, const float *xs16, const float *xpf, int M,

@@ -1795,7 +1795,8 @@ static hipError_t gemm_launch(const GemmJobs &J, const uint8_t *xp, const float 
     const int ngrp = gemm_ngroups(w_bpe<QT>() * W.Np * W.Kp * J.n, (A1 ? 2.0f : 4.0f) * mpad * W.Kp, tilesM,
                                   J.n * tilesN);
     if (po && (po->Kc != tilesN || J.n != 1)) return hipErrorInvalidValue;
-    if (mh_use_gemm_ks(W, M, J.n, po != nullptr)) return mh_launch_gemm_ks(QT, J, xp, xs16, xpf, M, act, po, A1, st);
+    if (mh_use_gemm_ks(QT, W, M, J.n, po != nullptr, A1))
+        return mh_launch_gemm_ks(QT, J, xp, xs16, xpf, M, act, po, A1, st);
     if (po) {
         if constexpr (A1) {
             return hipErrorInvalidValue;

@@ -403,9 +403,9 @@ __device__ __forceinline__ void wave_lds_order() {
 }
 
 // Products of few rows, K split over a workgroup's waves (gemm_ksplit.hip):
-// whether M rows of `jobs` products of W's shape take that form (prep: the
-// FFN's prepared output, as mh_launch_gemm_prep_out), and its launch
-bool mh_use_gemm_ks(const DevW &W, int M, int jobs, bool prep);
+// whether M rows of `jobs` products of W's shape and format take that form (prep:
+// the FFN's prepared output, as mh_launch_gemm_prep_out; a1: INT8ACT), and its launch
+bool mh_use_gemm_ks(int qtype, const DevW &W, int M, int jobs, bool prep, bool a1);
 hipError_t mh_launch_gemm_ks(int qtype, const GemmJobs &J, const uint8_t *xp, const float *xs16, const float *xpf, int M,
                              int act, const PrepOut *po, bool a1, hipStream_t st);
 

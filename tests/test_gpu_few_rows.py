@@ -63,6 +63,19 @@ def test_rounds_and_ragged_columns(gpu, n, k):
     _check(gpu, M.Q8_0, n, k, 1600 if n > 512 else 12100, [17, 64, 65, 750], act=1)
 
 
+# the row counts on both sides of each line of the rule that chooses this form
+# (256, 512, 640, 768, 1024, 1280, 1408 tiles of 32 x 32 by K and format)
+EDGES = [(1024, 256, [256, 257]), (1024, 512, [512, 513, 768, 769]), (1024, 1024, [768, 769, 1024, 1025]),
+         (640, 1280, [1024, 1025, 1632, 1633]), (1024, 2048, [1280, 1281, 1408, 1409])]
+
+
+@pytest.mark.parametrize("qt", [M.F32, M.INT4, M.Q8_0, M.Q4_K, M.Q6_K], ids=lambda q: M.NAMES[q])
+@pytest.mark.parametrize("n,k,rows", EDGES, ids=lambda v: str(v) if isinstance(v, int) else "")
+def test_rows_at_the_rules_edges(gpu, qt, n, k, rows):
+    say("few rows, rule edges", M.NAMES[qt], k, "->", n)
+    _check(gpu, qt, n, k, 2200, rows)
+
+
 @pytest.mark.parametrize("qt", [M.Q4_0, M.Q8_0, M.Q2_K, M.Q5_K, M.Q6_K], ids=lambda q: M.NAMES[q])
 def test_int8_activation_rows(gpu, qt):
     say("few rows, int8 activations", M.NAMES[qt])
@@ -79,7 +92,7 @@ def test_ffn_hand_off(gpu, q1, q2):
     """The prepared hand-off against the larger FFN's (k_gemm's epilogue)."""
     import torch
     say("few rows FFN", M.NAMES[q1], M.NAMES[q2])
-    d, f, big = 512, 1024, 700
+    d, f, big = 512, 1024, 2100   # (256 workgroups of the prepared output at 1024 rows)
     w1 = M.DeviceWeight(gpu, M.Weight.make(gpu, q1, gpu.randn(5, 0.05, (f, d))))
     w2 = M.DeviceWeight(gpu, M.Weight.make(gpu, q2, gpu.randn(6, 0.05, (d, f))))
     x = torch.from_numpy(gpu.randn(7, 1.0, (big, d))).cuda()
@@ -95,7 +108,7 @@ def test_ffn_hand_off(gpu, q1, q2):
     try:
         ref = _bits(ffn(big))
         assert np.isfinite(ref.view(np.float32)).all()
-        for m in (17, 64, 65, 250, 512, 513):
+        for m in (17, 64, 65, 250, 512, 513, 1024, 1025):
             assert np.array_equal(_bits(ffn(m)), ref[:m]), f"M={m}"
     finally:
         w1.close()
