@@ -172,6 +172,45 @@ def test_aed_given_tokens(gpu, orc, qt, ffn, n):
     dev.close()
 
 
+# the row counts that take other kernels: the one-row and 8- and 16-row GEMV, the
+# GEMM from 17, one and two 32-row tiles, one and two batches of 64 and the third's
+# first row, one and more splits of 64 keys
+@pytest.mark.parametrize("qt,ffn", [(M.Q8_0, 512), (M.Q4_K, 2048), (M.F32, 256)])
+def test_aed_scored_rows_do_not_depend_on_the_batch(gpu, qt, ffn):
+    """The first n of 150 scored tokens, scored alone: the same bits."""
+    import torch
+    say("aed rows of a batch", M.NAMES[qt], ffn)
+    d, H, vocab, T = 256, 4, 300, 70
+    dev = M.DeviceAed(gpu, make_params(31 + ffn, d, H, ffn, vocab, 2, 150), H, qt)
+    denc = torch.from_numpy(np.random.default_rng(19).standard_normal((T, d)).astype(np.float32)).cuda()
+    toks = [int(t) for t in np.random.default_rng(20).integers(0, vocab, 150)]
+    full = dev.forced(denc.data_ptr(), T, toks).view(np.uint32)
+    for n in (1, 2, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 149):
+        part = dev.forced(denc.data_ptr(), T, toks[:n]).view(np.uint32)
+        assert np.array_equal(part, full[:n]), f"{n} tokens"
+    dev.close()
+
+
+@pytest.mark.parametrize("qt,ffn,n", [(M.Q8_0, 512, 4), (M.Q4_K, 2048, 1), (M.F32, 256, 70)])
+def test_aed_decoded_tokens_lead_their_scores(gpu, qt, ffn, n):
+    """Each greedy token is the argmax of its position's scored logits. Decoding
+    and scoring sum their layer norms in other orders, so a near tie (the bar of
+    the logits) may go either way."""
+    import torch
+    say("aed decoded against scored", M.NAMES[qt], ffn, n)
+    d, H, vocab, T, cap = 256, 4, 300, 70, 40
+    dev = M.DeviceAed(gpu, make_params(57 + ffn, d, H, ffn, vocab, 2, n + cap), H, qt)
+    denc = torch.from_numpy(np.random.default_rng(23).standard_normal((T, d)).astype(np.float32)).cuda()
+    prompt = [int(t) for t in np.random.default_rng(24).integers(0, vocab, n)]
+    out = dev.decode(denc.data_ptr(), T, prompt, eos=-1, cap=cap)
+    assert len(out) == cap
+    lg = dev.forced(denc.data_ptr(), T, prompt + out)[n - 1:-1]
+    for i, (row, tok) in enumerate(zip(lg, out)):
+        tol = 1e-4 * np.abs(row).max() + 1e-5 * np.sqrt((row ** 2).mean())
+        assert row[tok] >= row.max() - tol, f"token {i}: {tok} against {int(row.argmax())}"
+    dev.close()
+
+
 def test_aed_rejects_unsupported(gpu):
     import torch
     params = make_params(1, 96, 1, 128, 100, 1, 8)   # head size 96
