@@ -308,6 +308,62 @@ def test_encoder_layer_in_other_numerics(gpu, mode):
         dev.close()
 
 
+# ff1 and ff2 of two formats: in QMAT numerics at T nseq <= 16 one of an FFN's
+# products takes the int8 path and the other is EXACT, in either order
+MIXED = {"ff1_w2": M.Q8_0, "ff2_w1": M.Q8_0}
+
+
+@pytest.mark.parametrize("bn", [True, False], ids=["bn", "ln"])
+@pytest.mark.parametrize("qt,other,mode,T,nseq", [
+    (M.INT8, {}, M.INT8ACT, 40, 2), (M.INT4, {}, M.INT8ACT, 40, 2), (M.INT8, MIXED, M.INT8ACT, 40, 2),
+    (M.INT8, {}, M.QMAT, 8, 2), (M.INT4, {}, M.QMAT, 5, 3), (M.INT8, MIXED, M.QMAT, 8, 2),
+    (M.INT4, MIXED, M.QMAT, 16, 1)],
+    ids=["int8-int8act", "int4-int8act", "mixed-int8act", "int8-qmat", "int4-qmat", "int8-mixed-qmat", "int4-mixed-qmat"])
+def test_encoder_layer_biases_in_int8_products(gpu, qt, other, mode, T, nseq, bn):
+    """Biased layers whose products run on the int8 path (bias, then SiLU, as
+    passes of their own behind it): within the int8 path's budget of the EXACT
+    layer (relative L2 < 1e-2). Each bias left out of the EXACT layer moves it by
+    more than that budget and the int8 path's own error together, so a bias lost
+    here would show. The k bias has no such check: it adds one constant to all of
+    a row's scores, which the softmax takes out."""
+    import torch
+    say("encoder layer, biases in int8 products", M.NAMES[qt], sorted(other), mode, T, nseq, bn)
+    d, H, f, k = 256, 4, 512, 9
+    p = make_params(26, d, f, k, True, bn)
+    names = [f"{n}_b{i}" for n in ("ff1", "ff2") for i in (1, 2)] + ["q_b", "v_b", "o_b", "pw1_b", "pw2_b"]
+    for n in names:
+        p[n] = p[n] * np.float32(30.0 if n == "q_b" else 5.0)
+    dev = M.DeviceEncoderLayer(gpu, p, qt)
+    for n, q in other.items():
+        w = M.DeviceWeight(gpu, M.Weight.make(gpu, q, p[n]))
+        dev._keep.append(w)
+        setattr(dev.c, n, w.h)
+    x = np.random.default_rng(27).standard_normal((nseq * T, d)).astype(np.float32)
+    ped = torch.from_numpy(E.pos_emb(T, d).astype(np.float32)).cuda()
+
+    def run(m):
+        assert gpu.set_numerics(m) == m
+        xd = torch.from_numpy(x).cuda()
+        dev.run(xd.data_ptr(), T, nseq, ped.data_ptr(), d, H, k, 0)
+        torch.cuda.synchronize()
+        return xd.cpu().numpy()
+    try:
+        ex, y = run(M.EXACT), run(mode)
+        rel = float(np.linalg.norm(y - ex) / np.linalg.norm(ex))
+        say(f"  relative L2 vs EXACT {rel:.3g}")
+        assert np.isfinite(y).all() and 0 < rel < 1e-2
+        for n in names:
+            ptr = getattr(dev.c, n)
+            setattr(dev.c, n, None)
+            off = float(np.linalg.norm(run(M.EXACT) - ex) / np.linalg.norm(ex))
+            setattr(dev.c, n, ptr)
+            say(f"  without {n}: {off:.3g}")
+            assert off > 1e-2 + rel, n
+    finally:
+        gpu.set_numerics(M.EXACT)
+        dev.close()
+
+
 @pytest.mark.parametrize("k", [1, 3, 8, 9, 15, 16])
 @pytest.mark.parametrize("T,nseq", [(7, 2), (8, 1), (33, 1), (97, 1), (66, 96)],
                          ids=["T7x2", "T8", "T33", "T97", "T66x96"])
