@@ -14,11 +14,17 @@
 // keys it sees and on nothing else; calls on several streams share nothing, and a
 // call under stream capture allocates nothing.
 // Not on full attention's f16 hi + lo operands (attention.hip): [70, 13], 16 x 750
-// frames, d 1024, 8 heads take 131 us there and 166 here (a layer of 4 x 251
-// frames 281 us either way), but its V split has one exponent per 32 keys and
+// frames, d 1024, 8 heads take 134 us there and 172 here (a layer of 4 x 251
+// frames 287 and 297 us), but its V split has one exponent per 32 keys and
 // feature, so keys that a row does not see take bits from those it does (hidden
 // rows 2^20 times larger: off by more than the header's bound), and its planes
 // need a workspace, which calls on two streams, or replays of two graphs, share.
+//
+// Sums. A score is two sums of DK / 2 products, added; a tile's P . V is summed
+// from zero and then joins the context. Relative error against 64 bits (2-norm,
+// N(0, 1) inputs) at [70, 13], 750 frames, d 1024, 8 heads: 2.8e-7, with one chain
+// each 4.2e-7 (3.1e-7 on the split operands); at [200, 50], 1000 frames, d 512
+// 3.2e-7, 5.1e-7 (3.5e-7). It costs 3% of the call.
 //
 // One workgroup = two waves = 32 query rows of one head of one segment; wave w
 // owns rows t0 + 16w .. +15 (wider blocks visit more keys that their rows cannot
@@ -37,7 +43,7 @@
 //   4. runs an online softmax (running row max and sum, base-2 exponentials of
 //      scores pre-scaled by log2(e)/sqrt(DK)), and
 //   5. multiplies the probabilities (re-laid out as an MFMA A operand through
-//      LDS) by the V tile into its 16 x DK context accumulator.
+//      LDS) by the V tile and adds that to its 16 x DK context, rescaled.
 //
 // MFMA 16x16x4 f32 operand layout (lane l, c = l & 15, g = l >> 4):
 //   A: row c, k-slot g;  B: column c, k-slot g;  D: rows 4g + e (e = 0..3), column c.
@@ -230,12 +236,14 @@ __global__ __launch_bounds__(NTH, 1) void k_attn_win(const float *__restrict__ q
         }
         __syncthreads();
         const float *rw = Rs + ((prow + 16 + c) % NB) * L::KS + NS * g;
+        f4 cp[2] = {carry, carry};
 #pragma unroll
         for (int i = 0; i < NS / 4; i++) {
             const f4 rx = *(const f4 *)(rw + 4 * i);
 #pragma unroll
-            for (int u = 0; u < 4; u++) carry = mfma16(qb[4 * i + u], rx[u], carry);
+            for (int u = 0; u < 4; u++) cp[i / (NS / 8)] = mfma16(qb[4 * i + u], rx[u], cp[i / (NS / 8)]);
         }
+        carry = cp[0] + cp[1];
         gload(ja, 1);
     }
 
@@ -251,8 +259,11 @@ __global__ __launch_bounds__(NTH, 1) void k_attn_win(const float *__restrict__ q
         if (jt + KT < jb) gload(jt + KT, ti + 1);
 
         // 1. content scores (16 rows x 32 keys), 2. position tiles D1, D2
-        f4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-        f4 bd[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        f4 sp[2][2], bp[2][2];   // [half of the features][tile of 16]
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int n = 0; n < 2; n++) sp[h][n] = bp[h][n] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < NS / 4; i++) {
             f4 kx[2], rx[2];
@@ -262,12 +273,15 @@ __global__ __launch_bounds__(NTH, 1) void k_attn_win(const float *__restrict__ q
             for (int n = 0; n < 2; n++) rx[n] = *(const f4 *)(Rs + rr[n] * L::KS + NS * g + 4 * i);
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                s[0] = mfma16(qa[4 * i + u], kx[0][u], s[0]);
-                s[1] = mfma16(qa[4 * i + u], kx[1][u], s[1]);
-                bd[0] = mfma16(qb[4 * i + u], rx[0][u], bd[0]);
-                bd[1] = mfma16(qb[4 * i + u], rx[1][u], bd[1]);
+                const int h = i / (NS / 8);
+                sp[h][0] = mfma16(qa[4 * i + u], kx[0][u], sp[h][0]);
+                sp[h][1] = mfma16(qa[4 * i + u], kx[1][u], sp[h][1]);
+                bp[h][0] = mfma16(qb[4 * i + u], rx[0][u], bp[h][0]);
+                bp[h][1] = mfma16(qb[4 * i + u], rx[1][u], bp[h][1]);
             }
         }
+        const f4 s[2] = {sp[0][0] + sp[1][0], sp[0][1] + sp[1][1]};
+        const f4 bd[2] = {bp[0][0] + bp[1][0], bp[0][1] + bp[1][1]};
         // 3. rel-shift: row i = 4g + e, key jj = 16n + c takes band column jj - i + 15
         //    (delta = jt + jj - (tw + i) = b + (jj - i + 15))
 #pragma unroll
@@ -299,10 +313,6 @@ __global__ __launch_bounds__(NTH, 1) void k_attn_win(const float *__restrict__ q
             sv[1][e] = exp2f(sv[1][e] - mn);
             l[e] = l[e] * alpha[e] + sum16(sv[0][e] + sv[1][e]);
         }
-#pragma unroll
-        for (int n = 0; n < NT; n++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[n][e] *= alpha[e];
         // 5. probabilities to the A layout (row c, keys 8g .. 8g+7), then P . V
         wave_lds_order();   // the band reads above precede these writes
 #pragma unroll
@@ -325,8 +335,11 @@ __global__ __launch_bounds__(NTH, 1) void k_attn_win(const float *__restrict__ q
         for (int n = 0; n < NT; n++) {
             if (n + 1 < NT) rdv(n + 1, vb[(n + 1) & 1]);
             const f4 *vx = vb[n & 1];
+            f4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int u = 0; u < 8; u++) acc[n] = mfma16(pa[u], vx[u >> 2][u & 3], acc[n]);
+            for (int u = 0; u < 8; u++) o = mfma16(pa[u], vx[u >> 2][u & 3], o);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[n][e] = fmaf(acc[n][e], alpha[e], o[e]);
         }
     }
 #pragma unroll
