@@ -182,8 +182,8 @@ int mynah_asr_hip_qqkv_dev(const mynah_asr_hip_weight *wq, const mynah_asr_hip_w
  * forbid hipMalloc). No counterpart in the reference. The same product and
  * the same bits as mynah_asr_hip_qgemm_dev; the prepared input goes to a
  * 32 MiB device array that each GPU holds from the library's first such call
- * until the process ends, and K is never split over workgroups (the split-K
- * launches need a workspace of their own). `stream` is used as given (NULL =
+ * until the process ends, and K is never split over workgroups (qgemm_dev does
+ * so for few rows and long K, in a workspace). `stream` is used as given (NULL =
  * the null stream; no per-thread stream is created). Returns -1 when the
  * prepared input of T rows does not fit the 32 MiB (see
  * mynah_asr_hip_noalloc_bytes). Every call on one GPU shares that GPU's

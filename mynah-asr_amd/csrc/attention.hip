@@ -37,10 +37,13 @@
 //   5. multiplies the probabilities, already the MFMA's A operand (V's fragments
 //      hold a tile's keys in that order), by the V tile into the context.
 // What bounds it: the fragments, 48 KiB per wave and tile (DK 128) through the
-// 64 B/clk L1 path (6100 of the 7900 cycles that eight waves of a CU take for a
+// 64 B/clk L1 path (6100 of the 7800 cycles that eight waves of a CU take for a
 // tile each), then the MFMAs (72 of 32 cycles, 4600 cycles on each SIMD) and
-// about 400 VALU instructions; of a workgroup's 65 000 cycles at T = 750, 10 000
-// prepare the rows and load the first operands and 4500 join the contexts.
+// about 400 VALU instructions. At T = 750 a workgroup takes 65 100 cycles: 13 750
+// until its first tile (rows, first operands and position block), 46 500 for the
+// tiles, 4600 to join the contexts. The chip holds 1.73 to 1.83 GHz meanwhile, so
+// the six rounds of 512 workgroups of 16 x 750 frames are 220 of the kernel's 240
+// us; the rest is their start and end.
 // Measured, d 1024, 8 heads, full window, with the splits: 16 x 750 frames 430 ->
 // 275 us, 1 x 750 118 -> 36, 1 x 63 28 -> 13 (before: 128-row blocks staging K, V
 // and rk in LDS). No faster, each measured: eight waves per workgroup (15% slower

@@ -447,7 +447,7 @@ struct AedBufs {
 };
 // Given positions per batch: two 32-row tiles, so one pass over the weights
 // serves 64 positions; more would only grow the scratch (the splits of a batch
-// take at most as many floats as one layer's cross K). One position at a time
+// take max(T, max_len), rounded up to 64, times d floats). One position at a time
 // costs 244 us (4 layers of 1024, ffn 4096: a chain of 38 launches), scoring
 // 27 positions in batches 0.4 ms instead of 6.6.
 constexpr int kAedRows = 64;
@@ -812,9 +812,9 @@ size_t noalloc_need(const mynah_asr_hip_weight *W, int T, size_t *o_xs16, size_t
     return xp + xs16 + xpf;
 }
 
-// qgemm_dev's product with its prepared input in `scratch` and K unsplit (the
-// split-K launches need a workspace of their own): the same kernels on the
-// same data, so the same bits.
+// qgemm_dev's product with its prepared input in `scratch`, and a GEMV's K in one
+// launch (its split over workgroups needs a workspace): the same operations on
+// the same data, so the same bits.
 int gemm_noalloc(const mynah_asr_hip_weight *W, const float *dx, float *dy, int T, int act, hipStream_t st) {
     size_t o_xs16 = 0, o_xpf = 0;
     const size_t need = noalloc_need(W, T, &o_xs16, &o_xpf);

@@ -22,11 +22,11 @@
 
 namespace {
 
-// PC waves side by side over columns, S = 8 / PC over chunks; each wave WM x WN
-// groups of 32 x 32.
-template <int QT, bool A1, int WM, int WN, int PC> struct KsTile {
+// PC waves side by side over columns, S = 8 / PC over chunks; each wave 32 rows by
+// WN groups of 32 columns.
+template <int QT, int WN, int PC> struct KsTile {
     static constexpr int NW = 8, S = NW / PC, NT = 64 * NW;
-    static constexpr int TR = 32 * WM, TC = 32 * WN * PC;
+    static constexpr int TR = 32, TC = 32 * WN * PC;
     static constexpr int TCS = TC + 8;    // LDS row stride: the two lane halves' rows (4 apart) fall in different banks
     // ksteps of operands in flight per wave: two for the 32 x 32 tile, so that
     // two workgroups share a CU (128 registers)
@@ -34,16 +34,16 @@ template <int QT, bool A1, int WM, int WN, int PC> struct KsTile {
     static constexpr size_t LDS = (size_t)S * TR * TCS * 4 + (size_t)S * TR * 4;
 };
 
-template <int QT, int EPI, bool A1, int WM, int WN, int PC>
-__global__ __launch_bounds__(512, (WM * WN == 1 ? 4 : 2)) void k_gemm_ks(GemmJobs J, const uint8_t *__restrict__ xp,
+template <int QT, int EPI, bool A1, int WN, int PC>
+__global__ __launch_bounds__(512, (WN == 1 ? 4 : 2)) void k_gemm_ks(GemmJobs J, const uint8_t *__restrict__ xp,
                                                     const uint8_t *__restrict__ xm, const float *__restrict__ xpf, int M,
                                                     int act, int tilesM, int tilesN, int pr, PrepOut po) {
     using F = Fmt<QT>;
-    using L = KsTile<QT, A1, WM, WN, PC>;
+    using L = KsTile<QT, WN, PC>;
     constexpr int S = L::S, TR = L::TR, TC = L::TC, TCS = L::TCS, NT = L::NT, PF = L::PF;
     constexpr int TERMS = A1 ? 1 : 2;
     constexpr bool HALVES = A1 && QT == QT_Q5_K;   // (as in k_gemm)
-    static_assert(EPI != EPI_PREP || (TC == 128 && TR == 32 && !A1), "the prepared output is one chunk of 32 rows");
+    static_assert(EPI != EPI_PREP || (TC == 128 && !A1), "the prepared output is one chunk of 32 rows");
     extern __shared__ __attribute__((aligned(16))) float lds[];
     float *part = lds, *pfs = lds + S * TR * TCS;
     // The tiles of a launch as 8 rectangles of (row band, column tile), one per
@@ -62,33 +62,29 @@ __global__ __launch_bounds__(512, (WM * WN == 1 ? 4 : 2)) void k_gemm_ks(GemmJob
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hh = lane >> 5, col = lane & 31;
     const int pcI = wave % PC, s = wave / PC;
-    const int Kc = W.Kp / 128, G0 = tm * WM;
+    const int Kc = W.Kp / 128;
     int gn[WN];
 #pragma unroll
     for (int j = 0; j < WN; j++) gn[j] = (tn * PC + pcI) * WN + j;
 
-    AK<WM> a[PF];
+    AK<1> a[PF];
     BK<QT, WN> b[PF];
     BH<QT, WN> hd;
-    half8 xmv[WM];
+    half8 xmv = {};
     float pf = 0.0f;
-    auto load_k = [&](int c, int sl, AK<WM> &aa, BK<QT, WN> &bb) {
+    auto load_k = [&](int c, int sl, AK<1> &aa, BK<QT, WN> &bb) {
         load_bk<QT, WN>(W, Kc, gn, c, sl, lane, bb);
 #pragma unroll
-        for (int i = 0; i < WM; i++)
-#pragma unroll
-            for (int kh = 0; kh < 2; kh++) {
-                const uint8_t *p = xp + ((((size_t)(G0 + i) * Kc + c) * HSTEPS + 2 * sl + kh) * TERMS * 64 + lane) * 16;
-                aa.h[i][kh] = *(const half8 *)p;
-                if constexpr (!A1) aa.l[i][kh] = *(const half8 *)(p + 1024);
-            }
+        for (int kh = 0; kh < 2; kh++) {
+            const uint8_t *p = xp + ((((size_t)tm * Kc + c) * HSTEPS + 2 * sl + kh) * TERMS * 64 + lane) * 16;
+            aa.h[0][kh] = *(const half8 *)p;
+            if constexpr (!A1) aa.l[0][kh] = *(const half8 *)(p + 1024);
+        }
     };
     auto load_h = [&](int c) {
         load_bh<QT, WN>(W, Kc, gn, c, lane, hd);
-        if constexpr (F::MINS)
-#pragma unroll
-            for (int i = 0; i < WM; i++) xmv[i] = *(const half8 *)(xm + (((size_t)(G0 + i) * Kc + c) * 64 + lane) * 16);
-        if (pcI == 0 && lane < TR) pf = xpf[((size_t)(G0 + (lane >> 5)) * Kc + c) * 32 + col];
+        if constexpr (F::MINS) xmv = *(const half8 *)(xm + (((size_t)tm * Kc + c) * 64 + lane) * 16);
+        if (pcI == 0 && lane < TR) pf = xpf[((size_t)tm * Kc + c) * 32 + col];
     };
     if (s < Kc) {
         load_h(s);
@@ -107,17 +103,15 @@ __global__ __launch_bounds__(512, (WM * WN == 1 ? 4 : 2)) void k_gemm_ks(GemmJob
 
     for (int cb = 0; cb < Kc; cb += S) {
         const int c = cb + s;
-        f16v acc[WM][WN];
+        f16v acc[1][WN];
         const float pfc = pf;
         if (c < Kc) {
-            int half0[HALVES ? WM : 1][HALVES ? WN : 1][HALVES ? 16 : 1];
+            int half0[HALVES ? WN : 1][HALVES ? 16 : 1];
 #pragma unroll
-            for (int i = 0; i < WM; i++)
-#pragma unroll
-                for (int j = 0; j < WN; j++) acc[i][j] = zero16();
+            for (int j = 0; j < WN; j++) acc[0][j] = zero16();
 #pragma unroll
             for (int sl = 0; sl < KSTEPS; sl++) {
-                kstep<QT, WM, WN, A1>(a[sl % PF], b[sl % PF], hd, sl, acc);
+                kstep<QT, 1, WN, A1>(a[sl % PF], b[sl % PF], hd, sl, acc);
                 if (sl + PF < KSTEPS) load_k(c, sl + PF, a[sl % PF], b[sl % PF]);
                 // pin the order: the loads of later ksteps stay behind this one's
                 // MFMAs, and its block factors' fmas ahead of the next one's (left
@@ -125,35 +119,27 @@ __global__ __launch_bounds__(512, (WM * WN == 1 ? 4 : 2)) void k_gemm_ks(GemmJob
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (!fold_fmt<QT>() && QT != QT_F32)
 #pragma unroll
-                    for (int i = 0; i < WM; i++)
-#pragma unroll
-                        for (int j = 0; j < WN; j++) asm volatile("" : "+v"(acc[i][j]));
+                    for (int j = 0; j < WN; j++) asm volatile("" : "+v"(acc[0][j]));
                 if constexpr (HALVES) {
                     if (sl == KSTEPS / 2 - 1)
 #pragma unroll
-                        for (int i = 0; i < WM; i++)
+                        for (int j = 0; j < WN; j++)
 #pragma unroll
-                            for (int j = 0; j < WN; j++)
-#pragma unroll
-                                for (int e = 0; e < 16; e++) {
-                                    half0[i][j][e] = (int)acc[i][j][e];
-                                    acc[i][j][e] = 0.0f;
-                                }
+                            for (int e = 0; e < 16; e++) {
+                                half0[j][e] = (int)acc[0][j][e];
+                                acc[0][j][e] = 0.0f;
+                            }
                 }
             }
             if constexpr (HALVES) {
 #pragma unroll
-                for (int i = 0; i < WM; i++)
+                for (int j = 0; j < WN; j++)
 #pragma unroll
-                    for (int j = 0; j < WN; j++)
-#pragma unroll
-                        for (int e = 0; e < 16; e++) acc[i][j][e] = (float)(half0[i][j][e] + (int)acc[i][j][e]);
+                    for (int e = 0; e < 16; e++) acc[0][j][e] = (float)(half0[j][e] + (int)acc[0][j][e]);
             }
             if constexpr (fold_fmt<QT>()) {
 #pragma unroll
-                for (int i = 0; i < WM; i++)
-#pragma unroll
-                    for (int j = 0; j < WN; j++) fold_finish<QT>(xmv[i], hd.h[j], acc[i][j]);
+                for (int j = 0; j < WN; j++) fold_finish<QT>(xmv, hd.h[j], acc[0][j]);
             }
             // the next chunk's first operands are in flight during the exchange
             if (c + S < Kc) {
@@ -165,12 +151,10 @@ __global__ __launch_bounds__(512, (WM * WN == 1 ? 4 : 2)) void k_gemm_ks(GemmJob
         if (cb > 0) __syncthreads();   // the round before is folded
         if (c < Kc) {
 #pragma unroll
-            for (int i = 0; i < WM; i++)
+            for (int j = 0; j < WN; j++)
 #pragma unroll
-                for (int j = 0; j < WN; j++)
-#pragma unroll
-                    for (int e = 0; e < 16; e++)
-                        part[(s * TR + 32 * i + drow(e, hh)) * TCS + 32 * (WN * pcI + j) + col] = acc[i][j][e];
+                for (int e = 0; e < 16; e++)
+                    part[(s * TR + drow(e, hh)) * TCS + 32 * (WN * pcI + j) + col] = acc[0][j][e];
             if (pcI == 0 && lane < TR) pfs[s * TR + lane] = pfc;
         }
         __syncthreads();
@@ -224,7 +208,7 @@ __global__ __launch_bounds__(512, (WM * WN == 1 ? 4 : 2)) void k_gemm_ks(GemmJob
             uint8_t *o = blk + ((hu * 2) * 64 + row + 32 * h2) * 16 + 8 * (l32 & 1);
             __builtin_memcpy(o, hv, 8);
             __builtin_memcpy(o + 1024, lv, 8);
-            if (l32 == 0) po.xpf[((size_t)G0 * po.Kc + tn) * 32 + row] = ldexpf(1.0f, -sh);
+            if (l32 == 0) po.xpf[((size_t)tm * po.Kc + tn) * 32 + row] = ldexpf(1.0f, -sh);
             if (po.xsum) {
                 const float even = __shfl_xor(s4, 1, 64);
                 float s8 = even;
@@ -242,17 +226,17 @@ __global__ __launch_bounds__(512, (WM * WN == 1 ? 4 : 2)) void k_gemm_ks(GemmJob
             }
         }
         __syncthreads();
-        uint8_t *gx = po.xp + ((size_t)G0 * po.Kc + tn) * 16 * 1024;
+        uint8_t *gx = po.xp + ((size_t)tm * po.Kc + tn) * 16 * 1024;
 #pragma unroll
         for (int i = 0; i < 1024 / NT; i++) *(uint4 *)(gx + (i * NT + tid) * 16) = *(const uint4 *)(blk + (i * NT + tid) * 16);
         if (po.xsum && tid < 64)
-            *(uint4 *)(po.xm + (((size_t)G0 * po.Kc + tn) * 64 + tid) * 16) = *(const uint4 *)(xmb + tid * 16);
+            *(uint4 *)(po.xm + (((size_t)tm * po.Kc + tn) * 64 + tid) * 16) = *(const uint4 *)(xmb + tid * 16);
         return;
     }
     const bool vec = W.n % V == 0 && ((uintptr_t)y & (4 * V - 1)) == 0;
 #pragma unroll
     for (int v = 0; v < VN; v++) {
-        const int idx = v * NT + tid, m = 32 * G0 + idx / (TC / V), n = TC * tn + V * (idx % (TC / V));
+        const int idx = v * NT + tid, m = TR * tm + idx / (TC / V), n = TC * tn + V * (idx % (TC / V));
         if (m >= M || n >= W.n) continue;
         float *yp = y + (size_t)m * W.n + n;
         float o[V];
@@ -279,14 +263,14 @@ __global__ __launch_bounds__(512, (WM * WN == 1 ? 4 : 2)) void k_gemm_ks(GemmJob
     }
 }
 
-template <int QT, int EPI, bool A1, int WM, int WN, int PC>
+template <int QT, int EPI, bool A1, int WN, int PC>
 hipError_t launch_ks(const GemmJobs &J, const uint8_t *xp, const float *xs16, const float *xpf, int M, int act,
                      const PrepOut &po, hipStream_t st) {
-    using L = KsTile<QT, A1, WM, WN, PC>;
+    using L = KsTile<QT, WN, PC>;
     const DevW &W = J.W[0];
     const float wbytes = w_bpe<QT>() * W.Np * W.Kp * J.n, abytes = (A1 ? 2.0f : 4.0f) * mh_mpad(M) * W.Kp;
     const int tilesM = (EPI == EPI_PREP ? mh_mpad(M) : M + L::TR - 1) / L::TR, tilesN = W.Np / L::TC, nt = J.n * tilesN;
-    static const hipError_t attr = hipFuncSetAttribute((const void *)k_gemm_ks<QT, EPI, A1, WM, WN, PC>,
+    static const hipError_t attr = hipFuncSetAttribute((const void *)k_gemm_ks<QT, EPI, A1, WN, PC>,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::LDS);
     if (attr != hipSuccess) return attr;
     // row parts of the XCD grid: the fewest bytes over the eight L2s, times the
@@ -299,7 +283,7 @@ hipError_t launch_ks(const GemmJobs &J, const uint8_t *xp, const float *xs16, co
         const float cost = (wbytes * p + abytes * (8 / p)) * (8.0f * rect / ((float)tilesM * nt));
         if (p == 1 || cost < best) best = cost, pr = p, wgs = 8 * rect;
     }
-    hipLaunchKernelGGL((k_gemm_ks<QT, EPI, A1, WM, WN, PC>), dim3((unsigned)wgs), dim3(L::NT), L::LDS, st, J, xp,
+    hipLaunchKernelGGL((k_gemm_ks<QT, EPI, A1, WN, PC>), dim3((unsigned)wgs), dim3(L::NT), L::LDS, st, J, xp,
                        (const uint8_t *)xs16, xpf, M, act, tilesM, tilesN, pr, po);
     return hipGetLastError();
 }
@@ -308,10 +292,10 @@ template <int QT, bool A1>
 hipError_t ks_t(const GemmJobs &J, const uint8_t *xp, const float *xs16, const float *xpf, int M, int act,
                 const PrepOut *po, hipStream_t st) {
     if (po) {
-        if constexpr (!A1) return launch_ks<QT, EPI_PREP, false, 1, 2, 2>(J, xp, xs16, xpf, M, 1, *po, st);
+        if constexpr (!A1) return launch_ks<QT, EPI_PREP, false, 2, 2>(J, xp, xs16, xpf, M, 1, *po, st);
         return hipErrorInvalidValue;
     }
-    return launch_ks<QT, EPI_Y, A1, 1, 1, 1>(J, xp, xs16, xpf, M, act, PrepOut{}, st);
+    return launch_ks<QT, EPI_Y, A1, 1, 1>(J, xp, xs16, xpf, M, act, PrepOut{}, st);
 }
 
 template <int QT>

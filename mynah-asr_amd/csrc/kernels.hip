@@ -99,10 +99,8 @@ template <int QT, bool A1 = false, int NCG = 4, int NRG = 2, bool BD = false> st
 // workgroups per CU the register budget is sized for: as many as the LDS
 // ring allows (three double-buffered workgroups: 25-27 KiB stages, 24 KiB
 // one-kstep stages for f32 weights; four of 32-row tiles, three for f32
-// weights), two for Q6_K (its eight per-half-step f32 factors need more
-// registers), and two for the split-K form of the
-// formats whose chunk-result stores would otherwise spill (INT4; Q5_K with
-// int8 activations, whose chunk halves join in int32)
+// weights and Q6_K), two for the 64 x 256 tiles and for Q6_K (its eight
+// per-half-step f32 factors need more registers)
 #ifndef GQ_V
 #define GQ_V 0
 #endif
@@ -144,11 +142,9 @@ __global__ __launch_bounds__(256, (gemm_occ<QT, EPI, A1, WN, WM>())) void k_gemm
                                                  int ngrp) {
     using F = Fmt<QT>;
     // the weight planes go straight to registers, one stage ahead (measured
-    // 3-6% faster than through LDS on every format: less LDS traffic), except
-    // in the split-K form (its chunk-result stores leave no registers for
-    // them: with them it spilled, and 4096->1024 at 750 rows took 129 us, not
-    // 50) and, for f32 weights, in the FFN's fused form (its epilogue's LDS
-    // tile needs the larger stages)
+    // 3-6% faster than through LDS on every format: less LDS traffic), except,
+    // for f32 weights, in the FFN's fused form (its epilogue's LDS tile needs the
+    // larger stages)
     constexpr bool BD = QT != QT_F32 || EPI == EPI_Y;
     using L = StageLayout<QT, A1, 4 * WN, WM, BD>;
     typename F::RawK rb[2][WN][L::SPS];   // BD: the weight planes of the stage in flight and the current one
@@ -1747,11 +1743,16 @@ static int gemm_ngroups(float wbytes, float abytes, int tilesM, int nt) {
     return best;
 }
 
-// 32 x 128 workgroup tiles when the 64 x 128 ones give at most two per CU;
-// measured on 750 rows: 1024->4096 (384 tiles) 25.9 -> 23.4 us, 1024->1024
-// (96) 17.7 -> 13.3 us; at 6000 rows 1024->1024 (752) 36 -> 40 us and at 1500
-// rows 1024->4096 (768) 36.6 -> 39.7 us, so there the 64-row tiles stay. The
-// same bits either way.
+// 32 x 128 workgroup tiles when the 64 x 128 ones give at most two per CU (the
+// products of few rows are k_gemm_ks's before that). 64-row / 32-row tiles, us,
+// prepared products:
+//   1024 -> 1024   1100 rows (144 tiles)  Q8_0 15.2 / 13.3   F32 16.8 / 15.6
+//                  2000 (256)                  16.9 / 14.6       20.8 / 19.8
+//   1024 -> 4096    750 (384)                  23.1 / 20.1       28.3 / 27.5
+//   1024 -> 1024   4000 (504)                  25.0 / 25.4       31.0 / 35.5
+//   1024 -> 4096   1500 (768)                  36.6 / 39.7
+// Between 400 and 512 tiles the 64-row ones are level or faster too (K = 4096 at
+// 440 tiles 75.0 / 83.1). The same bits either way.
 static bool gemm_narrow(int grid) { return grid <= 512; }
 
 // 64 x 256 workgroup tiles (two column groups per wave, two workgroups per

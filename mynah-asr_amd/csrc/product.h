@@ -350,17 +350,6 @@ __device__ __forceinline__ int wshift(const DevW &W, int n) {
     return 0;
 }
 
-__device__ __forceinline__ f16v load_rows16(const float *b) {
-    // the lane's 16 D-layout rows from a [32]-row float vector (b at row 4*hh)
-    f16v r;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const float4 v = *(const float4 *)(b + 8 * q);
-        r[4 * q + 0] = v.x; r[4 * q + 1] = v.y; r[4 * q + 2] = v.z; r[4 * q + 3] = v.w;
-    }
-    return r;
-}
-
 // Where a product's result goes: EPI_Y stores y (SiLU applied when act);
 // EPI_PREP (the first product of the FFN) applies SiLU and, instead of
 // storing the f32 intermediate, prepares it as the second product's input —

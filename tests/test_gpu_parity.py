@@ -288,11 +288,11 @@ def test_split_k_gemv_in_place_and_repeated(gpu, orc, qt):
 
 @pytest.mark.parametrize("qt", ALL, ids=lambda q: M.NAMES[q])
 def test_split_k_gemm_rows_match_gemm(gpu, orc, qt):
-    """A product with few tiles splits K over workgroups (chunk results to a
-    workspace, then their fold in chunk order); its rows must carry the bits
+    """A product with few tiles splits K over a workgroup's waves (chunk results
+    to LDS, then their fold in chunk order); its rows must carry the bits
     of the same rows in a product with enough tiles to run unsplit. K = 2048,
-    N = 1024: M = 40 and 700 split (8 and 88 tiles), M = 2100 does not (264
-    tiles); with and without SiLU."""
+    N = 1024: M = 40 and 700 split (64 and 704 tiles of 32 x 32), M = 2100 does
+    not (2112); with and without SiLU."""
     import torch
     say("split-K gemm", M.NAMES[qt])
     k, n = 2048, 1024

@@ -37,8 +37,8 @@ def _run(torch, dw, x, T, n, act, noalloc):
     return y
 
 
-# (format, n, k, first M, second M): GEMM sizes on both calls, one pair that
-# would split K in qgemm_dev (M = 40 at K = 4096), pairs crossing to the GEMV
+# (format, n, k, first M, second M): GEMM sizes on both calls, one pair whose second
+# splits K over a workgroup (M = 40 at K = 4096), pairs crossing to the GEMV
 # (Q8_0 4096 -> 1024 at M = 4: qgemm_dev runs the split-K GEMV there, the
 # allocation-free entry the one-launch GEMV, which must give the same bits)
 CASES = [
