@@ -336,7 +336,9 @@ int mynah_asr_hip_aed_decode_dev(const mynah_asr_hip_aed *a, const float *enc, i
                                  int n_prompt, int eos, int *tokens, int cap, void *stream);
 /* The same steps over given tokens (host, n <= max_seq): logits (device,
  * [n, vocab]) of every position, as the decode loop computes them before its
- * argmax. 0 or -1. */
+ * argmax, but as rows of batches of up to 64 positions (so does a prompt): a
+ * position's bits do not depend on the tokens after it; against a decoded
+ * position, layer norms sum in another order (last bits). 0 or -1. */
 int mynah_asr_hip_aed_forced_dev(const mynah_asr_hip_aed *a, const float *enc, int T, const int *tokens, int n,
                                  float *logits, void *stream);
 

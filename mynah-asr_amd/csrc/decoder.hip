@@ -14,8 +14,10 @@
 //   k_bias_rows  y[t] += b                                    decoder_aed.c:132-136
 //
 // Positions whose tokens are given (the prompt; all of them when tokens are
-// scored) run as rows of one batch: a row of the products carries the bits of
-// the row alone, and row p attends to the keys up to p.
+// scored) run as rows of one batch: every step works row by row, in an order that
+// does not depend on the other rows, and row p attends to the keys up to p, so a
+// row carries the bits of the row alone. Decoded positions take the GEMVs'
+// prologues instead of k_ln_rows and k_att_combine: the same sums in another order.
 // A decoded position p and its token live in device memory (`st`: st[0] = p,
 // st[1] = the last argmax), so one captured launch sequence serves every step
 // (decoder_aed.c:213-222 chooses the same tokens).
